@@ -113,7 +113,7 @@ struct crt_context {
     uint32_t   *st_inst = nullptr, *st_inst_out = nullptr;
     float      *st_ng[3] = {};
     uint8_t    *st_occ = nullptr;
-    uint32_t   *st_cnt = nullptr;   // [0] count, [8..15] work counters, [16] error
+    uint32_t   *st_cnt = nullptr;   // kQcWords words: count, error flag, work counters
     uint8_t    *noalloc = nullptr;  // this device's crt_intersect_noalloc scratch (noalloc.hip)
     std::mutex  mu;                 // serialises queries on the context stream
     std::atomic<int> live{0};       // scenes, renderers and caches created on the context
@@ -611,19 +611,19 @@ int run_paths(crt_renderer *r, const PathBuffers &b, const RenderParams &rp, hip
         if (sort && i > 0) {
             // reorder the secondary rays (counted in the extend phase)
             uint32_t n = 0;
-            HIP_CHECK(hipMemcpyAsync(&n, b.cnt + cur, sizeof n, hipMemcpyDeviceToHost, s));
+            HIP_CHECK(hipMemcpyAsync(&n, b.cnt + cnt_queue(cur), sizeof n, hipMemcpyDeviceToHost, s));
             HIP_CHECK(hipStreamSynchronize(s));
             n = std::min(n, b.P);
-            HIP_CHECK(launch_ray_sort(b.q[cur], b.qpath[cur], b.cnt + cur, n, b.q[cur ^ 1u], b.qpath[cur ^ 1u],
-                                      b.cnt + (cur ^ 1u), sc.bmin, sc.bmax, r->sort, s));
+            HIP_CHECK(launch_ray_sort(b.q[cur], b.qpath[cur], b.cnt + cnt_queue(cur), n, b.q[cur ^ 1u], b.qpath[cur ^ 1u],
+                                      b.cnt + cnt_queue(cur ^ 1u), sc.bmin, sc.bmax, r->sort, s));
             cur ^= 1u;
         }
         // the epilogue clears the queue the shading appends to (the previous bounce's
         // input), the shadow queue, and the work counters; it counts the extension rays
-        TraceQueue q = make_queue(b.q[cur], b.hits, b.cnt + cur, b.cnt + kCntWorkExt, b.cnt + kCntErr);
+        TraceQueue q = make_queue(b.q[cur], b.hits, b.cnt + cnt_queue(cur), b.cnt + kCntWorkExt, b.cnt + kCntErr);
         q.tstats     = b.tstats;
         q.done       = b.cnt + kCntDoneExt;
-        q.clear0     = b.cnt + (cur ^ 1u);
+        q.clear0     = b.cnt + cnt_queue(cur ^ 1u);
         q.clear1     = b.cnt + kCntShadow;
         q.stat       = b.stats + 0;
         HIP_CHECK(launch_trace_closest(sc, q, spill, tc, s));
@@ -1084,7 +1084,7 @@ int stage_reserve(crt_context *ctx, uint32_t n)
     HIP_CHECK(dalloc(&ctx->st_inst_out, cap));
     for (float *&p : ctx->st_ng) HIP_CHECK(dalloc(&p, cap));
     HIP_CHECK(dalloc(&ctx->st_occ, cap));
-    HIP_CHECK(dalloc(&ctx->st_cnt, 32));
+    HIP_CHECK(dalloc(&ctx->st_cnt, (size_t)kQcWords));
     ctx->stage_cap = cap;
     return CRT_OK;
 }
@@ -1115,7 +1115,7 @@ int query(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_hits *hits, ui
             *dst[k] = const_cast<float *>(in[k]);
         }
     }
-    HIP_CHECK(hipMemsetAsync(ctx->st_cnt, 0, sizeof(uint32_t) * 32, s));
+    HIP_CHECK(hipMemsetAsync(ctx->st_cnt, 0, sizeof(uint32_t) * kQcWords, s));
     HIP_CHECK(hipMemcpyAsync(ctx->st_cnt, &n, sizeof n, hipMemcpyHostToDevice, s));
     if (hits) {
         HitSoA h{};
@@ -1125,7 +1125,7 @@ int query(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_hits *hits, ui
         h.v    = dev && hits->v ? hits->v : ctx->st_v;
         h.tri  = ctx->st_tri;
         h.inst = ctx->st_inst;
-        TraceQueue q = make_queue(rs, h, ctx->st_cnt, ctx->st_cnt + 8, ctx->st_cnt + 16, false);
+        TraceQueue q = make_queue(rs, h, ctx->st_cnt, ctx->st_cnt + kQcWork, ctx->st_cnt + kQcErr, false);
         HIP_CHECK(launch_trace_closest(scene->dev, q, ctx->spill, trace_cfg(ctx), s));
         uint32_t *prim = dev ? hits->prim_id : ctx->st_prim;
         uint32_t *geom = dev ? hits->geom_id : (hits->geom_id ? ctx->st_geom : nullptr);
@@ -1147,13 +1147,13 @@ int query(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_hits *hits, ui
                 if (ng[k]) HIP_CHECK(hipMemcpyAsync(ng[k], ctx->st_ng[k], sizeof(float) * n, hipMemcpyDeviceToHost, s));
         }
     } else {
-        TraceQueue q = make_queue(rs, HitSoA{}, ctx->st_cnt, ctx->st_cnt + 8, ctx->st_cnt + 16, false);
+        TraceQueue q = make_queue(rs, HitSoA{}, ctx->st_cnt, ctx->st_cnt + kQcWork, ctx->st_cnt + kQcErr, false);
         uint8_t   *occ = memory == CRT_MEM_DEVICE ? occluded : ctx->st_occ;
         HIP_CHECK(launch_trace_any(scene->dev, q, occ, ctx->spill, trace_cfg(ctx), s));
         if (memory == CRT_MEM_HOST) HIP_CHECK(hipMemcpyAsync(occluded, ctx->st_occ, n, hipMemcpyDeviceToHost, s));
     }
     uint32_t err = 0;
-    HIP_CHECK(hipMemcpyAsync(&err, ctx->st_cnt + 16, sizeof err, hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipMemcpyAsync(&err, ctx->st_cnt + kQcErr, sizeof err, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
     if (err) return fail(CRT_ERR_HIP, "traversal stack overflow");
     return CRT_OK;
@@ -1193,7 +1193,7 @@ int cast_records(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_records
             *dst[k] = const_cast<float *>(in[k]);
         }
     }
-    HIP_CHECK(hipMemsetAsync(ctx->st_cnt, 0, sizeof(uint32_t) * 32, s));
+    HIP_CHECK(hipMemsetAsync(ctx->st_cnt, 0, sizeof(uint32_t) * kQcWords, s));
     HIP_CHECK(hipMemcpyAsync(ctx->st_cnt, &n, sizeof n, hipMemcpyHostToDevice, s));
     HitSoA h{};
     h.t    = ctx->st_t;
@@ -1201,7 +1201,7 @@ int cast_records(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_records
     h.v    = ctx->st_v;
     h.tri  = ctx->st_tri;
     h.inst = ctx->st_inst;
-    TraceQueue q = make_queue(rs, h, ctx->st_cnt, ctx->st_cnt + 8, ctx->st_cnt + 16, true);
+    TraceQueue q = make_queue(rs, h, ctx->st_cnt, ctx->st_cnt + kQcWork, ctx->st_cnt + kQcErr, true);
     HIP_CHECK(launch_trace_closest(scene->dev, q, ctx->spill, trace_cfg(ctx), s));
     // where each field lands on the device, and where it goes on the host
     struct Field {
@@ -1233,7 +1233,7 @@ int cast_records(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_records
         for (int k = 0; k < 12; ++k)
             if (f[k].user) HIP_CHECK(hipMemcpyAsync(f[k].user, f[k].stage, f[k].elem * n, hipMemcpyDeviceToHost, s));
     uint32_t err = 0;
-    HIP_CHECK(hipMemcpyAsync(&err, ctx->st_cnt + 16, sizeof err, hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipMemcpyAsync(&err, ctx->st_cnt + kQcErr, sizeof err, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
     if (err) return fail(CRT_ERR_HIP, "traversal stack overflow");
     return CRT_OK;
@@ -1985,13 +1985,13 @@ int crt_intersect_noalloc(crt_scene *scene, const crt_rays *rays, uint32_t n, cr
     h.tri  = reinterpret_cast<uint32_t *>(sp + kNaTri);
     h.inst = reinterpret_cast<uint32_t *>(sp + kNaInst);
     HIP_CHECK(launch_noalloc_init(cnt, n, s));
-    TraceQueue q = make_queue(rs, h, cnt, cnt + 8, cnt + 16, false);
+    TraceQueue q = make_queue(rs, h, cnt, cnt + kQcWork, cnt + kQcErr, false);
     HIP_CHECK(launch_trace_closest(scene->dev, q, reinterpret_cast<uint32_t *>(sp + kNaSpill),
                                    TraceConfig{kNoAllocGrid, ctx->stack}, s));
     HIP_CHECK(launch_hits_to_api(scene->dev, h, n, hits->prim_id, hits->geom_id, hits->ng_x, hits->ng_y, hits->ng_z,
                                  hits->inst_id, s));
     uint32_t err = 0;
-    HIP_CHECK(hipMemcpyAsync(&err, cnt + 16, sizeof err, hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipMemcpyAsync(&err, cnt + kQcErr, sizeof err, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
     if (err) return fail(CRT_ERR_HIP, "traversal stack overflow");
     return CRT_OK;
@@ -2774,7 +2774,7 @@ int record_trace(const PathBuffers &b, const BatchDev &bd, const TraceScene *tsc
     uint32_t cur = 0;
     for (uint32_t i = 0; i < max_bounces; ++i) {
         HIP_CHECK(launch_bounce_prep(b, cur, s));
-        TraceQueue q = make_queue(b.q[cur], b.hits, b.cnt + cur, b.cnt + kCntWorkExt, b.cnt + kCntErr);
+        TraceQueue q = make_queue(b.q[cur], b.hits, b.cnt + cnt_queue(cur), b.cnt + kCntWorkExt, b.cnt + kCntErr);
         q.ray_path = b.qpath[cur];
         q.path_job = b.pjob;
         q.scenes   = tscenes;

@@ -164,6 +164,8 @@ hipError_t bvh_rebase(void *nodes, uint32_t count, uint32_t width, uint32_t node
 hipError_t tri_add_prim_base(float4 *tri, uint32_t ntri, uint32_t base, hipStream_t s);
 
 // ---- traversal ----------------------------------------------------------------------
+constexpr uint32_t kXcds    = 8;
+constexpr uint32_t kCntLine = 32;   // words per 128-byte line
 struct TraceScene;
 struct TraceQueue {
     RaySoA          rays;
@@ -174,7 +176,7 @@ struct TraceQueue {
     // semantics of crt_intersect / crt_occluded).
     uint32_t        unit_dir;
     const uint32_t *count;     // device: number of rays
-    uint32_t       *counters;  // device: work counters (kXcds entries), zeroed by the caller's kernel
+    uint32_t       *counters;  // device: work counters (kXcds of them, kCntLine words apart), 0 at launch
     uint32_t       *error;     // device: set to 1 if a traversal stack would overflow
     unsigned long long *tstats;  // device [5] or null: node visits, leaf visits, triangle tests,
                                  // wave iterations of the node loop and of the leaf loop
@@ -182,7 +184,7 @@ struct TraceQueue {
     const uint32_t   *ray_path;
     const uint32_t   *path_job;
     const TraceScene *scenes;
-    // Epilogue (done != null): the last block to finish zeroes the work counters, the words
+    // Epilogue (done != null): the last block with rays zeroes the work counters, the words
     // clear0 / clear1 (when set; never `count`), adds the ray count to *stat (when set) and
     // resets *done, which must be 0 at launch.  It prepares the next bounce's counters
     // without a kernel of its own.
@@ -241,7 +243,6 @@ hipError_t launch_atrous(const float4 *colour, const float4 *normal, const float
 uint32_t trace_grid(int device, uint32_t waves_per_cu);
 uint64_t trace_spill_bytes(uint32_t grid);
 constexpr uint32_t kTraceBlock = 256;
-constexpr uint32_t kXcds       = 8;
 // default LDS stack entries per lane: 16 entries (34.3 KB per 256-lane block) let the
 // traversals of both wavefronts in flight hold their blocks on a CU at once (4 x 34.3 KB of
 // 160 KB), where 32 entries (67.6 KB per block) admit only one traversal's two blocks
@@ -249,14 +250,16 @@ constexpr uint32_t kStackLds   = 16;
 constexpr uint32_t kSpillDepth = 256;   // global spill entries per lane (multiple of kStackLds)
 
 // ---- allocation-free queries (noalloc.hip) ---------------------------------------------
-// Layout of the per-device scratch array (byte offsets): counters (count, work counters at
-// +8, error flag at +16), leaf-order triangle and instance indices, u and v for callers that
+// Layout of the per-device scratch array (byte offsets): counters (query_cnt words), leaf-order triangle and instance indices, u and v for callers that
 // pass none, and the traversal spill stack of a kNoAllocGrid-block launch.
 constexpr uint32_t kNoAllocRays     = 1u << 20;   // rays per crt_intersect_noalloc call
 constexpr uint32_t kNoAllocGrid     = 64;         // traversal blocks (a multiple of kXcds = 8)
-constexpr uint32_t kNoAllocCounters = 64;
+// Words of a query's counters: the ray count, the error flag and the work counters, on lines
+// of their own.
+enum : uint32_t { kQcCount = 0, kQcErr = kCntLine, kQcWork = 2 * kCntLine, kQcWords = (2 + kXcds) * kCntLine };
 constexpr size_t   kNaCnt   = 0;
-constexpr size_t   kNaTri   = 256;
+constexpr size_t   kNaTri   = 2048;
+static_assert(kQcWords * 4 <= kNaTri, "the counters fit before the hit indices");
 constexpr size_t   kNaInst  = kNaTri + 4ull * kNoAllocRays;
 constexpr size_t   kNaU     = kNaInst + 4ull * kNoAllocRays;
 constexpr size_t   kNaV     = kNaU + 4ull * kNoAllocRays;
@@ -305,12 +308,18 @@ struct PathBuffers {
     unsigned long long *tstats;
 };
 constexpr uint32_t kStatSlots = 64;
-// layout of PathBuffers::cnt
+// Layout of PathBuffers::cnt.  Words that blocks of one launch add to, or that launches in
+// flight together use, lie kCntLine words (one 128-byte line) apart: atomics on one line from
+// the whole chip are served one after the other.
 enum : uint32_t {
-    kCntQ0 = 0, kCntQ1 = 1, kCntShadow = 2, kCntShadow2 = 3, kCntErr = 4, kCntNrcQ = 5, kCntTrain = 6,
-    kCntNrcBad = 7,   // a cache prediction of the wavefront was not finite: its accumulation is skipped
-    kCntWorkExt = 8, kCntWorkShadow = 16, kCntDoneExt = 24, kCntDoneShadow = 25, kCntWords = 32
+    kCntQ0 = 0, kCntQ1 = kCntQ0 + kCntLine, kCntShadow = 2 * kCntLine, kCntShadow2 = 3 * kCntLine,
+    kCntNrcQ = 4 * kCntLine, kCntTrain = 5 * kCntLine, kCntErr = 6 * kCntLine,
+    kCntNrcBad = kCntErr + 1,   // a cache prediction of the wavefront was not finite: its accumulation is skipped
+    kCntDoneExt = 7 * kCntLine, kCntDoneShadow = 8 * kCntLine,
+    kCntWorkExt = 9 * kCntLine, kCntWorkShadow = (9 + kXcds) * kCntLine,
+    kCntWords = (9 + 2 * kXcds) * kCntLine
 };
+CRT_HD uint32_t cnt_queue(uint32_t cur) { return kCntQ0 + cur * kCntLine; }   // count of extension queue cur
 
 // Neural radiance cache hooks of the integrator.  Camera paths (slots < npix) query the
 // cache at `term` (footprint rule); training paths (slots >= npix) start at random pixels,

@@ -162,8 +162,8 @@ __global__ __launch_bounds__(256) void k_generate(SceneDev sc, PathBuffers b, Re
         // the pass's counters: queue 0, the cache queries, and the traversal work counters and
         // finished-block counts (the traversal epilogues clear the rest bounce by bounce)
         if (threadIdx.x < 8) {
-            b.cnt[kCntWorkExt + threadIdx.x]    = 0;
-            b.cnt[kCntWorkShadow + threadIdx.x] = 0;
+            b.cnt[kCntWorkExt + threadIdx.x * kCntLine]    = 0;
+            b.cnt[kCntWorkShadow + threadIdx.x * kCntLine] = 0;
         }
         if (threadIdx.x == 0) {
             b.cnt[kCntQ0]          = rp.max_bounces > 0 ? ncl + ntrain : 0u;
@@ -184,20 +184,20 @@ __global__ void k_bounce_prep(PathBuffers b, uint32_t cur)
 {
     const uint32_t t = threadIdx.x;
     if (t < 8) {
-        b.cnt[kCntWorkExt + t]    = 0;
-        b.cnt[kCntWorkShadow + t] = 0;
+        b.cnt[kCntWorkExt + t * kCntLine]    = 0;
+        b.cnt[kCntWorkShadow + t * kCntLine] = 0;
     }
     if (t == 0) {
-        b.cnt[cur ^ 1u]       = 0;
-        b.cnt[kCntShadow]     = 0;
-        atomicAdd(&b.stats[0], (unsigned long long)b.cnt[cur]);
+        b.cnt[cnt_queue(cur ^ 1u)] = 0;
+        b.cnt[kCntShadow]          = 0;
+        atomicAdd(&b.stats[0], (unsigned long long)b.cnt[cnt_queue(cur)]);
     }
 }
 
 __global__ void k_shadow_prep(PathBuffers b)
 {
     const uint32_t t = threadIdx.x;
-    if (t < 8) b.cnt[kCntWorkShadow + t] = 0;
+    if (t < 8) b.cnt[kCntWorkShadow + t * kCntLine] = 0;
     if (t == 0) {
         b.cnt[kCntShadow2] = 0;
         atomicAdd(&b.stats[1], (unsigned long long)b.cnt[kCntShadow]);
@@ -552,7 +552,7 @@ __global__ __launch_bounds__(256) void k_shade(SceneDev sc, PathBuffers b, Rende
                                                uint32_t bounce, uint32_t cur, const uint32_t *perm)
 {
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t n = b.cnt[cur];
+    const uint32_t n = b.cnt[cnt_queue(cur)];
     const bool     live = t < n;
     // perm: queue entries in material-class order (the queue index itself otherwise)
     const uint32_t k = live && perm ? perm[t] : t;
@@ -585,7 +585,7 @@ __global__ __launch_bounds__(256) void k_shade(SceneDev sc, PathBuffers b, Rende
         b.spath[ns]    = p;
         b.scontrib[ns] = make_float4(o.scontrib.x, o.scontrib.y, o.scontrib.z, 0.0f);
     }
-    const uint32_t nn = block_append(&b.cnt[cur ^ 1u], o.push_next);
+    const uint32_t nn = block_append(&b.cnt[cnt_queue(cur ^ 1u)], o.push_next);
     if (o.push_next) {
         put_ray(b.q[cur ^ 1u], nn, o.no, o.nd);
         b.qpath[cur ^ 1u][nn] = p;
@@ -688,7 +688,7 @@ __global__ void k_shadow_swap(PathBuffers b)
         b.cnt[kCntShadow2] = 0;
         atomicAdd(&b.stats[1], (unsigned long long)m);
     }
-    if (threadIdx.x < 8) b.cnt[kCntWorkShadow + threadIdx.x] = 0;
+    if (threadIdx.x < 8) b.cnt[kCntWorkShadow + threadIdx.x * kCntLine] = 0;
 }
 
 // raw[pixel] += the radiance of each of the wavefront's samples of the pixel, in sample

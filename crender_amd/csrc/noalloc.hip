@@ -26,7 +26,7 @@ void         *g_scratch[kMaxDevices] = {};
 // also behaves under stream capture
 __global__ void k_noalloc_init(uint32_t *cnt, uint32_t n)
 {
-    if (threadIdx.x < kNoAllocCounters) cnt[threadIdx.x] = threadIdx.x == 0 ? n : 0u;
+    if (threadIdx.x < kQcWords) cnt[threadIdx.x] = threadIdx.x == kQcCount ? n : 0u;
 }
 
 }  // namespace
@@ -54,7 +54,7 @@ hipError_t noalloc_scratch(int device, void **ptr)
 
 hipError_t launch_noalloc_init(uint32_t *cnt, uint32_t n, hipStream_t s)
 {
-    k_noalloc_init<<<1, kNoAllocCounters, 0, s>>>(cnt, n);
+    k_noalloc_init<<<1, kQcWords, 0, s>>>(cnt, n);
     return hipGetLastError();
 }
 

@@ -172,9 +172,9 @@ hipError_t launch_ray_sort(const RaySoA &src, const uint32_t *src_path, const ui
 hipError_t launch_shade_sort(const SceneDev &sc, const PathBuffers &b, uint32_t cur, hipStream_t s)
 {
     const uint32_t nb = (b.P + 255) / 256;
-    k_class_count<<<nb, 256, 0, s>>>(sc, b.hits, b.cnt + cur, b.shade_bcount);
+    k_class_count<<<nb, 256, 0, s>>>(sc, b.hits, b.cnt + cnt_queue(cur), b.shade_bcount);
     k_class_scan<<<1, 1024, 0, s>>>(b.shade_bcount, nb * kShadeClasses);
-    k_class_scatter<<<nb, 256, 0, s>>>(sc, b.hits, b.cnt + cur, b.shade_bcount, b.shade_perm);
+    k_class_scatter<<<nb, 256, 0, s>>>(sc, b.hits, b.cnt + cnt_queue(cur), b.shade_bcount, b.shade_perm);
     return hipGetLastError();
 }
 
