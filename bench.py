@@ -594,7 +594,7 @@ def main(argv=None) -> int:
             "workload": f"triangle soup {args.tris} tris, 1920x1080, 1 spp, primary + 3 diffuse bounces "
                         f"(depth 4), compat estimator, sun off, constant sky",
             "bvh_width": info["width"],
-            "waves_per_cu": args.waves_per_cu or 8,
+            "waves_per_cu": args.waves_per_cu or 16,
             "trace_stack": args.stack or 16,
             # sample passes per wavefront: floor(wavefront paths / (W*H)) in [1, 8], 2^24 paths by default
             "passes_per_wavefront": max(1, min(8, (args.wavefront_paths or (1 << 24)) // (res[0] * res[1]))),

@@ -102,6 +102,9 @@ struct crt_context {
     // fills the GPU while the other's launches drain; the second has its own spill area
     hipStream_t stream2 = nullptr;
     uint32_t   *spill2  = nullptr;
+    // spill entries per lane the committed scenes can need (grows with the deepest), and the
+    // number each of the two areas was allocated with
+    uint32_t    spill_depth = 32, spill_alloc[2] = {0, 0};
     uint32_t    stack  = kStackLds;   // LDS stack entries per traversal lane (8, 16, 32)
     uint32_t    refill = 0, park_min = 0, leaf_rounds = 0;   // traversal thresholds (0: defaults)
     uint32_t    batch_paths = 0;   // tuned wavefront size of crt_render_batch (0 = default)
@@ -239,14 +242,17 @@ namespace {
 
 TraceConfig trace_cfg(const crt_context *ctx)
 {
-    return TraceConfig{ctx->grid, ctx->stack, ctx->refill, ctx->park_min, ctx->leaf_rounds};
+    return TraceConfig{ctx->grid, ctx->stack, ctx->refill, ctx->park_min, ctx->leaf_rounds, ctx->spill_depth};
 }
 
 int ensure_spill(crt_context *ctx, int set = 0)
 {
     uint32_t *&sp = set ? ctx->spill2 : ctx->spill;
-    if (sp) return CRT_OK;
-    HIP_CHECK(hipMalloc((void **)&sp, trace_spill_bytes(ctx->grid)));
+    if (sp && ctx->spill_alloc[set] == ctx->spill_depth) return CRT_OK;
+    dfree(sp);
+    sp = nullptr;
+    HIP_CHECK(hipMalloc((void **)&sp, trace_spill_bytes(ctx->grid, ctx->spill_depth)));
+    ctx->spill_alloc[set] = ctx->spill_depth;
     return CRT_OK;
 }
 
@@ -601,11 +607,15 @@ int run_paths(crt_renderer *r, const PathBuffers &b, const RenderParams &rp, hip
     }
     const uint32_t timed = t.timing ? std::min<uint32_t>(nb, crt_renderer::kTimedBounces) : 0u;
     const bool sort = (ctx->opt.flags & CRT_FLAG_SORT_RAYS) && r->sort.keys;
-    // While the cache trains beside the traversal, the traversal keeps a 16-entry LDS stack:
-    // two 32-entry traversal blocks (2 x 67.6 KB) leave no room in a CU's LDS for a training
-    // block (31.7 KB), two 16-entry ones (2 x 34.3 KB) do.
+    // While the cache trains beside the traversal, the traversal leaves room in a CU's LDS for
+    // a training block (31.7 KB): a stack of at most 16 entries and, at the default grid, three
+    // blocks (3 x 34.8 KB) instead of four.
     TraceConfig tc = trace_cfg(ctx);
-    if (rp.nrc.enabled && r->nopt.train) tc.stack = std::min<uint32_t>(tc.stack, 16u);
+    if (rp.nrc.enabled && r->nopt.train) {
+        tc.stack = std::min<uint32_t>(tc.stack, 16u);
+        if (ctx->opt.trace_waves_per_cu == 0)
+            tc.grid = tc.grid / (kXcds * kTraceBlocksPerCu) * kXcds * kTraceBlocksPerCuTraining;
+    }
     for (uint32_t i = 0; i < nb; ++i) {
         const bool tm = i < timed;
         if (sort && i > 0) {
@@ -1908,6 +1918,8 @@ int crt_scene_commit(crt_scene *scene)
     bi.sah_cost        = br.sah;
     bi.build_ms        = br.ms;
     bi.bytes           = (uint64_t)br.node_count * 128u + (uint64_t)ntri * 48u;
+    // a lane spills at most its deepest stack, a whole LDS stack (8 to 32 entries) at a time
+    ctx->spill_depth = std::max(ctx->spill_depth, std::min(kSpillDepth, (max_stack + 31u) / 32u * 32u));
     scene->hash      = h;
     scene->committed = true;
     scene->dirty     = false;
@@ -2890,7 +2902,7 @@ int crt_render_batch(crt_context *ctx, const crt_job *jobs, uint32_t njobs, cons
         if ((st = lalloc(L, &b[k].pjob, P))) return st;
         if ((st = lalloc(L, &b[k].ppix, P))) return st;
         if ((st = lalloc(L, &b[k].psamp, P))) return st;
-        if ((st = lalloc(L, reinterpret_cast<uint8_t **>(&spill[k]), trace_spill_bytes(ctx->grid)))) return st;
+        if ((st = lalloc(L, reinterpret_cast<uint8_t **>(&spill[k]), trace_spill_bytes(ctx->grid, ctx->spill_depth)))) return st;
     }
     // jobs, per-job traversal views, outputs
     std::vector<JobDev>     hj(njobs);
@@ -3077,7 +3089,7 @@ int crt_autotune(crt_context *ctx, const crt_job *jobs, uint32_t njobs, uint32_t
         return CRT_OK;
     };
     if (ctx->batch_paths == 0) ctx->batch_paths = 4u << 20;
-    uint32_t blocks = ctx->opt.trace_waves_per_cu ? (ctx->opt.trace_waves_per_cu + 3) / 4 : 2;
+    uint32_t blocks = ctx->opt.trace_waves_per_cu ? (ctx->opt.trace_waves_per_cu + 3) / 4 : kTraceBlocksPerCu;
     uint32_t width  = scenes[0]->dev.width;
     int st = recommit(width);   // one width for the batch
     if (st) return st;

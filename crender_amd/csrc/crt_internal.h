@@ -166,6 +166,7 @@ hipError_t tri_add_prim_base(float4 *tri, uint32_t ntri, uint32_t base, hipStrea
 // ---- traversal ----------------------------------------------------------------------
 constexpr uint32_t kXcds    = 8;
 constexpr uint32_t kCntLine = 32;   // words per 128-byte line
+constexpr uint32_t kSpillDepth = 256;   // most global spill entries per lane (multiple of 32)
 struct TraceScene;
 struct TraceQueue {
     RaySoA          rays;
@@ -194,6 +195,7 @@ struct TraceQueue {
     // set by the launcher from TraceConfig: idle lanes that trigger a refill, and the number
     // of lanes still able to park a leaf below which a wave leaves the inner-node phase
     uint32_t refill_idle, park_min;
+    uint32_t spill_depth;   // entries per lane of the spill area (multiple of 32)
     uint32_t leaf_rounds;   // leaf-loop iterations per leaf phase before the wave resumes the
                             // inner-node phase (0: until no lane holds a leaf)
 };
@@ -205,6 +207,7 @@ struct TraceConfig {
     uint32_t refill = 0;
     uint32_t park_min = 0;
     uint32_t leaf_rounds = 0;
+    uint32_t spill_depth = kSpillDepth;   // entries per lane of the spill area given to the launch
 };
 hipError_t launch_trace_closest(const SceneDev &sc, const TraceQueue &q, uint32_t *spill, const TraceConfig &tc,
                                 hipStream_t s);
@@ -240,14 +243,21 @@ struct PostDev {
 hipError_t launch_post(const PostDev &p, const float4 *in, float4 *out, float4 *t0, float4 *t1, hipStream_t s);
 hipError_t launch_atrous(const float4 *colour, const float4 *normal, const float4 *albedo, float4 *out, float4 *t0,
                          float4 *t1, uint32_t w, uint32_t h, int levels, float sc, float sn, float sa, hipStream_t s);
-uint32_t trace_grid(int device, uint32_t waves_per_cu);
-uint64_t trace_spill_bytes(uint32_t grid);
+uint32_t trace_grid(int device, uint32_t blocks_per_cu);
+uint64_t trace_spill_bytes(uint32_t grid, uint32_t spill_depth);
 constexpr uint32_t kTraceBlock = 256;
-// default LDS stack entries per lane: 16 entries (34.3 KB per 256-lane block) let the
-// traversals of both wavefronts in flight hold their blocks on a CU at once (4 x 34.3 KB of
-// 160 KB), where 32 entries (67.6 KB per block) admit only one traversal's two blocks
+// default LDS stack entries per lane: 16 entries (34.8 KB per 256-lane block) let a CU hold
+// four blocks (139 of 160 KB), where 32 entries (67.6 KB per block) admit two
 constexpr uint32_t kStackLds   = 16;
-constexpr uint32_t kSpillDepth = 256;   // global spill entries per lane (multiple of kStackLds)
+// Default traversal blocks per CU: as many as fit with the default stack.  One launch then
+// fills the chip by itself, and a second wavefront's blocks start as the first one's end.
+// Two blocks (16 resident with both launches in flight) against four, 1080p: soup 8 passes
+// 16.4 -> 11.4 ms, 20 passes 28.1 -> 26.5, terrain 8 passes 16.1 -> 12.5, 2.07M camera rays
+// 0.83 -> 0.66 ms; three 13.0 / 27.8 / 13.6 / 0.70, eight (they queue) 12.2 / 29.0 / 13.1 / 0.79.
+constexpr uint32_t kTraceBlocksPerCu = 4;
+// ... and while the radiance cache trains beside the traversal, so that a training block
+// (31.7 KB) still fits next to the traversal's (3 x 34.8 KB)
+constexpr uint32_t kTraceBlocksPerCuTraining = 3;
 
 // ---- allocation-free queries (noalloc.hip) ---------------------------------------------
 // Layout of the per-device scratch array (byte offsets): counters (query_cnt words), leaf-order triangle and instance indices, u and v for callers that

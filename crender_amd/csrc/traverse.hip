@@ -11,7 +11,7 @@
 //     (blocks are dispatched round-robin over XCDs), so neighbouring rays share an L2;
 //     an XCD that drains its slice takes from the others.  A wave owns 64 rays from the
 //     start and takes further ones in chunks (RaySupply).
-//   * refill: when 32 or more lanes of a wave are idle, they take rays of the wave's chunk
+//   * refill: when 16 or more lanes of a wave are idle, they take rays of the wave's chunk
 //     by ballot rank.
 //   * per-lane short stack in LDS (entry-major (ref, distance) pairs; 8, 16 or 32 entries), spilled
 //     a full stack at a time to a per-lane global region when full.  Entries carry the child's entry
@@ -32,7 +32,9 @@ namespace {
 constexpr float kInf = __builtin_huge_valf();
 constexpr uint32_t kEmpty = kInvalidRef;
 constexpr uint32_t kMissKey = 0xFFFFFFFFu;
-constexpr uint32_t kRefillIdle = 32;           // default idle lanes that trigger a refill
+// default idle lanes that trigger a refill.  1080p soup 20 passes / terrain 8 passes with rays
+// from the wave's own chunk: 8 -> 26.4 / 12.5 ms, 16 -> 26.5 / 12.5, 24 -> 26.7 / 12.5, 32 -> 26.9 / 12.5
+constexpr uint32_t kRefillIdle = 16;
 // default: a wave leaves the inner-node phase for its parked leaves once fewer than 16 lanes
 // can still park one.  Measured on the 1M soup / 14.8M terrain at 1080p with two wavefronts in
 // flight: 4 -> 2690 / 3031 Mrays/s, 8 -> 2814 / 3090, 16 -> 2852-2861 / 3079, 32 -> 2758 / 2979.
@@ -208,17 +210,17 @@ template <uint32_t S>
 struct Stack {
     uint2    *s;        // LDS [S + 1][kTraceBlock] of (ref, entry distance bits); row S absorbs
                         // the writes of children that missed
-    uint4    *g;        // this lane's global spill: kSpillDepth (ref, distance) entries, contiguous, so
+    uint4    *g;        // this lane's global spill: `depth` (ref, distance) entries, contiguous, so
                         // that a spill of S entries writes S * 8 bytes of whole lines (uint4 = 2 entries)
     uint32_t  tid;
-    uint32_t  sp, gsp;
+    uint32_t  sp, gsp, depth;
 
     uint32_t *err;
 
     __device__ __forceinline__ void push(uint32_t ref, float dist)
     {
         if (sp == S) {
-            if (gsp + S > kSpillDepth) {
+            if (gsp + S > depth) {
                 // cannot happen for trees admitted at commit; never write out of bounds
                 *err = 1u;
                 return;
@@ -433,7 +435,8 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
 
     Stack<S> st;
     st.s      = s_stack;
-    st.g      = reinterpret_cast<uint4 *>(spill) + (size_t)(blockIdx.x * blockDim.x + threadIdx.x) * (kSpillDepth / 2);
+    st.g      = reinterpret_cast<uint4 *>(spill) + (size_t)(blockIdx.x * blockDim.x + threadIdx.x) * (q.spill_depth / 2);
+    st.depth  = q.spill_depth;
     st.tid    = threadIdx.x;
     st.sp = st.gsp = 0;
     st.err = q.error;
@@ -676,17 +679,16 @@ uint32_t trace_grid(int device, uint32_t blocks_per_cu)
 {
     hipDeviceProp_t p;
     if (hipGetDeviceProperties(&p, device) != hipSuccess) return 1024;
-    // two 256-lane blocks per CU: fewer rays in flight keep more of the BVH in cache
-    if (blocks_per_cu == 0) blocks_per_cu = 2;
+    if (blocks_per_cu == 0) blocks_per_cu = kTraceBlocksPerCu;
     uint32_t g = (uint32_t)p.multiProcessorCount * blocks_per_cu;
     // whole multiple of the XCD count so every XCD gets the same number of blocks
     g = (g + kXcds - 1) / kXcds * kXcds;
     return g;
 }
 
-uint64_t trace_spill_bytes(uint32_t grid)
+uint64_t trace_spill_bytes(uint32_t grid, uint32_t spill_depth)
 {
-    return (uint64_t)grid * kTraceBlock * kSpillDepth * 2u * sizeof(uint32_t);
+    return (uint64_t)grid * kTraceBlock * spill_depth * 2u * sizeof(uint32_t);
 }
 
 namespace {
@@ -700,6 +702,7 @@ hipError_t dispatch_trace(uint32_t width, const TraceConfig &tc, const SceneDev 
     TraceQueue q   = qin;
     q.refill_idle  = tc.refill ? std::min(tc.refill, 64u) : kRefillIdle;
     q.park_min     = tc.park_min ? std::min(tc.park_min, 64u) : kParkMin;
+    q.spill_depth  = tc.spill_depth;
     q.leaf_rounds  = tc.leaf_rounds ? (tc.leaf_rounds > 64u ? 0u : tc.leaf_rounds) : kLeafRounds;
     if (!kMulti && q.tstats) {
         // instrumented traversal: one stack depth (the counts do not depend on it)

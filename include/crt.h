@@ -119,7 +119,7 @@ typedef struct crt_options {
     int32_t  device;        /* HIP device ordinal */
     uint32_t bvh_width;     /* 0 = autotune, 2/4/8 */
     uint32_t max_leaf;      /* 0 = default (4) */
-    uint32_t trace_waves_per_cu; /* 0 = default persistent occupancy (8 waves per CU) */
+    uint32_t trace_waves_per_cu; /* 0 = default persistent occupancy (16 waves per CU) */
     uint32_t flags;         /* CRT_FLAG_* */
     uint32_t trace_stack;   /* LDS stack entries per traversal lane: 0 (= 16), 8, 16 or 32 */
     uint32_t wavefront_paths; /* camera paths per renderer wavefront: 0 = 2^24 (2^23 for a
@@ -127,7 +127,7 @@ typedef struct crt_options {
                                  floor(wavefront_paths / (W*H)) sample passes (1 to 8).  Two
                                  wavefronts are in flight (two sets of path buffers, two streams). */
     uint32_t trace_refill;  /* traversal waves fetch new rays once this many of their 64 lanes
-                               are idle: 0 = default (32), else 1 to 64 */
+                               are idle: 0 = default (16), else 1 to 64 */
     uint32_t trace_park_min;/* the inner-node phase of a wave ends once fewer than this many
                                lanes can still park a leaf: 0 = default (16), else 1 to 64 */
     uint32_t trace_leaf_rounds; /* leaf-loop rounds after which a wave whose parked leaves are
