@@ -156,12 +156,11 @@ struct crt_nrc {
     crt_context    *ctx = nullptr;
     crt_nrc_options opt{};
     float          *params = nullptr, *m = nullptr, *v = nullptr;
-    __bf16         *W = nullptr, *WT = nullptr;
-    __bf16         *act = nullptr;
-    float          *partial = nullptr, *partial_loss = nullptr, *grad = nullptr;
+    __bf16         *WF = nullptr, *WB = nullptr;   // weights in the matrix products' order (nrc.hip)
+    float          *partial = nullptr, *partial_loss = nullptr, *grad = nullptr;   // grad: the loss follows
+    float          *grad_host = nullptr;   // pinned: gradient and loss of the last call
     float          *q_stage = nullptr, *t_stage = nullptr, *o_stage = nullptr;
     uint32_t        stage_cap = 0;
-    uint32_t        tiles_alloc = 0;
     uint64_t        step = 0;
     int             users = 0;   // renderers the cache is attached to
     // Training after a renderer's wavefront runs on its own stream, beside the next
@@ -223,7 +222,7 @@ struct crt_renderer {
     crt_nrc               *nrc = nullptr;
     crt_nrc_render_options nopt{};
     double                 ms_nrc_train = 0.0;
-    uint32_t               loss_tiles = 0;   // tiles of the last training step (loss partials)
+    uint32_t               loss_parts = 0;   // loss partials of the last training step
     uint32_t               nrc_warm_done = 0;   // warm-up passes run since set_nrc
     // the cache's predictions became non-finite: it is not used again until set_nrc, and the
     // sample passes that used it are dropped and rendered again
@@ -783,7 +782,7 @@ int enqueue_tail(crt_renderer *r, PassTicket &t)
         // unconditional: a wait on an event that was never recorded is a no-op, and the
         // pending flag may have been cleared by a concurrent nrc_wait_training
         HIP_CHECK(hipStreamWaitEvent(s, r->nrc->ev_trained, 0));
-        HIP_CHECK(nrc_launch_infer_dev(b.nq, b.nq_out, b.cnt + kCntNrcQ, b.P, r->nrc->WT, s));
+        HIP_CHECK(nrc_launch_infer_dev(b.nq, b.nq_out, b.cnt + kCntNrcQ, b.P, r->nrc->WF, s));
         HIP_CHECK(launch_nrc_apply(b, s));
         if (t.timing) {
             t.ev_acc = crt_renderer::kEvAcc;
@@ -974,9 +973,9 @@ int nrc_train_step(crt_renderer *r, const PathBuffers &t, uint32_t mult, uint32_
     for (uint32_t k = 0; k < steps; ++k) {
         const float *q  = t.tq + (size_t)k * batch * 13;
         const float *tt = t.tt + (size_t)k * batch * 3;
-        HIP_CHECK(nrc_launch_train(q, tt, batch, n->W, n->WT, n->act, n->partial, n->partial_loss, s));
+        HIP_CHECK(nrc_launch_train(q, tt, batch, n->WF, n->WB, n->partial, n->partial_loss, s));
         n->step++;
-        HIP_CHECK(nrc_launch_adam(n->partial, nrc_partial_rows(batch), n->params, n->m, n->v, n->W, n->WT, n->opt.lr,
+        HIP_CHECK(nrc_launch_adam(n->partial, nrc_partial_rows(batch), n->params, n->m, n->v, n->WF, n->WB, n->opt.lr,
                                   n->opt.beta1, n->opt.beta2, n->opt.eps, n->step, 1, s));
     }
     HIP_CHECK(hipEventRecord(r->ev_train[1], s));
@@ -984,7 +983,7 @@ int nrc_train_step(crt_renderer *r, const PathBuffers &t, uint32_t mult, uint32_
     HIP_CHECK(hipEventRecord(n->ev_trained, s));
     n->pending = true;
     // the loss of the last step (sum of its per-tile partials) is read when stats ask for it
-    r->loss_tiles = (batch + 63) / 64;
+    r->loss_parts = nrc_partial_rows(batch);
     return CRT_OK;
 }
 
@@ -2333,10 +2332,10 @@ int crt_renderer_current_stats(crt_renderer *r, crt_stats *stats)
             stats->node_idle_leaf_wait += ts[7];
         }
     }
-    if (r->nrc && r->loss_tiles) {
+    if (r->nrc && r->loss_parts) {
         if (int wst = nrc_wait_training(r->nrc)) return wst;
         std::lock_guard<std::mutex> g(r->nrc->mu);
-        std::vector<float> pl(r->loss_tiles);
+        std::vector<float> pl(r->loss_parts);
         HIP_CHECK(hipStreamSynchronize(r->ctx->stream));
         HIP_CHECK(hipMemcpy(pl.data(), r->nrc->partial_loss, sizeof(float) * pl.size(), hipMemcpyDeviceToHost));
         double acc = 0.0;
@@ -2440,7 +2439,7 @@ extern "C" int crt_renderer_set_nrc(crt_renderer *r, crt_nrc *nrc, const crt_nrc
     r->nrc           = nrc;
     r->nopt          = o;
     r->nrc_warm_done = 0;
-    r->loss_tiles    = 0;
+    r->loss_parts    = 0;
     r->nrc_failed    = false;
     r->nrc_discarded = 0;
     r->train_timed   = false;
@@ -2453,8 +2452,6 @@ extern "C" int crt_renderer_set_nrc(crt_renderer *r, crt_nrc *nrc, const crt_nrc
 
 
 namespace {
-
-uint32_t nrc_tiles_alloc(uint32_t max_batch) { return ((max_batch + 63) / 64 + 3) / 4 * 4; }
 
 int nrc_stage(crt_nrc *n, uint32_t count)
 {
@@ -2495,7 +2492,7 @@ int nrc_upload(crt_nrc *n, const float *host)
     HIP_CHECK(hipMemcpyAsync(n->params, host, sizeof(float) * kNrcParams, hipMemcpyHostToDevice, s));
     HIP_CHECK(hipMemsetAsync(n->m, 0, sizeof(float) * kNrcParams, s));
     HIP_CHECK(hipMemsetAsync(n->v, 0, sizeof(float) * kNrcParams, s));
-    HIP_CHECK(nrc_launch_adam(nullptr, 0, n->params, n->m, n->v, n->W, n->WT, 0, 0, 0, 0, 1, 0, s));
+    HIP_CHECK(nrc_launch_adam(nullptr, 0, n->params, n->m, n->v, n->WF, n->WB, 0, 0, 0, 0, 1, 0, s));
     HIP_CHECK(hipStreamSynchronize(s));
     n->step = 0;
     return CRT_OK;
@@ -2544,19 +2541,20 @@ int crt_nrc_create(crt_context *ctx, const crt_nrc_options *opt, crt_nrc **out)
         hipEventCreateWithFlags(&n->ev_targets, hipEventDisableTiming) != hipSuccess ||
         hipEventCreateWithFlags(&n->ev_trained, hipEventDisableTiming) != hipSuccess)
         st = fail(CRT_ERR_HIP, "cache stream / events");
-    n->tiles_alloc = nrc_tiles_alloc(n->opt.max_batch);
+    const uint32_t parts = nrc_partial_rows(n->opt.max_batch);
     auto A = [&](auto **p, size_t c) {
         if (st == CRT_OK && dalloc(p, c) != hipSuccess) st = fail(CRT_ERR_OUT_OF_MEMORY, "nrc allocation");
     };
     A(&n->params, kNrcParams);
     A(&n->m, kNrcParams);
     A(&n->v, kNrcParams);
-    A(&n->W, kNrcParams);
-    A(&n->WT, kNrcParams);
-    A(&n->grad, kNrcParams);
-    A(&n->act, (size_t)n->tiles_alloc * 64 * kNrcActs);
-    A(&n->partial, (size_t)n->tiles_alloc * kNrcParams);
-    A(&n->partial_loss, n->tiles_alloc);
+    A(&n->WF, kNrcParams);
+    A(&n->WB, kNrcParams);
+    A(&n->grad, kNrcParams + 1);
+    A(&n->partial, (size_t)parts * kNrcParams);
+    A(&n->partial_loss, parts);
+    if (st == CRT_OK && hipHostMalloc((void **)&n->grad_host, sizeof(float) * (kNrcParams + 1)) != hipSuccess)
+        st = fail(CRT_ERR_OUT_OF_MEMORY, "pinned host allocation");
     if (st == CRT_OK) {
         std::vector<float> w;
         nrc_init_params(w, n->opt.seed);
@@ -2579,9 +2577,10 @@ int crt_nrc_destroy(crt_nrc *n)
     if (n->ev_targets) (void)hipEventDestroy(n->ev_targets);
     if (n->ev_trained) (void)hipEventDestroy(n->ev_trained);
     if (n->ts) (void)hipStreamDestroy(n->ts);
-    void *ps[] = {n->params, n->m, n->v, n->W, n->WT, n->grad, n->act, n->partial, n->partial_loss,
+    void *ps[] = {n->params, n->m, n->v, n->WF, n->WB, n->grad, n->partial, n->partial_loss,
                   n->q_stage, n->t_stage, n->o_stage};
     for (void *p : ps) dfree(p);
+    if (n->grad_host) (void)hipHostFree(n->grad_host);
     n->ctx->live--;
     delete n;
     return CRT_OK;
@@ -2615,34 +2614,24 @@ int crt_nrc_infer(crt_nrc *n, const float *queries, uint32_t count, float *out, 
     if (st) return st;
     float *o = memory == CRT_MEM_DEVICE ? out : n->o_stage;
     hipStream_t s = n->ctx->stream;
-    HIP_CHECK(nrc_launch_infer(q, o, count, n->WT, s));
+    HIP_CHECK(nrc_launch_infer(q, o, count, n->WF, s));
     if (memory == CRT_MEM_HOST) HIP_CHECK(hipMemcpyAsync(out, o, sizeof(float) * 3 * count, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
     return CRT_OK;
 }
 
-static int nrc_fwd_bwd(crt_nrc *n, const float *queries, const float *targets, uint32_t count, int memory,
-                       float *loss)
+// Enqueues forward and backward of a batch: gradient and loss partials (n->mu is held).
+static int nrc_fwd_bwd(crt_nrc *n, const float *queries, const float *targets, uint32_t count, int memory)
 {
     if (count > n->opt.max_batch) return fail(CRT_ERR_INVALID_ARG, "batch larger than max_batch");
-    if (int wst = nrc_wait_locked(n)) return wst;   // training enqueued by renderers (n->mu is held)
+    if (int wst = nrc_wait_locked(n)) return wst;   // training enqueued by renderers
     int st = memory == CRT_MEM_HOST ? nrc_stage(n, count) : CRT_OK;
     if (st) return st;
     const float *q = nrc_input(n, queries, (size_t)count * kNrcQuery, n->q_stage, memory, &st);
     if (st) return st;
     const float *t = nrc_input(n, targets, (size_t)count * 3, n->t_stage, memory, &st);
     if (st) return st;
-    hipStream_t s = n->ctx->stream;
-    HIP_CHECK(nrc_launch_train(q, t, count, n->W, n->WT, n->act, n->partial, n->partial_loss, s));
-    if (loss) {
-        const uint32_t tiles = (count + 63) / 64;
-        std::vector<float> pl(tiles);
-        HIP_CHECK(hipMemcpyAsync(pl.data(), n->partial_loss, sizeof(float) * tiles, hipMemcpyDeviceToHost, s));
-        HIP_CHECK(hipStreamSynchronize(s));
-        double acc = 0.0;
-        for (float x : pl) acc += x;
-        *loss = (float)acc;
-    }
+    HIP_CHECK(nrc_launch_train(q, t, count, n->WF, n->WB, n->partial, n->partial_loss, n->ctx->stream));
     return CRT_OK;
 }
 
@@ -2652,11 +2641,16 @@ int crt_nrc_gradient(crt_nrc *n, const float *queries, const float *targets, uin
     if (!n || !grad || ((!queries || !targets) && count)) return fail(CRT_ERR_INVALID_ARG, "null argument");
     if (count == 0) return fail(CRT_ERR_INVALID_ARG, "empty batch");
     std::lock_guard<std::mutex> g(n->mu);
-    int st = nrc_fwd_bwd(n, queries, targets, count, memory, loss);
+    int st = nrc_fwd_bwd(n, queries, targets, count, memory);
     if (st) return st;
-    HIP_CHECK(nrc_launch_sum_partials(n->partial, nrc_partial_rows(count), n->grad, n->ctx->stream));
-    HIP_CHECK(hipMemcpyAsync(grad, n->grad, sizeof(float) * kNrcParams, hipMemcpyDeviceToHost, n->ctx->stream));
-    HIP_CHECK(hipStreamSynchronize(n->ctx->stream));
+    hipStream_t s = n->ctx->stream;
+    HIP_CHECK(nrc_launch_sum_partials(n->partial, n->partial_loss, nrc_partial_rows(count), n->grad, s));
+    // gradient and loss in one copy to pinned memory: a copy to the caller's pageable memory
+    // is staged by the runtime, once per copy
+    HIP_CHECK(hipMemcpyAsync(n->grad_host, n->grad, sizeof(float) * (kNrcParams + 1), hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipStreamSynchronize(s));
+    std::memcpy(grad, n->grad_host, sizeof(float) * kNrcParams);
+    if (loss) *loss = n->grad_host[kNrcParams];
     return CRT_OK;
 }
 
@@ -2666,12 +2660,20 @@ int crt_nrc_train_step(crt_nrc *n, const float *queries, const float *targets, u
     if (int wst = nrc_wait_training(n)) return wst;   // training enqueued by renderers
     if (count == 0) return CRT_OK;
     std::lock_guard<std::mutex> g(n->mu);
-    int st = nrc_fwd_bwd(n, queries, targets, count, memory, loss);
+    int st = nrc_fwd_bwd(n, queries, targets, count, memory);
     if (st) return st;
+    hipStream_t    s     = n->ctx->stream;
+    const uint32_t parts = nrc_partial_rows(count);
     n->step++;
-    HIP_CHECK(nrc_launch_adam(n->partial, nrc_partial_rows(count), n->params, n->m, n->v, n->W, n->WT, n->opt.lr,
-                              n->opt.beta1, n->opt.beta2, n->opt.eps, n->step, 1, n->ctx->stream));
-    HIP_CHECK(hipStreamSynchronize(n->ctx->stream));
+    HIP_CHECK(nrc_launch_adam(n->partial, parts, n->params, n->m, n->v, n->WF, n->WB, n->opt.lr, n->opt.beta1,
+                              n->opt.beta2, n->opt.eps, n->step, 1, s));
+    if (loss) HIP_CHECK(hipMemcpyAsync(n->grad_host, n->partial_loss, sizeof(float) * parts, hipMemcpyDeviceToHost, s));
+    HIP_CHECK(hipStreamSynchronize(s));
+    if (loss) {
+        double acc = 0.0;
+        for (uint32_t k = 0; k < parts; ++k) acc += n->grad_host[k];
+        *loss = (float)acc;
+    }
     return CRT_OK;
 }
 

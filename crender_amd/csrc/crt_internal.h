@@ -403,7 +403,7 @@ hipError_t launch_fill(float4 *p, uint64_t n, float v, hipStream_t s);
 hipError_t launch_nrc_apply(const PathBuffers &b, hipStream_t s);
 hipError_t launch_nrc_targets(const PathBuffers &b, uint32_t rec_slots, uint32_t max_out, uint32_t train_live,
                               hipStream_t s);
-hipError_t nrc_launch_infer_dev(const float *q, float *out, const uint32_t *n_dev, uint32_t n_max, const __bf16 *WT,
+hipError_t nrc_launch_infer_dev(const float *q, float *out, const uint32_t *n_dev, uint32_t n_max, const __bf16 *WF,
                                 hipStream_t s);
 hipError_t launch_batch_generate(const BatchDev &bd, const PathBuffers &b, hipStream_t s);
 hipError_t launch_shade_multi(const BatchDev &bd, const PathBuffers &b, uint32_t bounce, uint32_t cur, hipStream_t s);

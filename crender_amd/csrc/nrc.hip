@@ -4,23 +4,26 @@
 // Network: 96 input features (12-frequency sin/cos of the position, direction, normal,
 // albedo, roughness, a constant 1, zero padding) -> 5 hidden layers of 64 (ReLU) -> 32
 // outputs of which 0..2 are RGB radiance.  No biases (the constant feature biases the
-// first layer).  Weights: FP32 master copy updated by Adam, bf16 copies in row-major
-// W[k][n] (B operand of the backward data product) and transposed WT[n][k] (B operand of
-// the forward product).
+// first layer).  Weights: FP32 master copy updated by Adam, and two bf16 copies in the
+// order the matrix instructions read them (fwd_pos, bwd_pos).
 //
-// MFMA operand mapping used throughout (one 16x16 output tile, 32-deep reduction):
-//   A: lane l supplies row (l % 16), reduction elements 8*(l/16) .. 8*(l/16)+7
-//   B: lane l supplies column (l % 16), the same reduction elements
-//   D: lane l holds rows 4*(l/16) .. 4*(l/16)+3 of column (l % 16)
-// A and B use the same element mapping, so the reduction is exact whatever order the
-// hardware sums the 32 products in.
+// MFMA operand mapping (v_mfma_f32_16x16x32_bf16: one 16x16 output tile, 32-deep reduction;
+// r = lane % 16, g = lane / 16):
+//   A: lane supplies row r, eight reduction elements j = 0 .. 7 of its group g
+//   B: lane supplies column r, the same reduction elements
+//   D: lane holds rows 4g .. 4g + 3 of column r
+// A and B name their reduction elements alike, so any assignment of the 32 elements to
+// (g, j) gives the same sums.  Every product is formed transposed: A = weights (rows =
+// output features), B = activations (columns = samples).  The result then has a sample per
+// lane and four consecutive features in its registers, and two result tiles together are,
+// converted to bf16, the B operand of the next layer with reduction element (g, j) =
+// feature 32 c + 16 (j / 4) + 4 g + j % 4.  Activations never leave the registers; the
+// weights are stored in that order instead, so a fragment is one 16-byte load per lane.
+// The 96 input features are assigned to (g, j) so that every lane group computes nine sin/cos
+// pairs and up to six other inputs (kmap0).
 //
-// Inference: each wave owns 64 samples (4 row tiles of 16); activations between layers go
-// through the wave's slice of LDS.  Training: a workgroup of four waves owns 64 samples and
-// splits every layer's output columns over its waves; it stores every layer's input
-// activations (sample-major, bf16) in a global scratch so the backward pass can form
-// dW = X^T G, writes per-tile gradient partials (no atomics), and the Adam kernel sums the
-// partials per parameter.
+// A product with the identity turns a tile with a sample per lane into one with a feature per
+// lane (exact: one term per sum), the operand form of dW = X^T G.
 #include <hip/hip_runtime.h>
 #include <math.h>
 #include "crt_internal.h"
@@ -31,321 +34,450 @@ namespace crt {
 namespace {
 
 typedef __bf16 bf16;
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+typedef short  s16x4 __attribute__((ext_vector_type(4)));
 typedef float  f32x4 __attribute__((ext_vector_type(4)));
+
+constexpr int kFrag = 512;   // elements of one weight fragment: 64 lanes x 8
 
 __device__ __forceinline__ f32x4 mma(bf16x8 a, bf16x8 b, f32x4 c)
 {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
+// 16-deep product: lane supplies reduction elements 4g .. 4g + 3
+__device__ __forceinline__ f32x4 mma16(bf16x4 a, bf16x4 b, f32x4 c)
+{
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(__builtin_bit_cast(s16x4, a), __builtin_bit_cast(s16x4, b), c, 0, 0, 0);
+}
+
+// A value the compiler takes for new at each call: the weight addresses of a tile go through
+// it, or every fragment would be loaded before the loop over tiles and spilled.
+__device__ __forceinline__ int fresh(int x)
+{
+    asm volatile("" : "+v"(x));
+    return x;
+}
 
 __device__ __forceinline__ bf16 to_bf16(float x) { return (bf16)x; }   // round to nearest even
-__device__ __forceinline__ float from_bf16(bf16 x) { return (float)x; }
-
-constexpr int kXStride = kNrcIn + 8;    // LDS row stride (bf16) of the sample-major activations
-constexpr int kGStride = kNrcHid + 8;
+__device__ __forceinline__ bf16x8 ld8(const bf16 *p) { return *reinterpret_cast<const bf16x8 *>(p); }
 
 __host__ __device__ constexpr int layer_k(int l) { return l == 0 ? kNrcIn : kNrcHid; }
 __host__ __device__ constexpr int layer_n(int l) { return l == kNrcLayers - 1 ? kNrcOut : kNrcHid; }
-__host__ __device__ constexpr int act_off(int l) { return l == 0 ? 0 : kNrcIn + (l - 1) * kNrcHid; }
+// first forward fragment of layer l: (row tile, 32-deep chunk) fragments, 12 + 4 x 8 + 4 = 48
+__host__ __device__ constexpr int fwd_frag(int l) { return l == 0 ? 0 : 12 + 8 * (l - 1); }
+// first backward fragment of layer l >= 1: 4 x 8 + 4 = 36
+__host__ __device__ constexpr int bwd_frag(int l) { return 8 * (l - 1); }
 
-// features of one query: p[3] in [0,1], d[3], n[3], albedo[3], roughness
-__device__ __forceinline__ void encode_row(const float *q, bf16 *row)
+// input row (0 .. 95) of reduction element (chunk, g, j) of the first layer
+__device__ __forceinline__ int kmap0(int chunk, int g, int j)
 {
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-        float f = 3.14159265358979323846f;
-#pragma unroll
-        for (int k = 0; k < 12; ++k) {
-            const float arg = q[c] * f;
-            float s, co;
-            sincosf(arg, &s, &co);
-            row[c * 24 + 2 * k]     = to_bf16(s);
-            row[c * 24 + 2 * k + 1] = to_bf16(co);
-            f *= 2.0f;
+    const int s = 8 * chunk + j;   // the lane group's feature 0 .. 23
+    if (s < 18) return 18 * g + s;                          // sin / cos pairs 9 g .. 9 g + 8
+    if (s < 21) return g < 3 ? 72 + 3 * g + (s - 18) : 81 + (s - 18);   // direction, normal, albedo | roughness, 1, 0
+    return 84 + 3 * g + (s - 21);                           // zero padding
+}
+
+// position of weight (k, c) of layer l among the forward fragments
+__device__ __forceinline__ int fwd_pos(int l, int k, int c)
+{
+    int kc, g, j;
+    if (l > 0) {
+        kc = k >> 5;
+        g  = (k >> 2) & 3;
+        j  = ((k >> 4) & 1) * 4 + (k & 3);
+    } else {
+        int s;
+        if (k < 72) {
+            g = k / 18;
+            s = k - 18 * g;
+        } else if (k < 84) {
+            g = (k - 72) / 3;
+            s = 18 + (k - 72) % 3;
+        } else {
+            g = (k - 84) / 3;
+            s = 21 + (k - 84) % 3;
         }
+        kc = s >> 3;
+        j  = s & 7;
+    }
+    const int nk = layer_k(l) / 32;
+    return (fwd_frag(l) + (c >> 4) * nk + kc) * kFrag + (g * 16 + (c & 15)) * 8 + j;
+}
+
+// position of weight (k, c) of layer l >= 1 among the backward fragments (rows = input
+// features, reduction over the output features)
+__device__ __forceinline__ int bwd_pos(int l, int k, int c)
+{
+    const int nc = layer_n(l) / 32, g = (c >> 2) & 3, j = ((c >> 4) & 1) * 4 + (c & 3);
+    return (bwd_frag(l) + (k >> 4) * nc + (c >> 5)) * kFrag + (g * 16 + (k & 15)) * 8 + j;
+}
+
+// The lane's 24 input features of its sample (three B operands).  q: the sample's query (any
+// query of the batch for the lanes beyond it, whose results are not used).  Pair p = 9 g + m is sin and cos of a 2^f with a the
+// FP32 product of pi and x_c, c = p / 12, f = p % 12.  a / 2 pi is formed once per component
+// as a sum of two floats; scaling both by 2^f and taking the fraction of the first are exact,
+// so the hardware sine and cosine (which take revolutions) see an argument within 2^-25 of a
+// revolution, with no reduction of the argument per feature.
+__device__ __forceinline__ void encode(const float *q, int g, bf16x8 (&f)[3])
+{
+    const int   c0 = 9 * g / 12, c1 = min(c0 + 1, 2);
+    const float x0 = q[c0], x1 = q[c1];
+    float e[3];
+    e[0] = q[g < 3 ? 3 + 3 * g : 12];
+    e[1] = q[g < 3 ? 4 + 3 * g : 12];
+    e[2] = q[g < 3 ? 5 + 3 * g : 12];
+    if (g == 3) {
+        e[1] = 1.0f;
+        e[2] = 0.0f;
+    }
+    const int f0 = 9 * g - 12 * c0;   // first frequency: 0, 9, 6, 3
+    constexpr double kInv2Pi = 0.15915494309189533577;
+    constexpr float  kHi = (float)kInv2Pi, kLo = (float)(kInv2Pi - (double)kHi);
+    const float a0 = x0 * 3.14159265358979323846f, a1 = x1 * 3.14159265358979323846f;
+    const float h0 = a0 * kHi, h1 = a1 * kHi;
+    const float l0 = fmaf(a0, kHi, -h0) + a0 * kLo, l1 = fmaf(a1, kHi, -h1) + a1 * kLo;
+    float v[24];
+#pragma unroll
+    for (int m = 0; m < 9; ++m) {
+        const bool  own = f0 + m < 12;
+        const float sc  = __uint_as_float((uint32_t)(127 + (own ? f0 + m : f0 + m - 12)) << 23);
+        const float rev = fmaf(own ? l0 : l1, sc, __builtin_amdgcn_fractf((own ? h0 : h1) * sc));
+        v[2 * m]     = __builtin_amdgcn_sinf(rev);
+        v[2 * m + 1] = __builtin_amdgcn_cosf(rev);
     }
 #pragma unroll
-    for (int k = 0; k < 10; ++k) row[72 + k] = to_bf16(q[3 + k]);
-    row[82] = to_bf16(1.0f);
-#pragma unroll
-    for (int k = 83; k < kNrcIn; ++k) row[k] = to_bf16(0.0f);
-}
-
-__device__ __forceinline__ bf16x8 lds8(const bf16 *p) { return *reinterpret_cast<const bf16x8 *>(p); }
-__device__ __forceinline__ bf16x8 glb8(const bf16 *p) { return *reinterpret_cast<const bf16x8 *>(p); }
-
-// Forward product of one layer for the wave's 64 rows held in X (sample-major, LDS).
-template <int L>
-__device__ __forceinline__ void layer_fwd(const bf16 *X, const bf16 *WT, f32x4 (&acc)[4][4])
-{
-    constexpr int K = layer_k(L), N = layer_n(L), NT = N / 16;
-    const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
-#pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int ct = 0; ct < 4; ++ct) acc[rt][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    const bf16 *w = WT + nrc_w_off(L);
-#pragma unroll
-    for (int kk = 0; kk < K / 32; ++kk) {
-        bf16x8 a[4];
-#pragma unroll
-        for (int rt = 0; rt < 4; ++rt) a[rt] = lds8(X + (rt * 16 + r16) * kXStride + kk * 32 + 8 * g);
-#pragma unroll
-        for (int ct = 0; ct < NT; ++ct) {
-            const bf16x8 b = glb8(w + (ct * 16 + r16) * K + kk * 32 + 8 * g);
-#pragma unroll
-            for (int rt = 0; rt < 4; ++rt) acc[rt][ct] = mma(a[rt], b, acc[rt][ct]);
-        }
+    for (int k = 0; k < 3; ++k) {
+        v[18 + k] = e[k];
+        v[21 + k] = 0.0f;
     }
+#pragma unroll
+    for (int c = 0; c < 3; ++c)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[c][j] = to_bf16(v[8 * c + j]);
 }
 
-// ReLU and write the layer output back into X (sample-major) as the next layer's input.
-template <int N>
-__device__ __forceinline__ void store_relu(bf16 *X, const f32x4 (&acc)[4][4])
+// max(x, 0), 0 for NaN, in one instruction where fmaxf takes two (it first quiets its operand).
+// The upper bound changes nothing: the largest float, like infinity, becomes infinity in bf16.
+__device__ __forceinline__ float relu(float x) { return __builtin_amdgcn_fmed3f(x, 0.0f, 3.402823466e+38f); }
+
+// D tiles 2c, 2c + 1 as the B operand of the next product; relu: clamp below at 0.
+template <bool kRelu>
+__device__ __forceinline__ bf16x8 pack(f32x4 lo, f32x4 hi)
 {
-    const int lane = threadIdx.x & 63, r16 = lane & 15, g = lane >> 4;
+    bf16x8 r;
 #pragma unroll
-    for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-        for (int ct = 0; ct < N / 16; ++ct)
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                X[(rt * 16 + 4 * g + i) * kXStride + ct * 16 + r16] = to_bf16(fmaxf(acc[rt][ct][i], 0.0f));
+    for (int i = 0; i < 4; ++i) {
+        r[i]     = to_bf16(kRelu ? relu(lo[i]) : lo[i]);
+        r[4 + i] = to_bf16(kRelu ? relu(hi[i]) : hi[i]);
+    }
+    return r;
 }
 
-template <int L>
-__device__ __forceinline__ void hidden(bf16 *X, const bf16 *WT)
+// acc[rt][ct] = rows 16 rt .. of (weights x activations) for CT tiles of 16 samples.
+template <int NK, int NR, int CT, class Load>
+__device__ __forceinline__ void product(Load frag, const bf16x8 (&b)[3][CT], f32x4 (&acc)[4][CT])
 {
-    f32x4 acc[4][4];
-    layer_fwd<L>(X, WT, acc);
-    __syncthreads();
-    store_relu<kNrcHid>(X, acc);
-    __syncthreads();
+#pragma unroll
+    for (int rt = 0; rt < NR; ++rt)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int kc = 0; kc < NK; ++kc)
+#pragma unroll
+        for (int rt = 0; rt < NR; ++rt) {
+            const bf16x8 a = frag(rt * NK + kc);
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct) acc[rt][ct] = mma(a, b[kc][ct], acc[rt][ct]);
+        }
 }
+
+template <int CT>
+__device__ __forceinline__ void activate(const f32x4 (&acc)[4][CT], bf16x8 (&b)[3][CT])
+{
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) b[c][ct] = pack<true>(acc[2 * c][ct], acc[2 * c + 1][ct]);
+}
+
+// Inference.  Bound by vector instructions (conversion, ReLU and the encoding: about 1000 and 72
+// transcendental ones per 64 samples, 65 us for 2.07M samples) beside the matrix pipe (184
+// products of 16 cycles, 39 us) and the query bytes (133 MB).  A block of four waves keeps the
+// 46 used weight fragments in LDS (46 KB: three blocks, 12 waves per CU, which 159 registers
+// a lane also allow) and loops over tiles of 256 samples; a wave owns 64 samples, so a
+// fragment read from LDS serves four products.  2,073,600 queries: 409 us with activations
+// passed through LDS, weights re-read from L2 by every wave and sincosf; 110 us like this.
+constexpr int kInferWaves = 4, kInferBlocks = 768;
+constexpr int kInferFrags = 46;   // 44 of the hidden layers, row tile 0 of the output
 
 // n_dev (when set) is a device-side count, clamped to the buffers' capacity n_host.
-__global__ __launch_bounds__(256) void k_nrc_infer(const float *__restrict__ q, float *__restrict__ out, uint32_t n_host,
-                                                   const uint32_t *__restrict__ n_dev, const bf16 *__restrict__ WT)
+__global__ __launch_bounds__(64 * kInferWaves, 3) void k_nrc_infer(const float *__restrict__ q, float *__restrict__ out,
+                                                                   uint32_t n_host, const uint32_t *__restrict__ n_dev,
+                                                                   const bf16 *__restrict__ WF)
 {
-    __shared__ bf16 xs[4 * 64 * kXStride];
+    __shared__ bf16x8 ws[kInferFrags * 64];
     const uint32_t n = n_dev ? min(*n_dev, n_host) : n_host;
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
-    bf16 *X = xs + wv * 64 * kXStride;
-    const uint32_t ntiles = (n + 255) / 256;
+    const int lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const uint32_t wv = threadIdx.x >> 6;
+    constexpr uint32_t kTile = 64 * kInferWaves;
+    const uint32_t ntiles = (uint32_t)(((uint64_t)n + kTile - 1) / kTile);
+    if (blockIdx.x >= ntiles) return;
+    for (int i = threadIdx.x; i < kInferFrags * 64; i += 64 * kInferWaves) ws[i] = ld8(WF + (size_t)i * 8);
+    __syncthreads();
     for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const uint32_t s0 = tile * 256 + wv * 64;
-        const uint32_t s  = s0 + lane;
-        float qq[kNrcQuery];
+        const uint32_t s0 = tile * kTile + wv * 64;
+        bf16x8 b[3][4];
 #pragma unroll
-        for (int k = 0; k < kNrcQuery; ++k) qq[k] = s < n ? q[(size_t)s * kNrcQuery + k] : 0.0f;
-        encode_row(qq, X + lane * kXStride);
-        __syncthreads();
-        hidden<0>(X, WT);
-        hidden<1>(X, WT);
-        hidden<2>(X, WT);
-        hidden<3>(X, WT);
-        hidden<4>(X, WT);
+        for (int ct = 0; ct < 4; ++ct) {
+            const uint32_t s = s0 + ct * 16 + r;
+            bf16x8 f[3];
+            encode(q + (size_t)min(s, n - 1u) * kNrcQuery, g, f);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) b[c][ct] = f[c];
+        }
         f32x4 acc[4][4];
-        layer_fwd<5>(X, WT, acc);
+#define FWD(L, NK, NR)                                                                        \
+    {                                                                                         \
+        const bf16x8 *w = ws + fwd_frag(L) * 64 + fresh(lane);                                \
+        product<NK, NR, 4>([&](int f) { return w[f * 64]; }, b, acc);                         \
+    }
+        FWD(0, 3, 4)
+        activate<4>(acc, b);
+        FWD(1, 2, 4)
+        activate<4>(acc, b);
+        FWD(2, 2, 4)
+        activate<4>(acc, b);
+        FWD(3, 2, 4)
+        activate<4>(acc, b);
+        FWD(4, 2, 4)
+        activate<4>(acc, b);
+        FWD(5, 2, 1)
+#undef FWD
+        if (g == 0) {
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const uint32_t row = s0 + rt * 16 + 4 * g + i;
-                if (r16 < 3 && row < n) out[(size_t)row * 3 + r16] = acc[rt][0][i];
+            for (int ct = 0; ct < 4; ++ct) {
+                const uint32_t s = s0 + ct * 16 + r;
+                if (s < n)
+                    for (int i = 0; i < 3; ++i) out[(size_t)s * 3 + i] = acc[0][ct][i];
             }
-        __syncthreads();
-    }
-}
-
-// One part of a query's features, for the four lane groups of the training workgroup:
-// part c < 3 = the 24 sin/cos features of position component c; part 3 = direction, normal,
-// albedo, roughness, the constant 1 and the zero padding.  Same values as encode_row.
-__device__ __forceinline__ void encode_part(const float *q, bf16 *row, int part)
-{
-    if (part < 3) {
-        float f = 3.14159265358979323846f;
-#pragma unroll
-        for (int k = 0; k < 12; ++k) {
-            const float arg = q[part] * f;
-            float s, co;
-            sincosf(arg, &s, &co);
-            row[part * 24 + 2 * k]     = to_bf16(s);
-            row[part * 24 + 2 * k + 1] = to_bf16(co);
-            f *= 2.0f;
         }
-    } else {
-#pragma unroll
-        for (int k = 0; k < 10; ++k) row[72 + k] = to_bf16(q[3 + k]);
-        row[82] = to_bf16(1.0f);
-#pragma unroll
-        for (int k = 83; k < kNrcIn; ++k) row[k] = to_bf16(0.0f);
     }
 }
 
-// Copies the tile's 64 activation rows (columns [0, C)) from LDS to the global scratch.
-template <int C>
-__device__ __forceinline__ void save_acts(const bf16 *X, bf16 *A, int off)
-{
-    for (int c = threadIdx.x; c < 64 * (C / 8); c += 256) {
-        const int row = c / (C / 8), col = (c % (C / 8)) * 8;
-        *reinterpret_cast<bf16x8 *>(A + row * kNrcActs + off + col) = lds8(X + row * kXStride + col);
-    }
-}
+// Training.  A block of four waves owns tiles of 64 samples, 16 per wave.  Forward and the
+// backward data products stay in each wave's registers (no barrier); for dW the waves exchange
+// the layer's activations and output gradients, a feature per lane, through LDS, and wave w
+// forms the column tile w of the layer's dW over all 64 samples.  The dW tiles accumulate in
+// registers over all the block's tiles (92 registers a lane), so a batch writes one gradient
+// partial per block, at most kNrcMaxParts of them, instead of one per 64 samples.  Two exchange
+// buffers alternate, so a layer costs one barrier.  40 KB of LDS leave room beside three
+// traversal blocks on a CU.  Bound by the chain of 12 products of one tile (a few microseconds)
+// for batches below 16,384; for larger ones by the weight fragments from L2 (82 KB per wave and
+// tile).  16,384 samples: 28 us with the activations saved to HBM and gathered from there by 2
+// bytes, 22 us like this; with the partials' sum (60 -> 6 us) and one pinned copy of gradient and
+// loss a gradient call went from 131 to 46 us.
+constexpr int kXt = 6 * 4 * 64, kGt = 4 * 4 * 64;   // exchanged fragments of 4 elements
 
-// Training: one workgroup (4 waves) = one tile of 64 samples.  The output columns of every
-// layer product are split over the waves (forward and dX: column tile = wave; dW: row tile
-// kt = wave, wave + 4, ...), with the tile's activations and output gradients shared in LDS,
-// so a step's serial chain of layer products is a quarter as long as with one wave per
-// tile.  Writes the tile's gradient partial (every parameter by exactly one wave, no
-// atomics) and its loss partial.
-__global__ __launch_bounds__(256) void k_nrc_train(const float *__restrict__ q, const float *__restrict__ target,
-                                                   uint32_t n, float inv_count, const bf16 *__restrict__ W,
-                                                   const bf16 *__restrict__ WT, bf16 *__restrict__ act,
-                                                   float *__restrict__ partial, float *__restrict__ partial_loss)
+__global__ __launch_bounds__(256, 1) void k_nrc_train(const float *__restrict__ q, const float *__restrict__ target,
+                                                      uint32_t n, float inv_count, const bf16 *__restrict__ WF,
+                                                      const bf16 *__restrict__ WB, float *__restrict__ partial,
+                                                      float *__restrict__ partial_loss)
 {
-    __shared__ bf16 X[64 * kXStride];
-    __shared__ bf16 Gs[64 * kGStride];    // G sample-major [s][n]
-    __shared__ bf16 Gt[64 * kGStride];    // G feature-major [n][s]
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r16 = lane & 15, g = lane >> 4;
-    const uint32_t tile = blockIdx.x;
-    const uint32_t s0 = tile * 64;
-    bf16 *A = act + (size_t)tile * 64 * kNrcActs;    // [64][kNrcActs] sample-major
-    {
-        const uint32_t s = s0 + lane;
-        float qq[kNrcQuery];
+    __shared__ bf16x4 xs[2][kXt], gs[2][kGt];
+    __shared__ float  wloss[4];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
+    const uint32_t ntiles = (n + 63u) / 64u;
+    // column r of ident[h] selects reduction element (r / 4, 4 h + r % 4)
+    bf16x8 ident[2];
 #pragma unroll
-        for (int k = 0; k < kNrcQuery; ++k) qq[k] = s < n ? q[(size_t)s * kNrcQuery + k] : 0.0f;
-        encode_part(qq, X + lane * kXStride, wv);
-    }
-    __syncthreads();
-    save_acts<kNrcIn>(X, A, 0);
-    // ---- forward: wave w computes output columns [16w, 16w + 16) of each hidden layer ----
-#define FWD_HIDDEN(L)                                                                             \
-    {                                                                                             \
-        constexpr int K = layer_k(L);                                                             \
-        f32x4 acc[4];                                                                             \
-        for (int rt = 0; rt < 4; ++rt) acc[rt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};                   \
-        const bf16 *w = WT + nrc_w_off(L);                                                        \
-        for (int kk = 0; kk < K / 32; ++kk) {                                                     \
-            const bf16x8 b = glb8(w + (wv * 16 + r16) * K + kk * 32 + 8 * g);                     \
-            for (int rt = 0; rt < 4; ++rt)                                                        \
-                acc[rt] = mma(lds8(X + (rt * 16 + r16) * kXStride + kk * 32 + 8 * g), b, acc[rt]); \
-        }                                                                                         \
-        __syncthreads();                                                                          \
-        for (int rt = 0; rt < 4; ++rt)                                                            \
-            for (int i = 0; i < 4; ++i)                                                           \
-                X[(rt * 16 + 4 * g + i) * kXStride + wv * 16 + r16] = to_bf16(fmaxf(acc[rt][i], 0.0f)); \
-        __syncthreads();                                                                          \
-        save_acts<kNrcHid>(X, A, act_off(L + 1));                                                 \
-    }
-    FWD_HIDDEN(0)
-    FWD_HIDDEN(1)
-    FWD_HIDDEN(2)
-    FWD_HIDDEN(3)
-    FWD_HIDDEN(4)
-#undef FWD_HIDDEN
-    // ---- output layer (waves 0, 1: column tiles 0, 1), loss and dL/dy ----
-    if (wv < kNrcOut / 16) {
-        constexpr int K = layer_k(5);
-        f32x4 acc[4];
-        for (int rt = 0; rt < 4; ++rt) acc[rt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-        const bf16 *w = WT + nrc_w_off(5);
-        for (int kk = 0; kk < K / 32; ++kk) {
-            const bf16x8 b = glb8(w + (wv * 16 + r16) * K + kk * 32 + 8 * g);
-            for (int rt = 0; rt < 4; ++rt) acc[rt] = mma(lds8(X + (rt * 16 + r16) * kXStride + kk * 32 + 8 * g), b, acc[rt]);
-        }
-        float lsum = 0.0f;
+    for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int rt = 0; rt < 4; ++rt)
+        for (int j = 0; j < 8; ++j) ident[h][j] = to_bf16(g == (r >> 2) && j == 4 * h + (r & 3) ? 1.0f : 0.0f);
+    const f32x4 zero = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    auto turn = [&](bf16x8 f, int h) {   // feature tile h of a chunk, samples in the registers
+        const f32x4 d = mma(f, ident[h], zero);
+        return bf16x4{to_bf16(d[0]), to_bf16(d[1]), to_bf16(d[2]), to_bf16(d[3])};
+    };
+    f32x4 dw0[6], dwh[4][4], dw5 = zero;   // dW tiles of column tile wv (layer 5: row tile wv)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = rt * 16 + 4 * g + i, col = wv * 16 + r16;
-                const uint32_t srow = s0 + row;
-                float gr = 0.0f;
-                if (col < 3 && srow < n) {
-                    const float y = acc[rt][i];
-                    const float t = target[(size_t)srow * 3 + col];
-                    const float e = y - t;
-                    const float den = y * y + kNrcEpsRel;
-                    lsum += e * e / den * inv_count;
-                    gr = 2.0f * e / den * inv_count;
-                }
-                const bf16 gb = to_bf16(gr);
-                Gs[row * kGStride + col] = gb;
-                Gt[col * kGStride + row] = gb;
+    for (int k = 0; k < 6; ++k) dw0[k] = zero;
+#pragma unroll
+    for (int l = 0; l < 4; ++l)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) dwh[l][k] = zero;
+    float lsum = 0.0f;
+    for (uint32_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const uint32_t s = tile * 64u + wv * 16 + r;
+        bf16x8 b[3][1];
+        bf16x4 xt[6];            // input features, turned
+        bf16x4 ht[5][4];         // hidden activations, turned
+        uint32_t live[5];        // bit 8 c + j: hidden activation (c, j) of this lane is positive
+        {
+            bf16x8 f[3];
+            encode(q + (size_t)min(s, n - 1u) * kNrcQuery, g, f);
+#pragma unroll
+            for (int c = 0; c < 3; ++c) {
+                b[c][0] = f[c];
+                xt[2 * c]     = turn(f[c], 0);
+                xt[2 * c + 1] = turn(f[c], 1);
             }
-        for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
-        if (wv == 0 && lane == 0) partial_loss[tile] = lsum;
+        }
+        f32x4 acc[4][1];
+#define FWD(L, NK, NR)                                                                  \
+    {                                                                                   \
+        const bf16 *w = WF + fwd_frag(L) * kFrag + fresh(lane * 8);                     \
+        product<NK, NR, 1>([&](int f) { return ld8(w + f * kFrag); }, b, acc);          \
     }
+#define HIDDEN(L, NK)                                                                   \
+    FWD(L, NK, 4)                                                                       \
+    activate<1>(acc, b);                                                                \
+    live[L] = 0u;                                                                       \
+    _Pragma("unroll") for (int c = 0; c < 2; ++c)                                       \
+    {                                                                                   \
+        ht[L][2 * c]     = turn(b[c][0], 0);                                            \
+        ht[L][2 * c + 1] = turn(b[c][0], 1);                                            \
+        _Pragma("unroll") for (int j = 0; j < 8; ++j)                                   \
+            live[L] |= (float)b[c][0][j] > 0.0f ? 1u << (8 * c + j) : 0u;               \
+    }
+        HIDDEN(0, 3)
+        HIDDEN(1, 2)
+        HIDDEN(2, 2)
+        HIDDEN(3, 2)
+        HIDDEN(4, 2)
+#undef HIDDEN
+        FWD(5, 2, 1)
+#undef FWD
+        // loss and dL/dy: the lanes of group 0 hold the three outputs of their sample
+        bf16x8 gy;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) gy[j] = to_bf16(0.0f);
+        if (g == 0 && s < n) {
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const float y = acc[0][0][i], e = y - target[(size_t)s * 3 + i], den = y * y + kNrcEpsRel;
+                lsum += e * e / den * inv_count;
+                gy[i] = to_bf16(2.0f * e / den * inv_count);
+            }
+        }
+        // Layer L: share its input X (NX feature tiles) and output gradient G (NG tiles), then
+        // accumulate dW.  The barrier also keeps this layer's stores behind the reads of the
+        // layer before last, which used the same buffer.
+        auto share = [&](const auto &x, const auto &gt, int buf) {
+#pragma unroll
+            for (int k = 0; k < (int)(sizeof x / sizeof x[0]); ++k) xs[buf][(k * 4 + wv) * 64 + lane] = x[k];
+#pragma unroll
+            for (int k = 0; k < (int)(sizeof gt / sizeof gt[0]); ++k) gs[buf][(k * 4 + wv) * 64 + lane] = gt[k];
+            __syncthreads();
+        };
+        b[0][0] = gy;
+        {
+            const bf16x4 gt[1] = {turn(gy, 0)};
+            share(ht[4], gt, 0);
+#pragma unroll
+            for (int p = 0; p < 4; ++p) dw5 = mma16(xs[0][(wv * 4 + p) * 64 + lane], gs[0][p * 64 + lane], dw5);
+        }
+        // gradient of layer L's input from b, masked by relu' of that input (hidden layer L - 1)
+#define DX(L, NC)                                                                                              \
+    {                                                                                                          \
+        const bf16 *w = WB + bwd_frag(L) * kFrag + fresh(lane * 8);                                            \
+        product<NC, 4, 1>([&](int f) { return ld8(w + f * kFrag); }, b, acc);                                  \
+    }                                                                                                          \
+    _Pragma("unroll") for (int t = 0; t < 4; ++t) _Pragma("unroll") for (int i = 0; i < 4; ++i)                \
+        acc[t][0][i] = live[L - 1] >> (8 * (t >> 1) + 4 * (t & 1) + i) & 1u ? acc[t][0][i] : 0.0f;             \
+    _Pragma("unroll") for (int c = 0; c < 2; ++c) b[c][0] = pack<false>(acc[2 * c][0], acc[2 * c + 1][0]);
+#define DW(L, X, NX, D, BUF)                                                                                   \
+    {                                                                                                          \
+        const bf16x4 gt[4] = {turn(b[0][0], 0), turn(b[0][0], 1), turn(b[1][0], 0), turn(b[1][0], 1)};         \
+        share(X, gt, BUF);                                                                                     \
+        _Pragma("unroll") for (int p = 0; p < 4; ++p)                                                          \
+        {                                                                                                      \
+            const bf16x4 gg = gs[BUF][(wv * 4 + p) * 64 + lane];                                               \
+            _Pragma("unroll") for (int k = 0; k < NX; ++k)                                                     \
+                D[k] = mma16(xs[BUF][(k * 4 + p) * 64 + lane], gg, D[k]);                                      \
+        }                                                                                                      \
+    }
+        DX(5, 1)
+        DW(4, ht[3], 4, dwh[3], 1)
+        DX(4, 2)
+        DW(3, ht[2], 4, dwh[2], 0)
+        DX(3, 2)
+        DW(2, ht[1], 4, dwh[1], 1)
+        DX(2, 2)
+        DW(1, ht[0], 4, dwh[0], 0)
+        DX(1, 2)
+        DW(0, xt, 6, dw0, 1)
+#undef DX
+#undef DW
+        // buffer 1 was read last and buffer 0 before a barrier: the next tile may start with 0
+    }
+    // the block's partial, in parameter order (columns 16 .. 31 of the output layer are zero)
+    float *P = partial + (size_t)blockIdx.x * kNrcParams;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) P[kmap0(k >> 1, g, 4 * (k & 1) + i) * kNrcHid + wv * 16 + r] = dw0[k][i];
+#pragma unroll
+        for (int l = 0; l < 4; ++l)
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+                P[nrc_w_off(l + 1) + (k * 16 + 4 * g + i) * kNrcHid + wv * 16 + r] = dwh[l][k][i];
+        float *p5 = P + nrc_w_off(5) + (wv * 16 + 4 * g + i) * kNrcOut + r;
+        p5[0]  = dw5[i];
+        p5[16] = 0.0f;
+    }
+    for (int o = 32; o > 0; o >>= 1) lsum += __shfl_xor(lsum, o);
+    if (lane == 0) wloss[wv] = lsum;
     __syncthreads();
-    float *P = partial + (size_t)tile * kNrcParams;
-    // ---- backward ----
-#define BWD(L)                                                                                              \
-    {                                                                                                       \
-        constexpr int K = layer_k(L), N = layer_n(L);                                                       \
-        /* dW = X_L^T G: row tiles kt = wave, wave + 4, ...; all N / 16 column tiles */                     \
-        for (int kt = wv; kt < K / 16; kt += 4) {                                                           \
-            bf16x8 a[2];                                                                                    \
-            for (int ss = 0; ss < 2; ++ss) {                                                                \
-                bf16 tmp[8];                                                                                \
-                for (int i = 0; i < 8; ++i) tmp[i] = A[(ss * 32 + 8 * g + i) * kNrcActs + act_off(L) + kt * 16 + r16]; \
-                a[ss] = bf16x8{tmp[0], tmp[1], tmp[2], tmp[3], tmp[4], tmp[5], tmp[6], tmp[7]};            \
-            }                                                                                               \
-            for (int ct = 0; ct < N / 16; ++ct) {                                                           \
-                f32x4 d = f32x4{0.0f, 0.0f, 0.0f, 0.0f};                                                    \
-                for (int ss = 0; ss < 2; ++ss) d = mma(a[ss], lds8(Gt + (ct * 16 + r16) * kGStride + ss * 32 + 8 * g), d); \
-                for (int i = 0; i < 4; ++i) P[nrc_w_off(L) + (kt * 16 + 4 * g + i) * N + ct * 16 + r16] = d[i]; \
-            }                                                                                               \
-        }                                                                                                   \
-        if (L > 0) {                                                                                        \
-            /* dX = (G W_L^T) * relu'(X_L): wave w computes columns [16w, 16w + 16); reduction over n */    \
-            f32x4 dx[4];                                                                                    \
-            for (int rt = 0; rt < 4; ++rt) dx[rt] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};                         \
-            for (int nn = 0; nn < N / 32; ++nn) {                                                           \
-                const bf16x8 b = glb8(W + nrc_w_off(L) + (wv * 16 + r16) * N + nn * 32 + 8 * g);            \
-                for (int rt = 0; rt < 4; ++rt)                                                              \
-                    dx[rt] = mma(lds8(Gs + (rt * 16 + r16) * kGStride + nn * 32 + 8 * g), b, dx[rt]);       \
-            }                                                                                               \
-            __syncthreads();                                                                                \
-            for (int rt = 0; rt < 4; ++rt)                                                                  \
-                for (int i = 0; i < 4; ++i) {                                                               \
-                    const int row = rt * 16 + 4 * g + i, col = wv * 16 + r16;                               \
-                    const float xv = from_bf16(A[row * kNrcActs + act_off(L) + col]);                        \
-                    const bf16 gb = to_bf16(xv > 0.0f ? dx[rt][i] : 0.0f);                                  \
-                    Gs[row * kGStride + col] = gb;                                                          \
-                    Gt[col * kGStride + row] = gb;                                                          \
-                }                                                                                           \
-            __syncthreads();                                                                                \
-        }                                                                                                   \
-    }
-    BWD(5)
-    BWD(4)
-    BWD(3)
-    BWD(2)
-    BWD(1)
-    BWD(0)
-#undef BWD
+    if (threadIdx.x == 0) partial_loss[blockIdx.x] = wloss[0] + wloss[1] + wloss[2] + wloss[3];
 }
 
-// Adam on the FP32 master weights from the summed per-tile partials; refreshes the bf16
-// copies.  Padded outputs (columns >= 3 of the last layer) and padded input features
-// (rows >= 83 of the first layer) stay zero.
-__global__ void k_nrc_adam(const float *__restrict__ partial, uint32_t nrows, float *params, float *m, float *v,
-                           bf16 *W, bf16 *WT, float lr, float b1, float b2, float eps, float bc1, float bc2, int update)
+// Sum of the partials of 256 parameters per block: 16 waves take the rows in turn, a lane four
+// consecutive parameters (16 bytes), and the waves' sums meet in LDS.  Thread t < 256 returns
+// the sum of parameter 256 blockIdx + t.  With one thread per parameter walking all the rows,
+// 256 rows (25 MB) took 60 us.
+constexpr int kSumWaves = 16;
+
+__device__ __forceinline__ float sum_rows(const float *__restrict__ partial, uint32_t nrows)
 {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (uint32_t)kNrcParams) return;
+    __shared__ float4 part[kSumWaves][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    const float *src = partial + blockIdx.x * 256 + lane * 4;
+#pragma unroll 4
+    for (uint32_t t = wv; t < nrows; t += kSumWaves) {
+        const float4 v = *reinterpret_cast<const float4 *>(src + (size_t)t * kNrcParams);
+        a.x += v.x;
+        a.y += v.y;
+        a.z += v.z;
+        a.w += v.w;
+    }
+    part[wv][lane] = a;
+    __syncthreads();
+    float s = 0.0f;
+    if (threadIdx.x < 256)
+        for (int w = 0; w < kSumWaves; ++w) s += reinterpret_cast<const float *>(part[w])[threadIdx.x];
+    return s;
+}
+
+// Adam on the FP32 master weights from the summed partials; refreshes the bf16 copies.
+// Padded outputs (columns >= 3 of the last layer) and padded input features (rows >= 83 of
+// the first layer) stay zero.
+__global__ __launch_bounds__(64 * kSumWaves) void k_nrc_adam(const float *__restrict__ partial, uint32_t nrows,
+                                                             float *params, float *m, float *v, bf16 *WF, bf16 *WB,
+                                                             float lr, float b1, float b2, float eps, float bc1,
+                                                             float bc2, int update)
+{
+    const float gsum = update ? sum_rows(partial, nrows) : 0.0f;
+    if (threadIdx.x >= 256) return;
+    const uint32_t p = blockIdx.x * 256 + threadIdx.x;
     int l = 0;
     while (l + 1 < kNrcLayers && p >= (uint32_t)nrc_w_off(l + 1)) ++l;
-    const uint32_t K = layer_k(l), N = layer_n(l);
+    const uint32_t N = layer_n(l);
     const uint32_t local = p - nrc_w_off(l), k = local / N, c = local % N;
     const bool frozen = (l == kNrcLayers - 1 && c >= 3) || (l == 0 && k >= 83);
     float w = params[p];
     if (update && !frozen) {
-        float gsum = 0.0f;
-        for (uint32_t t = 0; t < nrows; ++t) gsum += partial[(size_t)t * kNrcParams + p];
         const float mm = b1 * m[p] + (1.0f - b1) * gsum;
         const float vv = b2 * v[p] + (1.0f - b2) * gsum * gsum;
         m[p] = mm;
@@ -357,60 +489,72 @@ __global__ void k_nrc_adam(const float *__restrict__ partial, uint32_t nrows, fl
         w = 0.0f;
         params[p] = 0.0f;
     }
-    W[p] = to_bf16(w);
-    WT[nrc_w_off(l) + c * K + k] = to_bf16(w);
+    WF[fwd_pos(l, (int)k, (int)c)] = to_bf16(w);
+    if (l > 0) WB[bwd_pos(l, (int)k, (int)c)] = to_bf16(w);
 }
 
-__global__ void k_nrc_sum_partials(const float *__restrict__ partial, uint32_t nrows, float *out)
+// out[0 .. kNrcParams) = the summed gradient, out[kNrcParams] = the loss (summed in FP64 by a
+// wave that has no parameter to finish), so the caller fetches both with one copy.
+__global__ __launch_bounds__(64 * kSumWaves) void k_nrc_sum_partials(const float *__restrict__ partial,
+                                                                     const float *__restrict__ partial_loss,
+                                                                     uint32_t nrows, float *out)
 {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= (uint32_t)kNrcParams) return;
-    float s = 0.0f;
-    for (uint32_t t = 0; t < nrows; ++t) s += partial[(size_t)t * kNrcParams + p];
-    out[p] = s;
+    const float s = sum_rows(partial, nrows);
+    if (threadIdx.x < 256) out[blockIdx.x * 256 + threadIdx.x] = s;
+    if (blockIdx.x == 0 && threadIdx.x >= 256 && threadIdx.x < 320) {
+        double d = 0.0;
+        for (uint32_t t = threadIdx.x - 256; t < nrows; t += 64) d += partial_loss[t];
+        for (int o = 32; o > 0; o >>= 1) d += __shfl_xor(d, o);
+        if (threadIdx.x == 256) out[kNrcParams] = (float)d;
+    }
+}
+
+static_assert(kNrcParams % 256 == 0, "sum_rows takes whole groups of 256 parameters");
+
+hipError_t launch_infer(const float *q, float *out, uint32_t n, const uint32_t *n_dev, const __bf16 *WF, hipStream_t s)
+{
+    if (n == 0) return hipSuccess;
+    const uint32_t tiles = (uint32_t)(((uint64_t)n + 64 * kInferWaves - 1) / (64 * kInferWaves));
+    // three blocks per CU are resident; each loads the weights once
+    k_nrc_infer<<<std::min<uint32_t>(tiles, kInferBlocks), 64 * kInferWaves, 0, s>>>(q, out, n, n_dev, WF);
+    return hipGetLastError();
 }
 
 }  // namespace
 
-hipError_t nrc_launch_infer(const float *q, float *out, uint32_t n, const __bf16 *WT, hipStream_t s)
+hipError_t nrc_launch_infer(const float *q, float *out, uint32_t n, const __bf16 *WF, hipStream_t s)
 {
-    if (n == 0) return hipSuccess;
-    const uint32_t tiles = (n + 255) / 256;
-    k_nrc_infer<<<std::min<uint32_t>(tiles, 2048u), 256, 0, s>>>(q, out, n, nullptr, WT);
-    return hipGetLastError();
+    return launch_infer(q, out, n, nullptr, WF, s);
 }
 
-hipError_t nrc_launch_infer_dev(const float *q, float *out, const uint32_t *n_dev, uint32_t n_max, const __bf16 *WT,
+hipError_t nrc_launch_infer_dev(const float *q, float *out, const uint32_t *n_dev, uint32_t n_max, const __bf16 *WF,
                                 hipStream_t s)
 {
-    if (n_max == 0) return hipSuccess;
-    const uint32_t tiles = (n_max + 255) / 256;
-    k_nrc_infer<<<std::min<uint32_t>(tiles, 2048u), 256, 0, s>>>(q, out, n_max, n_dev, WT);
-    return hipGetLastError();
+    return launch_infer(q, out, n_max, n_dev, WF, s);
 }
 
-hipError_t nrc_launch_train(const float *q, const float *target, uint32_t n, const __bf16 *W, const __bf16 *WT,
-                            __bf16 *act, float *partial, float *partial_loss, hipStream_t s)
+hipError_t nrc_launch_train(const float *q, const float *target, uint32_t n, const __bf16 *WF, const __bf16 *WB,
+                            float *partial, float *partial_loss, hipStream_t s)
 {
     if (n == 0) return hipSuccess;
-    const uint32_t tiles = (n + 63) / 64;
-    k_nrc_train<<<tiles, 256, 0, s>>>(q, target, n, 1.0f / (3.0f * (float)n), W, WT, act, partial, partial_loss);
+    k_nrc_train<<<nrc_partial_rows(n), 256, 0, s>>>(q, target, n, 1.0f / (3.0f * (float)n), WF, WB, partial, partial_loss);
     return hipGetLastError();
 }
 
-hipError_t nrc_launch_adam(const float *partial, uint32_t nrows, float *params, float *m, float *v, __bf16 *W,
-                           __bf16 *WT, float lr, float b1, float b2, float eps, uint64_t step, int update,
+hipError_t nrc_launch_adam(const float *partial, uint32_t nrows, float *params, float *m, float *v, __bf16 *WF,
+                           __bf16 *WB, float lr, float b1, float b2, float eps, uint64_t step, int update,
                            hipStream_t s)
 {
     const float bc1 = 1.0f - powf(b1, (float)step), bc2 = 1.0f - powf(b2, (float)step);
-    k_nrc_adam<<<(kNrcParams + 255) / 256, 256, 0, s>>>(partial, nrows, params, m, v, W, WT, lr, b1, b2, eps,
-                                                         update ? bc1 : 1.0f, update ? bc2 : 1.0f, update);
+    k_nrc_adam<<<kNrcParams / 256, 64 * kSumWaves, 0, s>>>(partial, nrows, params, m, v, WF, WB, lr, b1, b2, eps,
+                                                           update ? bc1 : 1.0f, update ? bc2 : 1.0f, update);
     return hipGetLastError();
 }
 
-hipError_t nrc_launch_sum_partials(const float *partial, uint32_t nrows, float *out, hipStream_t s)
+hipError_t nrc_launch_sum_partials(const float *partial, const float *partial_loss, uint32_t nrows, float *out,
+                                   hipStream_t s)
 {
-    k_nrc_sum_partials<<<(kNrcParams + 255) / 256, 256, 0, s>>>(partial, nrows, out);
+    k_nrc_sum_partials<<<kNrcParams / 256, 64 * kSumWaves, 0, s>>>(partial, partial_loss, nrows, out);
     return hipGetLastError();
 }
 
