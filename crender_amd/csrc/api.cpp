@@ -92,6 +92,9 @@ constexpr uint32_t kWavefrontPaths      = 1u << 24;
 constexpr uint32_t kWavefrontPathsCache = 1u << 23;
 constexpr uint32_t kMaxWavefrontPasses = 8;
 
+// most workspace a context keeps between calls: 16 1080p images of 33 MB fit in half of it
+constexpr size_t kWorkspaceMax = 1ull << 30;
+
 struct crt_context {
     int         device = 0;
     crt_options opt{};
@@ -117,6 +120,8 @@ struct crt_context {
     float      *st_ng[3] = {};
     uint8_t    *st_occ = nullptr;
     uint32_t   *st_cnt = nullptr;   // kQcWords words: count, error flag, work counters
+    uint8_t    *ws = nullptr;       // Workspace
+    size_t      ws_bytes = 0;
     uint8_t    *noalloc = nullptr;  // this device's crt_intersect_noalloc scratch (noalloc.hip)
     std::mutex  mu;                 // serialises queries on the context stream
     std::atomic<int> live{0};       // scenes, renderers and caches created on the context
@@ -243,6 +248,36 @@ TraceConfig trace_cfg(const crt_context *ctx)
 {
     return TraceConfig{ctx->grid, ctx->stack, ctx->refill, ctx->park_min, ctx->leaf_rounds, ctx->spill_depth};
 }
+
+// Device memory for the length of one call, kept by the context between calls (an allocation
+// and its release cost a call 50 us and more) and given back with it.  The caller holds the
+// context's mutex and leaves no work running on the memory.  Requests above kWorkspaceMax are
+// allocated and freed by the call.
+struct Workspace {
+    uint8_t *base = nullptr;
+    bool     own  = false;
+    ~Workspace()
+    {
+        if (own) dfree(base);
+    }
+    int open(crt_context *ctx, size_t bytes)
+    {
+        if (bytes > kWorkspaceMax) {
+            HIP_CHECK(dalloc(&base, bytes));
+            own = true;
+            return CRT_OK;
+        }
+        if (bytes > ctx->ws_bytes) {
+            dfree(ctx->ws);
+            ctx->ws       = nullptr;
+            ctx->ws_bytes = 0;
+            HIP_CHECK(dalloc(&ctx->ws, bytes));
+            ctx->ws_bytes = bytes;
+        }
+        base = ctx->ws;
+        return CRT_OK;
+    }
+};
 
 int ensure_spill(crt_context *ctx, int set = 0)
 {
@@ -1334,6 +1369,7 @@ int crt_context_destroy(crt_context *ctx)
     for (float *p : ctx->st_ng) dfree(p);
     dfree(ctx->st_occ);
     dfree(ctx->st_cnt);
+    dfree(ctx->ws);
     (void)hipStreamDestroy(ctx->stream);
     (void)hipStreamDestroy(ctx->stream2);
     delete ctx;
@@ -3162,25 +3198,28 @@ int crt_autotune(crt_context *ctx, const crt_job *jobs, uint32_t njobs, uint32_t
 
 namespace {
 
-// Device copies of caller images (host memory) or the caller's device pointers; scratch.
+// Images of one call carved out of the context's workspace (the context's mutex is held and
+// the call ends with its stream idle).
 struct ImageScratch {
-    std::vector<void *> allocs;
-    ~ImageScratch()
+    Workspace ws;
+    size_t    n4;      // pixels per image
+    uint32_t  used = 0;
+    int open(crt_context *ctx, size_t pixels, uint32_t images)
     {
-        for (void *p : allocs) dfree(p);
+        n4 = pixels;
+        return ws.open(ctx, sizeof(float4) * pixels * images);
     }
+    float4 *image() { return reinterpret_cast<float4 *>(ws.base) + n4 * used++; }
 };
 
-int image_in(ImageScratch &sc, const float *p, size_t n4, int memory, hipStream_t s, const float4 **out)
+int image_in(ImageScratch &sc, const float *p, int memory, hipStream_t s, const float4 **out)
 {
     if (memory == CRT_MEM_DEVICE) {
         *out = reinterpret_cast<const float4 *>(p);
         return CRT_OK;
     }
-    float4 *d = nullptr;
-    int     st = lalloc(sc.allocs, &d, n4);
-    if (st) return st;
-    HIP_CHECK(hipMemcpyAsync(d, p, sizeof(float4) * n4, hipMemcpyHostToDevice, s));
+    float4 *d = sc.image();
+    HIP_CHECK(hipMemcpyAsync(d, p, sizeof(float4) * sc.n4, hipMemcpyHostToDevice, s));
     *out = d;
     return CRT_OK;
 }
@@ -3219,15 +3258,14 @@ int crt_post_process(crt_context *ctx, const crt_post_options *opt, const float 
         HIP_CHECK(hipStreamSynchronize(s));
         return CRT_OK;
     }
+    const bool   dev = memory == CRT_MEM_DEVICE;
     ImageScratch sc;
+    int st = sc.open(ctx, n4, (dev ? 0u : 2u) + (o.bloom ? 2u : 0u));
     const float4 *in = nullptr;
-    int st = image_in(sc, rgba_in, n4, memory, s, &in);
+    if (!st) st = image_in(sc, rgba_in, memory, s, &in);
     if (st) return st;
-    float4 *out = nullptr, *t0 = nullptr, *t1 = nullptr;
-    if (memory == CRT_MEM_DEVICE) out = reinterpret_cast<float4 *>(rgba_out);
-    else if ((st = lalloc(sc.allocs, &out, n4))) return st;
-    if ((st = lalloc(sc.allocs, &t0, n4))) return st;
-    if (o.bloom && (st = lalloc(sc.allocs, &t1, n4))) return st;
+    float4 *out = dev ? reinterpret_cast<float4 *>(rgba_out) : sc.image();
+    float4 *t0 = o.bloom ? sc.image() : nullptr, *t1 = o.bloom ? sc.image() : nullptr;
     PostDev p{};
     p.w = width;
     p.h = height;
@@ -3241,7 +3279,7 @@ int crt_post_process(crt_context *ctx, const crt_post_options *opt, const float 
     p.tonemap_type = o.tonemapping_type;
     p.exposure = o.exposure;
     p.gamma = o.gamma;
-    HIP_CHECK(launch_post(p, in, out, t0, t1 ? t1 : t0, s));
+    HIP_CHECK(launch_post(p, in, out, t0, t1, s));
     if (memory != CRT_MEM_DEVICE) HIP_CHECK(hipMemcpyAsync(rgba_out, out, sizeof(float4) * n4, hipMemcpyDeviceToHost, s));
     HIP_CHECK(hipStreamSynchronize(s));
     return CRT_OK;
@@ -3272,17 +3310,16 @@ int crt_denoise(crt_context *ctx, const crt_denoise_options *opt, const float *c
     std::lock_guard<std::mutex> lock(ctx->mu);
     HIP_CHECK(hipSetDevice(ctx->device));
     hipStream_t s = ctx->stream;
+    const bool   dev = memory == CRT_MEM_DEVICE;
     ImageScratch sc;
+    int st = sc.open(ctx, n4, (dev ? 0u : 4u) + 2u);
     const float4 *c = nullptr, *n = nullptr, *a = nullptr;
-    int st = image_in(sc, colour, n4, memory, s, &c);
-    if (!st) st = image_in(sc, normal, n4, memory, s, &n);
-    if (!st) st = image_in(sc, albedo, n4, memory, s, &a);
+    if (!st) st = image_in(sc, colour, memory, s, &c);
+    if (!st) st = image_in(sc, normal, memory, s, &n);
+    if (!st) st = image_in(sc, albedo, memory, s, &a);
     if (st) return st;
-    float4 *out = nullptr, *t0 = nullptr, *t1 = nullptr;
-    if (memory == CRT_MEM_DEVICE) out = reinterpret_cast<float4 *>(rgba_out);
-    else if ((st = lalloc(sc.allocs, &out, n4))) return st;
-    if ((st = lalloc(sc.allocs, &t0, n4))) return st;
-    if ((st = lalloc(sc.allocs, &t1, n4))) return st;
+    float4 *out = dev ? reinterpret_cast<float4 *>(rgba_out) : sc.image();
+    float4 *t0 = sc.image(), *t1 = sc.image();
     HIP_CHECK(launch_atrous(c, n, a, out, t0, t1, width, height, (int)o.levels, o.sigma_colour, o.sigma_normal,
                             o.sigma_albedo, s));
     if (memory != CRT_MEM_DEVICE) HIP_CHECK(hipMemcpyAsync(rgba_out, out, sizeof(float4) * n4, hipMemcpyDeviceToHost, s));
