@@ -44,7 +44,9 @@ def _run(cmd: list[str]) -> None:
 # FP contraction so that every product and sum rounds as written, like the CPU restatement
 # it is checked against (the traversal keeps its explicit fmaf node test).
 PER_FILE = {
-    "integrator.hip": ["-ffp-contract=off"],
+    # Constants stay where they are used: hoisted out of the shading kernel's loop over its
+    # queue they take 197 registers instead of 93.
+    "integrator.hip": ["-ffp-contract=off", "-mllvm", "-disable-machine-licm"],
 }
 
 

@@ -390,7 +390,7 @@ int ralloc(crt_renderer *r, T **p, size_t count)
 
 int alloc_rays_list(std::vector<void *> &list, RaySoA &q, size_t n)
 {
-    float **f[8] = {&q.ox, &q.oy, &q.oz, &q.dx, &q.dy, &q.dz, &q.tn, &q.tf};
+    float **f[6] = {&q.ox, &q.oy, &q.oz, &q.dx, &q.dy, &q.dz};   // no limits: see RaySoA
     for (float **p : f) {
         const int st = lalloc(list, p, n);
         if (st) return st;
@@ -423,7 +423,6 @@ int alloc_path_core(std::vector<void *> &L, PathBuffers &b, size_t P)
     LA(&b.shits.tri, P);
     LA(&b.spath, 2 * P);
     LA(&b.scontrib, 2 * P);
-    LA(&b.occ, P);
     LA(&b.thr, P);
     LA(&b.rad, P);
     LA(&b.cnt, (size_t)kCntWords);
@@ -476,7 +475,6 @@ int alloc_path_set(crt_renderer *r, PathBuffers &b, bool image)
     RA(&b.shits.tri, P);
     RA(&b.spath, 2 * P);
     RA(&b.scontrib, 2 * P);
-    RA(&b.occ, P);
     RA(&b.thr, P);
     RA(&b.rad, P);
     if (image) {
@@ -580,6 +578,14 @@ TraceQueue make_queue(const RaySoA &rays, const HitSoA &hits, const uint32_t *co
     return q;
 }
 
+// The sun rays of b's shadow queue add their contribution where they escape.
+void resolve_into(TraceQueue &q, const PathBuffers &b)
+{
+    q.res_path    = b.spath;
+    q.res_contrib = b.scontrib;
+    q.res_rad     = b.rad;
+}
+
 // A sample pass in flight: the event set it records into and what finishing it needs.
 struct PassTicket {
     int      set    = 0;          // event set (two, so a wavefront can be enqueued while one runs)
@@ -664,7 +670,9 @@ int run_paths(crt_renderer *r, const PathBuffers &b, const RenderParams &rp, hip
         }
         // the epilogue clears the queue the shading appends to (the previous bounce's
         // input), the shadow queue, and the work counters; it counts the extension rays
-        TraceQueue q = make_queue(b.q[cur], b.hits, b.cnt + cnt_queue(cur), b.cnt + kCntWorkExt, b.cnt + kCntErr);
+        HitSoA hits = b.hits;
+        if (!sc.uv) hits.u = hits.v = nullptr;   // the shading interpolates texture coordinates only
+        TraceQueue q = make_queue(b.q[cur], hits, b.cnt + cnt_queue(cur), b.cnt + kCntWorkExt, b.cnt + kCntErr);
         q.tstats     = b.tstats;
         q.done       = b.cnt + kCntDoneExt;
         q.clear0     = b.cnt + cnt_queue(cur ^ 1u);
@@ -689,8 +697,8 @@ int run_paths(crt_renderer *r, const PathBuffers &b, const RenderParams &rp, hip
                 qs.tstats     = b.tstats;
                 qs.done       = b.cnt + kCntDoneShadow;
                 qs.stat       = b.stats + 1;
-                HIP_CHECK(launch_trace_any(sc, qs, b.occ, spill, tc, s));
-                HIP_CHECK(launch_shadow_resolve(b, s));
+                resolve_into(qs, b);
+                HIP_CHECK(launch_trace_any(sc, qs, nullptr, spill, tc, s));
             } else {
                 // closest hit + alpha pass-through, renderer.cpp:330-345 (bounded at 64 steps)
                 HIP_CHECK(launch_shadow_prep(b, s));
@@ -1784,6 +1792,24 @@ int build_two_level(crt_scene *scene, const float *d_corners, const std::vector<
 
 extern "C" {
 
+namespace {
+
+// Least float c in [-1, 1] with acos_cr(c) < size, 2 if there is none: acos falls, so the
+// shading's test "the angle to the sun is below its size" (sampling.h:53-57) is c >= this.
+float sun_cos_in(float size)
+{
+    if (!(acos_cr(1.0f) < size)) return 2.0f;
+    int lo = f2ord(-1.0f), hi = f2ord(1.0f);   // acos_cr(hi) < size
+    while (lo < hi) {
+        const int mid = lo + (hi - lo) / 2;
+        if (acos_cr(ord2f(mid)) < size) hi = mid;
+        else lo = mid + 1;
+    }
+    return ord2f(hi);
+}
+
+}  // namespace
+
 int crt_scene_commit(crt_scene *scene)
 {
     if (!scene) return fail(CRT_ERR_INVALID_ARG, "null scene");
@@ -1932,6 +1958,8 @@ int crt_scene_commit(crt_scene *scene)
     d.sky_rot[1]  = scene->sky_rot[1];
     d.sun_enabled = scene->sun_enabled;
     d.sun.size      = scene->sun.size;
+    d.sun.cos_size  = (float)std::cos((double)scene->sun.size);
+    d.sun.cos_in    = sun_cos_in(scene->sun.size);
     d.sun.intensity = scene->sun.intensity;
     d.sun.dir       = mk3(scene->sun.direction[0], scene->sun.direction[1], scene->sun.direction[2]);
     d.sun.colour    = mk3(scene->sun.colour[0], scene->sun.colour[1], scene->sun.colour[2]);
@@ -2837,8 +2865,8 @@ int record_trace(const PathBuffers &b, const BatchDev &bd, const TraceScene *tsc
                 qs.ray_path = b.spath;
                 qs.path_job = b.pjob;
                 qs.scenes   = tscenes;
-                HIP_CHECK(launch_trace_any_multi(width, qs, b.occ, spill, tc, s));
-                HIP_CHECK(launch_shadow_resolve(b, s));
+                resolve_into(qs, b);
+                HIP_CHECK(launch_trace_any_multi(width, qs, nullptr, spill, tc, s));
             } else {
                 // alpha pass-through (renderer.cpp:330-345): host-driven, never captured
                 for (int step = 0; step < 64; ++step) {

@@ -97,6 +97,8 @@ static_assert(sizeof(InstDev) == 64, "InstDev is 64 bytes");
 struct SunDev {
     float size, intensity;
     f3    dir, colour;
+    float cos_size;   // cos(size), rounded as cos_cr of the shading was
+    float cos_in;     // least c in [-1, 1] whose acos_cr(c) < size (2 if there is none)
 };
 
 // Everything the kernels read about a committed scene.
@@ -130,12 +132,14 @@ struct SceneDev {
     uint32_t           ninst;
 };
 
-// SoA ray buffer
+// SoA ray buffer.  tn / tf null: every ray has the limits kRayNear and infinity, those of the
+// render loop (model.cpp:22-23).
+constexpr float kRayNear = 1e-5f;
 struct RaySoA {
     float *ox, *oy, *oz, *dx, *dy, *dz, *tn, *tf;
 };
 struct HitSoA {
-    float    *t, *u, *v;
+    float    *t, *u, *v;     // u, v null: not wanted
     uint32_t *tri;   // leaf-order triangle index or kInvalidRef
     uint32_t *inst;  // instance of the hit (two-level scenes; may be null)
 };
@@ -185,6 +189,11 @@ struct TraceQueue {
     const uint32_t   *ray_path;
     const uint32_t   *path_job;
     const TraceScene *scenes;
+    // any-hit launches: where rad is set, an unoccluded ray i adds contrib[i] to rad[path[i]]
+    // (a path has at most one ray in the queue) instead of storing its occlusion byte
+    const uint32_t *res_path;
+    const float4   *res_contrib;
+    float4         *res_rad;
     // Epilogue (done != null): the last block with rays zeroes the work counters, the words
     // clear0 / clear1 (when set; never `count`), adds the ray count to *stat (when set) and
     // resets *done, which must be 0 at launch.  It prepares the next bounce's counters
@@ -293,7 +302,6 @@ struct PathBuffers {
     RaySoA    sq;               // shadow queue
     uint32_t *spath;
     float4   *scontrib;         // radiance added if the shadow ray escapes
-    uint8_t  *occ;
     HitSoA    shits;            // closest hits of shadow rays (alpha pass-through)
     float4   *thr, *rad;
     float    *raw;              // W*H*3 running sum, flipped as renderer.cpp:358-365
@@ -395,7 +403,6 @@ hipError_t launch_shade(const SceneDev &sc, const PathBuffers &b, const RenderPa
 constexpr uint32_t kShadeClasses = 4;
 hipError_t launch_shade_sort(const SceneDev &sc, const PathBuffers &b, uint32_t cur, hipStream_t s);
 hipError_t launch_shadow_prep(const PathBuffers &b, hipStream_t s);
-hipError_t launch_shadow_resolve(const PathBuffers &b, hipStream_t s);
 hipError_t launch_shadow_alpha_step(const SceneDev &sc, const PathBuffers &b, hipStream_t s);
 hipError_t launch_accumulate(const PathBuffers &b, uint32_t nsamp, hipStream_t s);
 hipError_t launch_display(const float *raw, uint64_t n, uint32_t npix, float4 *out, hipStream_t s);

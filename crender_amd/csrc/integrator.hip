@@ -82,6 +82,11 @@ __device__ __forceinline__ float4 tex_uv(const SceneDev &sc, int32_t t, float u,
 __device__ __forceinline__ f3 sky(const SceneDev &sc, f3 d)
 {
     if (sc.sky_tex < 0) return mk3(0.0f, 0.0f, 0.0f);
+    const TextureDev td = sc.texs[sc.sky_tex];
+    if (td.w == 1u && td.h == 1u) {   // a constant sky: every direction finds its one texel
+        const float4 c = sc.texels[td.offset];
+        return mk3(c.x, c.y, c.z);
+    }
     const float dy = fminf(fmaxf(d.y, -1.0f), 1.0f);
     const float u  = 0.5f + atan2_cr(d.z, d.x) * kInvTau;
     const float v  = 0.5f - asin_cr(dy) * kInvPi;
@@ -98,9 +103,8 @@ __device__ __forceinline__ float4 mat_colour(const SceneDev &sc, const MaterialD
 // sampling.h:53-57
 __device__ __forceinline__ f3 sun_radiance(const SunDev &s, f3 dir)
 {
-    const float c   = fminf(fmaxf(dot(dir, -s.dir), -1.0f), 1.0f);
-    const float ang = acos_cr(c);
-    return ang < s.size ? s.colour * s.intensity : mk3(0.0f, 0.0f, 0.0f);
+    const float c = fminf(fmaxf(dot(dir, -s.dir), -1.0f), 1.0f);
+    return c >= s.cos_in ? s.colour * s.intensity : mk3(0.0f, 0.0f, 0.0f);
 }
 
 __device__ __forceinline__ void aov_write(const PathBuffers &b, uint32_t p, f3 alb, f3 nrm, float dep)
@@ -114,6 +118,8 @@ __device__ __forceinline__ void aov_write(const PathBuffers &b, uint32_t p, f3 a
     b.aov_dep[q] = make_float4(dd, dd, dd, 1.0f);
 }
 
+// The rays of a wavefront all have the limits kRayNear and infinity, which the traversal
+// supplies (RaySoA::tn and tf are null in its queues).
 __device__ __forceinline__ void put_ray(const RaySoA &q, uint32_t k, f3 o, f3 d)
 {
     q.ox[k] = o.x;
@@ -122,8 +128,6 @@ __device__ __forceinline__ void put_ray(const RaySoA &q, uint32_t k, f3 o, f3 d)
     q.dx[k] = d.x;
     q.dy[k] = d.y;
     q.dz[k] = d.z;
-    q.tn[k] = 1e-5f;              // model.cpp:22
-    q.tf[k] = kInf;               // model.cpp:23
 }
 
 // Rays of the wavefront: rp.nsamp camera rays per pixel (slot p = pixel * nsamp + j, sample
@@ -154,8 +158,8 @@ __global__ __launch_bounds__(256) void k_generate(SceneDev sc, PathBuffers b, Re
         camera_ray(rp.cam, ((float)x + j.a) / (float)b.W, ((float)y + j.b) / (float)b.H, rp.aspect, o, d);
         put_ray(b.q[0], t, o, d);
         b.qpath[0][t] = p;
-        b.thr[p] = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
-        b.rad[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        // throughput 1 and radiance 0 are implied at bounce 0, whose shading stores both
+        if (rp.max_bounces == 0) b.rad[p] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         if (rp.max_bounces == 0 && !trainp && p % ns == ns - 1u) aov_write(b, pix, mk3(0, 0, 0), mk3(0, 0, 0), 0.0f);
     }
     if (blockIdx.x == 0) {
@@ -317,19 +321,39 @@ __device__ __forceinline__ void shade_path(const SceneDev &sc, const PathBuffers
     const f3       o   = mk3(q.ox[k], q.oy[k], q.oz[k]);
     const f3       d   = mk3(q.dx[k], q.dy[k], q.dz[k]);
     const uint32_t tri = b.hits.tri[k];
-    float4         thr4 = b.thr[p];
-    f3             thr  = mk3(thr4.x, thr4.y, thr4.z);
-    float4         rad4 = b.rad[p];
-    f3             rad  = mk3(rad4.x, rad4.y, rad4.z);
+    // Path state is read and written where it is needed only: at bounce 0 it is implied, the
+    // radiance is touched when something is added to it, the throughput kept for the next
+    // bounce.  (float4 both ways for every ray were 64 of the 140 bytes a shaded ray moved.)
+    f3 thr = mk3(1.0f, 1.0f, 1.0f), rad = mk3(0.0f, 0.0f, 0.0f);
+    bool have_rad = bounce == 0, rad_changed = bounce == 0;
+    if (bounce > 0) {
+        const float4 t4 = b.thr[p];
+        thr = mk3(t4.x, t4.y, t4.z);
+    }
+    auto load_rad = [&]() {
+        if (have_rad) return;
+        const float4 r4 = b.rad[p];
+        rad      = mk3(r4.x, r4.y, r4.z);
+        have_rad = true;
+    };
+    // rad + c; adding zeros changes nothing (NaN counts as a change)
+    auto add_rad = [&](f3 c) {
+        if (c.x == 0.0f && c.y == 0.0f && c.z == 0.0f) return;
+        load_rad();
+        rad         = rad + c;
+        rad_changed = true;
+    };
     const bool     can_continue = bounce + 1 < (p >= b.ncam ? rp.nrc.train_term + 1 : rp.max_bounces);
     qthr = thr;
     if (tri == kInvalidRef) {
         const f3 s = sky(sc, d);
         if (bounce == 0 && aov_slot(b, rp, p)) aov_write(b, pix, s, mk3(0, 0, 0), 0.0f);
-        rad = rad + thr * s;
+        add_rad(thr * s);
     } else {
         const uint32_t     inst = sc.instanced && b.hits.inst ? b.hits.inst[k] : kInvalidRef;
-        const HitRec       h = hit_record(sc, o, d, b.hits.t[k], tri, b.hits.u[k], b.hits.v[k], inst, rp.mode == kModePbr);
+        // barycentrics are written for scenes with texture coordinates only
+        const float        bu = sc.uv ? b.hits.u[k] : 0.0f, bv = sc.uv ? b.hits.v[k] : 0.0f;
+        const HitRec       h = hit_record(sc, o, d, b.hits.t[k], tri, bu, bv, inst, rp.mode == kModePbr);
         const MaterialDev &m = sc.mats[sc.mat_idx[h.prim]];
         const float4       col = mat_colour(sc, m, h.u, h.v);
         seg = 1;
@@ -353,6 +377,7 @@ __device__ __forceinline__ void shade_path(const SceneDev &sc, const PathBuffers
                 const size_t slot = (size_t)(p - b.ncam) * rp.nrc.rec_slots + (bounce - rp.nrc.rec_first);
                 nrc_query(rp.nrc, h.point, d, n, cc, m, b.rq + slot * 13);
                 b.r_thr[slot] = make_float4(thr.x, thr.y, thr.z, 1.0f);
+                load_rad();
                 b.r_rad[slot] = make_float4(rad.x, rad.y, rad.z, 0.0f);
             }
             if (rp.nrc.enabled && bounce == 0) {
@@ -406,7 +431,7 @@ __device__ __forceinline__ void shade_path(const SceneDev &sc, const PathBuffers
                         const float cf  = ni <= 1.0f ? -dt : sqrtf(disc);
                         const float r0  = (1.0f - m.ior) / (1.0f + m.ior);
                         const float f0s = r0 * r0;
-                        const float fr  = f0s + (1.0f - f0s) * pow_cr(1.0f - cf, 5.0f);
+                        const float fr  = f0s + (1.0f - f0s) * pow5_cr(1.0f - cf);
                         refl = r2.b < fr;
                     }
                     if (refl) {
@@ -438,9 +463,10 @@ __device__ __forceinline__ void shade_path(const SceneDev &sc, const PathBuffers
                         const f3    t1v   = lensq > 0.0f ? mk3(-vh.y, vh.x, 0.0f) * (1.0f / sqrtf(lensq)) : mk3(1, 0, 0);
                         const f3    t2v   = cross(vh, t1v);
                         const float rr    = sqrtf(r.a);
-                        const float phi   = kTau * r.b;
-                        const float t1    = rr * cos_cr(phi);
-                        float       t2    = rr * sin_cr(phi);
+                        float sp, cp;
+                        sincos_cr(kTau * r.b, sp, cp);
+                        const float t1    = rr * cp;
+                        float       t2    = rr * sp;
                         const float s     = 0.5f * (1.0f + vh.z);
                         t2 = (1.0f - s) * sqrtf(1.0f - t1 * t1) + s * t2;
                         const float nz2 = fmaxf(0.0f, 1.0f - t1 * t1 - t2 * t2);
@@ -471,9 +497,9 @@ __device__ __forceinline__ void shade_path(const SceneDev &sc, const PathBuffers
             const f3 thr_prev = thr;
             if (rp.mode == kModeCompat) {
                 thr = thr * alb;
-                rad = rad + thr * m.emission;
+                add_rad(thr * m.emission);
             } else {
-                rad = rad + (thr_prev * cc) * m.emission;
+                add_rad((thr_prev * cc) * m.emission);
                 thr = thr * alb;
             }
             // sun NEE (renderer.cpp:315-354)
@@ -483,12 +509,13 @@ __device__ __forceinline__ void shade_path(const SceneDev &sc, const PathBuffers
                 const f3 nd_sun = -sun.dir;
                 f3 tb, bb;
                 onb(nd_sun, tb, bb);
-                const float ct  = 1.0f - r.d * (1.0f - cos_cr(sun.size));
-                const float st  = sqrtf(1.0f - ct * ct);
-                const float phi = kTau * r.c;
-                const f3    loc = mk3(cos_cr(phi) * st, ct, sin_cr(phi) * st);
+                const float ct = 1.0f - r.d * (1.0f - sun.cos_size);
+                const float st = sqrtf(1.0f - ct * ct);
+                float sp, cp;
+                sincos_cr(kTau * r.c, sp, cp);
+                const f3 loc = mk3(cp * st, ct, sp * st);
                 sd = tb * loc.x + nd_sun * loc.y + bb * loc.z;
-                const float pdf  = 1.0f / (kTau * (1.0f - cos_cr(sun.size)));
+                const float pdf  = 1.0f / (kTau * (1.0f - sun.cos_size));
                 const float cosv = fminf(fmaxf(dot(nee_n, sd), 0.0f), 1.0f);
                 if (cosv > 0.0f) {
                     const f3 L = sun_radiance(sun, sd);
@@ -541,70 +568,88 @@ __device__ __forceinline__ void shade_path(const SceneDev &sc, const PathBuffers
         if (r2.a >= qv) push_next = false;
         else thr = thr * (1.0f / qv);
     }
-    b.thr[p] = make_float4(thr.x, thr.y, thr.z, 0.0f);
-    b.rad[p] = make_float4(rad.x, rad.y, rad.z, 0.0f);
+    if (push_next) b.thr[p] = make_float4(thr.x, thr.y, thr.z, 0.0f);
+    if (rad_changed) b.rad[p] = make_float4(rad.x, rad.y, rad.z, 0.0f);
 }
 
-// One thread per queued extension ray.  kMulti: paths of many jobs (batched rendering),
-// each path's job, pixel and sample index come from pjob / ppix / psamp.
+// Shades a queue of extension rays, one per thread at a time; the blocks of a fixed grid loop
+// over the queue, whose length only the device knows (a block per 256 path slots, most of them
+// empty after the first bounces, took 75 to 100 us to launch at 1080p).  kMulti: paths of many
+// jobs (batched rendering), each path's job, pixel and sample index come from pjob / ppix /
+// psamp.  Bound by the chain of its loads (ray and hit, triangle, material) at five waves per
+// SIMD: 454 us for 16.6M rays of which half go on, about 2.9 TB/s.  With the sun, its FP64
+// angles used to bound it (sincos_cr, pow5_cr): terrain 1080p, 12 passes of depth 8, 16900 ->
+// 15660 us with them and the loop.
+struct ShadeArgs {
+    SceneDev        sc;
+    PathBuffers     b;
+    RenderParams    rp;
+    const JobDev   *jobs;
+    uint32_t        bounce, cur;
+    const uint32_t *perm;
+};
+
 template <bool kMulti>
-__global__ __launch_bounds__(256) void k_shade(SceneDev sc, PathBuffers b, RenderParams rp, const JobDev *jobs,
-                                               uint32_t bounce, uint32_t cur, const uint32_t *perm)
+__global__ __launch_bounds__(256, 5) void k_shade(ShadeArgs args)
 {
-    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t n = b.cnt[cnt_queue(cur)];
-    const bool     live = t < n;
-    // perm: queue entries in material-class order (the queue index itself otherwise)
-    const uint32_t k = live && perm ? perm[t] : t;
-    ShadeOut o;
-    o.push_next = o.push_shadow = o.do_query = false;
-    o.no = o.nd = o.so = o.sd = o.scontrib = o.qthr = mk3(0, 0, 0);
-    o.seg = 0;
-    uint32_t p = 0;
-    if (live) {
-        p = b.qpath[cur][k];
-        if constexpr (kMulti) {
-            const JobDev &J = jobs[b.pjob[p]];
-            shade_path(J.sc, b, J.rp, k, p, b.ppix[p], b.psamp[p], bounce, cur, o);
-        } else {
-            const uint32_t ns     = rp.nsamp ? rp.nsamp : 1u;
-            const bool     trainp = p >= b.ncam;
-            const uint32_t key    = trainp ? b.npix + (p - b.ncam) : p / ns;
-            shade_path(sc, b, rp, k, p, key, trainp ? (rp.sample | 0x80000000u) : rp.sample + p % ns, bounce, cur, o);
+    // The arguments are read through a pointer to them that the compiler takes for new in every
+    // iteration: loaded ahead of the loop, their 180 words would not fit in scalar registers.
+    typedef const __attribute__((address_space(4))) ShadeArgs KArgs;
+    KArgs *kp = (KArgs *)__builtin_amdgcn_kernarg_segment_ptr();
+    const uint32_t n = kp->b.cnt[cnt_queue(kp->cur)];
+    uint32_t       seg = 0;
+    for (uint32_t t0 = blockIdx.x * blockDim.x; t0 < n; t0 += gridDim.x * blockDim.x) {
+        asm volatile("" : "+s"(kp));
+        const ShadeArgs    &A  = *(const ShadeArgs *)kp;
+        const SceneDev     &sc = A.sc;
+        const PathBuffers  &b  = A.b;
+        const RenderParams &rp = A.rp;
+        const uint32_t bounce = A.bounce, cur = A.cur;
+        const uint32_t t = t0 + threadIdx.x;
+        const bool     live = t < n;
+        // perm: queue entries in material-class order (the queue index itself otherwise)
+        const uint32_t k = live && A.perm ? A.perm[t] : t;
+        ShadeOut o;
+        o.push_next = o.push_shadow = o.do_query = false;
+        o.no = o.nd = o.so = o.sd = o.scontrib = o.qthr = mk3(0, 0, 0);
+        o.seg = 0;
+        uint32_t p = 0;
+        if (live) {
+            p = b.qpath[cur][k];
+            if constexpr (kMulti) {
+                const JobDev &J = A.jobs[b.pjob[p]];
+                shade_path(J.sc, b, J.rp, k, p, b.ppix[p], b.psamp[p], bounce, cur, o);
+            } else {
+                const uint32_t ns     = rp.nsamp ? rp.nsamp : 1u;
+                const bool     trainp = p >= b.ncam;
+                const uint32_t key    = trainp ? b.npix + (p - b.ncam) : p / ns;
+                shade_path(sc, b, rp, k, p, key, trainp ? (rp.sample | 0x80000000u) : rp.sample + p % ns, bounce, cur, o);
+            }
         }
+        if (!kMulti && rp.nrc.enabled) {
+            const uint32_t nqs = block_append(&b.cnt[kCntNrcQ], o.do_query);
+            if (o.do_query) {
+                for (int i = 0; i < 13; ++i) b.nq[(size_t)nqs * 13 + i] = o.nq[i];
+                b.nq_path[nqs] = p;
+                b.nq_thr[nqs]  = make_float4(o.qthr.x, o.qthr.y, o.qthr.z, 0.0f);
+            }
+        }
+        if (kMulti || sc.sun_enabled) {
+            const uint32_t ns = block_append(&b.cnt[kCntShadow], o.push_shadow);
+            if (o.push_shadow) {
+                put_ray(b.sq, ns, o.so, o.sd);
+                b.spath[ns]    = p;
+                b.scontrib[ns] = make_float4(o.scontrib.x, o.scontrib.y, o.scontrib.z, 0.0f);
+            }
+        }
+        const uint32_t nn = block_append(&b.cnt[cnt_queue(cur ^ 1u)], o.push_next);
+        if (o.push_next) {
+            put_ray(b.q[cur ^ 1u], nn, o.no, o.nd);
+            b.qpath[cur ^ 1u][nn] = p;
+        }
+        seg += p < b.ncam ? o.seg : 0u;
     }
-    const uint32_t nqs = (!kMulti && rp.nrc.enabled) ? block_append(&b.cnt[kCntNrcQ], o.do_query) : 0u;
-    if (o.do_query) {
-        for (int k = 0; k < 13; ++k) b.nq[(size_t)nqs * 13 + k] = o.nq[k];
-        b.nq_path[nqs] = p;
-        b.nq_thr[nqs]  = make_float4(o.qthr.x, o.qthr.y, o.qthr.z, 0.0f);
-    }
-    const uint32_t ns = block_append(&b.cnt[kCntShadow], o.push_shadow);
-    if (o.push_shadow) {
-        put_ray(b.sq, ns, o.so, o.sd);
-        b.spath[ns]    = p;
-        b.scontrib[ns] = make_float4(o.scontrib.x, o.scontrib.y, o.scontrib.z, 0.0f);
-    }
-    const uint32_t nn = block_append(&b.cnt[cnt_queue(cur ^ 1u)], o.push_next);
-    if (o.push_next) {
-        put_ray(b.q[cur ^ 1u], nn, o.no, o.nd);
-        b.qpath[cur ^ 1u][nn] = p;
-    }
-    block_add_stat(b.stats, 2, p < b.ncam ? o.seg : 0u);
-}
-
-__global__ __launch_bounds__(256) void k_shadow_resolve(PathBuffers b)
-{
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= b.cnt[kCntShadow]) return;
-    if (b.occ[k]) return;
-    const uint32_t p = b.spath[k];
-    const float4   c = b.scontrib[k];
-    float4         r = b.rad[p];
-    r.x += c.x;
-    r.y += c.y;
-    r.z += c.z;
-    b.rad[p] = r;
+    if (blockIdx.x * blockDim.x < n) block_add_stat(kp->b.stats, 2, seg);
 }
 
 // True if the shadow ray k stopped on a transparent texel (colour.w == 0); o2 = where it continues.
@@ -673,8 +718,6 @@ __global__ __launch_bounds__(256) void k_shadow_compact(PathBuffers b)
         const float4   cc = b.scontrib[s];
         // source indices >= n and destinations < m <= n never overlap
         q.ox[k] = ox; q.oy[k] = oy; q.oz[k] = oz; q.dx[k] = dx; q.dy[k] = dy; q.dz[k] = dz;
-        q.tn[k] = 1e-5f;
-        q.tf[k] = kInf;
         b.spath[k]    = pp;
         b.scontrib[k] = cc;
     }
@@ -692,23 +735,55 @@ __global__ void k_shadow_swap(PathBuffers b)
 }
 
 // raw[pixel] += the radiance of each of the wavefront's samples of the pixel, in sample
-// order: the same sums as one accumulation per pass.
+// order: the same sums as one accumulation per pass.  A pixel's nsamp slots lie side by side,
+// so the block reads its 256 pixels' slots in order (a wave 1 KB at a time) and passes them
+// through LDS to the pixel's thread; a thread reading its own slots touches a line per lane
+// and load (260 us for 16.6M slots, against 60 for their bytes).
+constexpr uint32_t kAccSamples = 8;   // samples per pixel and round (most a wavefront carries)
+
 __global__ __launch_bounds__(256) void k_accumulate(PathBuffers b, uint32_t nsamp)
 {
-    const uint32_t p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= b.npix || b.cnt[kCntNrcBad]) return;
-    const uint32_t x = p % b.W, y = p / b.W;
-    const uint32_t q = (b.W - 1 - x) + (b.H - 1 - y) * b.W;
-    float sx = b.raw[3 * (size_t)q + 0], sy = b.raw[3 * (size_t)q + 1], sz = b.raw[3 * (size_t)q + 2];
-    for (uint32_t j = 0; j < nsamp; ++j) {
-        const float4 r = b.rad[(size_t)p * nsamp + j];
-        sx += r.x;
-        sy += r.y;
-        sz += r.z;
+    __shared__ float lds[3][256 * kAccSamples + 64 * kAccSamples / 8];
+    if (b.cnt[kCntNrcBad]) return;
+    const uint32_t p0 = blockIdx.x * blockDim.x, p = p0 + threadIdx.x;
+    const uint32_t px = min(256u, b.npix - p0);
+    float sx = 0.0f, sy = 0.0f, sz = 0.0f;
+    size_t q = 0;
+    if (p < b.npix) {
+        const uint32_t x = p % b.W, y = p / b.W;
+        q  = (size_t)(b.W - 1 - x) + (size_t)(b.H - 1 - y) * b.W;
+        sx = b.raw[3 * q + 0];
+        sy = b.raw[3 * q + 1];
+        sz = b.raw[3 * q + 2];
     }
-    b.raw[3 * (size_t)q + 0] = sx;
-    b.raw[3 * (size_t)q + 1] = sy;
-    b.raw[3 * (size_t)q + 2] = sz;
+    auto at = [](uint32_t i) { return i + (i >> 5); };   // one word of padding per 32
+    if (nsamp <= kAccSamples) {
+        for (uint32_t i = threadIdx.x; i < px * nsamp; i += 256) {
+            const float4 r = b.rad[(size_t)p0 * nsamp + i];
+            lds[0][at(i)] = r.x;
+            lds[1][at(i)] = r.y;
+            lds[2][at(i)] = r.z;
+        }
+        __syncthreads();
+        if (p < b.npix)
+            for (uint32_t j = 0; j < nsamp; ++j) {
+                const uint32_t i = at(threadIdx.x * nsamp + j);
+                sx += lds[0][i];
+                sy += lds[1][i];
+                sz += lds[2][i];
+            }
+    } else if (p < b.npix) {
+        for (uint32_t j = 0; j < nsamp; ++j) {
+            const float4 r = b.rad[(size_t)p * nsamp + j];
+            sx += r.x;
+            sy += r.y;
+            sz += r.z;
+        }
+    }
+    if (p >= b.npix) return;
+    b.raw[3 * q + 0] = sx;
+    b.raw[3 * q + 1] = sy;
+    b.raw[3 * q + 2] = sz;
 }
 
 // renderer.cpp:371-383: pow(clamp(sum / n, 0, 1), 1/2.2); FLT_MAX before the first pass
@@ -896,8 +971,6 @@ __global__ __launch_bounds__(256) void k_batch_generate(BatchDev bd, PathBuffers
         camera_ray(J.rp.cam, ((float)x + j.a) / (float)J.W, ((float)y + j.b) / (float)J.H, J.rp.aspect, o, d);
         put_ray(b.q[0], p, o, d);
         b.qpath[0][p] = p;
-        b.thr[p]      = make_float4(1.0f, 1.0f, 1.0f, 0.0f);
-        b.rad[p]      = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         b.pjob[p]     = sg.job;
         b.ppix[p]     = pix;
         b.psamp[p]    = sample;
@@ -940,6 +1013,9 @@ __global__ void k_batch_advance(uint32_t *cursor, uint32_t step)
 
 }  // namespace
 
+// Shading blocks: five per CU are resident (93 registers a lane), twice over so that they end evenly.
+constexpr uint32_t kShadeBlocks = 2u * 5u * 256u;
+
 static inline uint32_t blocks(uint64_t n) { return (uint32_t)((n + 255) / 256); }
 
 hipError_t launch_generate(const SceneDev &sc, const PathBuffers &b, const RenderParams &rp, hipStream_t s)
@@ -956,17 +1032,12 @@ hipError_t launch_bounce_prep(const PathBuffers &b, uint32_t cur, hipStream_t s)
 hipError_t launch_shade(const SceneDev &sc, const PathBuffers &b, const RenderParams &rp, uint32_t bounce,
                         uint32_t cur, hipStream_t s, const uint32_t *perm)
 {
-    k_shade<false><<<blocks(b.P), 256, 0, s>>>(sc, b, rp, nullptr, bounce, cur, perm);
+    k_shade<false><<<std::min(blocks(b.P), kShadeBlocks), 256, 0, s>>>(ShadeArgs{sc, b, rp, nullptr, bounce, cur, perm});
     return hipGetLastError();
 }
 hipError_t launch_shadow_prep(const PathBuffers &b, hipStream_t s)
 {
     k_shadow_prep<<<1, 64, 0, s>>>(b);
-    return hipGetLastError();
-}
-hipError_t launch_shadow_resolve(const PathBuffers &b, hipStream_t s)
-{
-    k_shadow_resolve<<<blocks(b.P), 256, 0, s>>>(b);
     return hipGetLastError();
 }
 hipError_t launch_shadow_alpha_step(const SceneDev &sc, const PathBuffers &b, hipStream_t s)
@@ -1032,7 +1103,8 @@ hipError_t launch_batch_generate(const BatchDev &bd, const PathBuffers &b, hipSt
 
 hipError_t launch_shade_multi(const BatchDev &bd, const PathBuffers &b, uint32_t bounce, uint32_t cur, hipStream_t s)
 {
-    k_shade<true><<<blocks(b.P), 256, 0, s>>>(SceneDev{}, b, RenderParams{}, bd.jobs, bounce, cur, nullptr);
+    k_shade<true><<<std::min(blocks(b.P), kShadeBlocks), 256, 0, s>>>(
+        ShadeArgs{SceneDev{}, b, RenderParams{}, bd.jobs, bounce, cur, nullptr});
     return hipGetLastError();
 }
 

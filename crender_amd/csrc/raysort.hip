@@ -56,8 +56,6 @@ __global__ __launch_bounds__(256) void k_ray_gather(RaySoA src, const uint32_t *
     dst.dx[i] = src.dx[j];
     dst.dy[i] = src.dy[j];
     dst.dz[i] = src.dz[j];
-    dst.tn[i] = src.tn[j];
-    dst.tf[i] = src.tf[j];
     dst_path[i] = src_path[j];
 }
 

@@ -512,8 +512,8 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
                 r.o   = mk3(q.rays.ox[rid], q.rays.oy[rid], q.rays.oz[rid]);
                 r.d   = mk3(q.rays.dx[rid], q.rays.dy[rid], q.rays.dz[rid]);
                 if (q.unit_dir && (r.d.x != 0.0f || r.d.y != 0.0f || r.d.z != 0.0f)) r.d = normalize(r.d);
-                r.tn  = q.rays.tn[rid];
-                r.tmax = q.rays.tf[rid];
+                r.tn   = q.rays.tn ? q.rays.tn[rid] : kRayNear;
+                r.tmax = q.rays.tf ? q.rays.tf[rid] : kInf;
                 r.inv = mk3(safe_rcp(r.d.x), safe_rcp(r.d.y), safe_rcp(r.d.z));
                 r.wt  = wt_setup(r.d);
                 r.best_tri = kInvalidRef;
@@ -637,7 +637,18 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
         }
         if (active && cur == kEmpty) {
             if (kAny) {
-                occ[rid] = r.best_tri != kInvalidRef ? 1 : 0;
+                const bool hit = r.best_tri != kInvalidRef;
+                if (!q.res_rad) {
+                    occ[rid] = hit ? 1 : 0;
+                } else if (!hit) {
+                    const uint32_t p = q.res_path[rid];
+                    const float4   c = q.res_contrib[rid];
+                    float4         v = q.res_rad[p];
+                    v.x += c.x;
+                    v.y += c.y;
+                    v.z += c.z;
+                    q.res_rad[p] = v;
+                }
             } else {
                 const bool h = r.best_tri != kInvalidRef;
                 q.hits.t[rid]   = h ? r.tmax : kInf;

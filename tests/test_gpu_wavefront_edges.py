@@ -1,0 +1,43 @@
+"""Edges of the wavefront kernels' launches: images smaller and larger than a block, wavefronts
+of one to eight passes (accumulation through LDS), and more paths than the shading grid has
+threads (2,560 blocks of 256), where its blocks loop.  Images equal the oracle's bit for bit."""
+import numpy as np
+import pytest
+
+from crender_amd import Context, Renderer, scene_from_spec, scenes
+
+pytestmark = pytest.mark.gpu
+
+
+def _render(spec, w, h, bounces, spp, mode, **kw):
+    ctx = Context(0, **kw)
+    sc = scene_from_spec(ctx, spec)
+    r = Renderer(ctx, sc, w, h, bounces)
+    r.set_resolution(w, h)
+    r.set_options(mode=mode, rr_start=3, seed=11)
+    r.render(spp)
+    out = r.raw()
+    r.close()
+    sc.close()
+    ctx.close()
+    return out
+
+
+@pytest.mark.parametrize("mode", [0, 1])
+@pytest.mark.parametrize("w,h,spp", [(1, 1, 8), (17, 15, 7), (16, 16, 3), (257, 1, 5), (33, 31, 9)])
+def test_small_images(oracle, w, h, spp, mode):
+    spec = scenes.sunlit(4, mode=mode)
+    spec.max_bounces, spec.rr_start = 5, 3
+    got = _render(spec, w, h, 5, spp, mode)
+    assert np.array_equal(got, _render(spec, w, h, 5, spp, mode, wavefront_paths=1))   # one pass at a time
+    ref = oracle.render(spec, res=(w, h), spp=spp, seed=11, trav=oracle.BRUTE32)["raw"]
+    assert np.isclose(got, ref, rtol=1e-5, atol=1e-7).all(axis=2).mean() >= 0.999
+
+
+def test_more_paths_than_shading_threads(oracle):
+    spec = scenes.cornell(1)
+    spec.max_bounces, spec.rr_start = 2, 3
+    w, h = 1024, 650   # 665,600 paths
+    got = _render(spec, w, h, 2, 1, 0)
+    ref = oracle.render(spec, res=(w, h), spp=1, seed=11, trav=oracle.BRUTE32)["raw"]
+    assert np.isclose(got, ref, rtol=1e-5, atol=1e-7).all(axis=2).mean() >= 0.999
