@@ -92,8 +92,9 @@ constexpr uint32_t kWavefrontPaths      = 1u << 24;
 constexpr uint32_t kWavefrontPathsCache = 1u << 23;
 constexpr uint32_t kMaxWavefrontPasses = 8;
 
-// most workspace a context keeps between calls: 16 1080p images of 33 MB fit in half of it
-constexpr size_t kWorkspaceMax = 1ull << 30;
+// most workspace a context keeps between calls: a batch of 2^22-path wavefronts takes 1.4 GB,
+// the six images of a 1080p frame 0.2 GB
+constexpr size_t kWorkspaceMax = 4ull << 30;
 
 struct crt_context {
     int         device = 0;
@@ -400,35 +401,52 @@ int alloc_rays_list(std::vector<void *> &list, RaySoA &q, size_t n)
 
 int alloc_rays(crt_renderer *r, RaySoA &q, size_t n) { return alloc_rays_list(r->allocs, q, n); }
 
-// Queue, hit, path-state and cache-query buffers of P paths (no image buffers).
-int alloc_path_core(std::vector<void *> &L, PathBuffers &b, size_t P)
+// Buffers carved one after the other out of a block, each on a 256-byte boundary; with no
+// block yet, the bytes they would take.
+struct Arena {
+    uint8_t *base = nullptr;
+    size_t   used = 0;
+    template <class T>
+    void get(T **p, size_t count)
+    {
+        *p = base ? reinterpret_cast<T *>(base + used) : nullptr;
+        used += (sizeof(T) * count + 255) & ~(size_t)255;
+    }
+};
+
+// Path buffers of a batch: P path slots of queue, hit and path state.  uv: some scene has
+// texture coordinates, sun: some scene has its sun on, alpha: shadow rays pass transparent
+// texels (their continuations are staged behind the queue).
+void carve_batch_paths(Arena &A, PathBuffers &b, size_t P, bool uv, bool sun, bool alpha)
 {
-    int st;
-#define LA(ptr, n)                               \
-    if ((st = lalloc(L, ptr, n)) != CRT_OK) return st
-    if ((st = alloc_rays_list(L, b.q[0], P))) return st;
-    if ((st = alloc_rays_list(L, b.q[1], P))) return st;
-    if ((st = alloc_rays_list(L, b.sq, 2 * P))) return st;
-    LA(&b.qpath[0], P);
-    LA(&b.qpath[1], P);
-    LA(&b.hits.t, P);
-    LA(&b.hits.u, P);
-    LA(&b.hits.v, P);
-    LA(&b.hits.tri, P);
-    LA(&b.hits.inst, P);
-    LA(&b.shits.inst, P);
-    LA(&b.shits.t, P);
-    LA(&b.shits.u, P);
-    LA(&b.shits.v, P);
-    LA(&b.shits.tri, P);
-    LA(&b.spath, 2 * P);
-    LA(&b.scontrib, 2 * P);
-    LA(&b.thr, P);
-    LA(&b.rad, P);
-    LA(&b.cnt, (size_t)kCntWords);
-    LA(&b.stats, (size_t)4 * kStatSlots);
-#undef LA
-    return CRT_OK;
+    auto rays = [&](RaySoA &q, size_t n) {
+        for (float **f : {&q.ox, &q.oy, &q.oz, &q.dx, &q.dy, &q.dz}) A.get(f, n);
+    };
+    auto hits = [&](HitSoA &h, bool bary) {
+        A.get(&h.t, P);
+        A.get(&h.tri, P);
+        if (bary) A.get(&h.u, P);
+        if (bary) A.get(&h.v, P);
+    };
+    for (int k = 0; k < 2; ++k) {
+        rays(b.q[k], P);
+        A.get(&b.qpath[k], P);
+    }
+    hits(b.hits, uv);
+    if (sun) {
+        const size_t n = alpha ? 2 * P : P;
+        rays(b.sq, n);
+        A.get(&b.spath, n);
+        A.get(&b.scontrib, n);
+        if (alpha) hits(b.shits, true);
+    }
+    A.get(&b.thr, P);
+    A.get(&b.rad, P);
+    A.get(&b.pjob, P);
+    A.get(&b.ppix, P);
+    A.get(&b.psamp, P);
+    A.get(&b.cnt, (size_t)kCntWords);
+    A.get(&b.stats, (size_t)4 * kStatSlots);
 }
 
 int alloc_nrc_queries(std::vector<void *> &L, PathBuffers &b, size_t P)
@@ -2814,11 +2832,10 @@ void plan_batch(const crt_job *jobs, uint32_t njobs, uint32_t P, BatchPlan &plan
 
 // Two sets of path buffers replay alternate chunks on two streams (set k renders chunks k,
 // k + 2, ...), so one chunk's traversal overlaps the other's; each chunk's accumulation
-// waits for the previous chunk's, so the job sums are added in chunk order.  Per set: a
-// stream, a chunk cursor, a spill area and, with graphs, one graph for the traversal part of
+// waits for the previous chunk's, so the job sums are added in chunk order.  Per set: one of
+// the context's streams and spill areas, a chunk cursor and, with graphs, one graph for the traversal part of
 // a replay and one for its accumulation.
 struct BatchRun {
-    std::vector<void *> allocs;
     hipStream_t         stream[2] = {nullptr, nullptr};
     hipGraph_t          graph[2][2] = {};      // [set][0: generate + bounces, 1: accumulate + advance]
     hipGraphExec_t      exec[2][2]  = {};
@@ -2835,9 +2852,6 @@ struct BatchRun {
                 if (g) (void)hipGraphDestroy(g);
         for (hipEvent_t e : events)
             if (e) (void)hipEventDestroy(e);
-        for (void *p : allocs) dfree(p);
-        for (hipStream_t s : stream)
-            if (s) (void)hipStreamDestroy(s);
     }
 };
 
@@ -2918,7 +2932,7 @@ int crt_render_batch(crt_context *ctx, const crt_job *jobs, uint32_t njobs, cons
     crt_batch_options_default(&o);
     if (opt) o = *opt;
     uint32_t width = 0, max_bounces = 0;
-    bool any_sun = false, any_alpha = false;
+    bool any_sun = false, any_alpha = false, any_uv = false;
     uint64_t work = 0;
     for (uint32_t j = 0; j < njobs; ++j) {
         const crt_job &J = jobs[j];
@@ -2933,6 +2947,7 @@ int crt_render_batch(crt_context *ctx, const crt_job *jobs, uint32_t njobs, cons
         if (width && w != width) return fail(CRT_ERR_INVALID_ARG, "scenes of one batch must share the BVH width");
         width       = w;
         max_bounces = std::max(max_bounces, J.max_bounces);
+        any_uv      = any_uv || J.scene->dev.uv;
         if (J.scene->dev.sun_enabled) {
             any_sun = true;
             any_alpha = any_alpha || J.scene->dev.any_alpha;
@@ -2945,35 +2960,63 @@ int crt_render_batch(crt_context *ctx, const crt_job *jobs, uint32_t njobs, cons
     uint64_t P64 = o.max_paths ? o.max_paths : (ctx->batch_paths ? ctx->batch_paths : (4u << 20));
     P64 = std::min<uint64_t>(P64, work);
     P64 = std::min<uint64_t>(P64, 1u << 27);
+    // Chunks of about one size where the caller set none, so that the last one does not run
+    // alone: an even share of the work, and a whole pass of the largest image that may not fit
+    // into what an earlier chunk has left.
+    if (!o.max_paths && work > P64) {
+        uint64_t chunks = (work + P64 - 1) / P64, largest = 0;
+        for (uint32_t j = 0; j < njobs; ++j)
+            largest = std::max(largest, std::min<uint64_t>((uint64_t)jobs[j].width * jobs[j].height, P64));
+        P64 = std::min(P64, (work + chunks - 1) / chunks + largest);
+    }
     const uint32_t P = (uint32_t)((P64 + 255) / 256 * 256);
     BatchPlan plan;
     plan_batch(jobs, njobs, P, plan);
     const bool use_graph = o.use_graph && !any_alpha;
 
     HIP_CHECK(hipSetDevice(ctx->device));
-    BatchRun run;
     const uint32_t nrep  = (uint32_t)plan.chunks.size();
     const uint32_t nsets = nrep > 1 ? 2u : 1u;
-    for (uint32_t k = 0; k < nsets; ++k) HIP_CHECK(hipStreamCreateWithFlags(&run.stream[k], hipStreamNonBlocking));
-    hipStream_t s = run.stream[0];
-    auto &L = run.allocs;
-    int st;
+    // everything on the device out of the context's workspace: allocated and freed per call it
+    // took 22 of the 30 ms of eight small scenes.  The spill areas are the context's own.
+    int         st;
+    Workspace   ws;
+    BatchRun    run;
+    Arena       arena;
     PathBuffers b[2]{};
     uint32_t   *spill[2] = {nullptr, nullptr};
+    std::vector<float *> dev_out(njobs, nullptr);
+    JobDev     *d_jobs = nullptr;
+    TraceScene *d_ts = nullptr;
+    BatchSeg   *d_segs = nullptr;
+    BatchChunk *d_chunks = nullptr;
+    uint32_t   *d_cursor = nullptr;   // one per set: chunk k, then k + nsets, ...
+    for (int pass = 0; pass < 2; ++pass) {   // sizes, then addresses
+        arena = Arena{ws.base, 0};
+        for (uint32_t k = 0; k < nsets; ++k) carve_batch_paths(arena, b[k], P, any_uv, any_sun, any_alpha);
+        for (uint32_t j = 0; j < njobs; ++j) {
+            if (jobs[j].memory == CRT_MEM_DEVICE) dev_out[j] = jobs[j].rgb_sum;
+            else arena.get(&dev_out[j], (size_t)jobs[j].width * jobs[j].height * 3);
+        }
+        arena.get(&d_jobs, njobs);
+        arena.get(&d_ts, njobs);
+        arena.get(&d_segs, plan.segs.size());
+        arena.get(&d_chunks, plan.chunks.size());
+        arena.get(&d_cursor, 2);
+        if (pass == 0 && (st = ws.open(ctx, arena.used))) return st;
+    }
     for (uint32_t k = 0; k < nsets; ++k) {
+        if ((st = ensure_spill(ctx, (int)k))) return st;
+        spill[k]      = k ? ctx->spill2 : ctx->spill;
+        run.stream[k] = k ? ctx->stream2 : ctx->stream;
         b[k].P    = P;
         b[k].npix = P;   // no cache-training paths in batches
         b[k].ncam = P;
-        if ((st = alloc_path_core(L, b[k], P))) return st;
-        if ((st = lalloc(L, &b[k].pjob, P))) return st;
-        if ((st = lalloc(L, &b[k].ppix, P))) return st;
-        if ((st = lalloc(L, &b[k].psamp, P))) return st;
-        if ((st = lalloc(L, reinterpret_cast<uint8_t **>(&spill[k]), trace_spill_bytes(ctx->grid, ctx->spill_depth)))) return st;
     }
+    hipStream_t s = run.stream[0];
     // jobs, per-job traversal views, outputs
     std::vector<JobDev>     hj(njobs);
     std::vector<TraceScene> hts(njobs);
-    std::vector<float *>    dev_out(njobs, nullptr);
     for (uint32_t j = 0; j < njobs; ++j) {
         const crt_job &J = jobs[j];
         JobDev &d = hj[j];
@@ -2989,25 +3032,10 @@ int crt_render_batch(crt_context *ctx, const crt_job *jobs, uint32_t njobs, cons
         d.W              = J.width;
         d.H              = J.height;
         const size_t n3  = (size_t)J.width * J.height * 3;
-        if (J.memory == CRT_MEM_DEVICE) {
-            dev_out[j] = J.rgb_sum;
-        } else if ((st = lalloc(L, &dev_out[j], n3))) {
-            return st;
-        }
         HIP_CHECK(hipMemsetAsync(dev_out[j], 0, sizeof(float) * n3, s));
         d.raw   = dev_out[j];
         hts[j]  = TraceScene{J.scene->dev.nodes, J.scene->dev.tri, J.scene->dev.root, J.scene->dev.ntri};
     }
-    JobDev     *d_jobs = nullptr;
-    TraceScene *d_ts = nullptr;
-    BatchSeg   *d_segs = nullptr;
-    BatchChunk *d_chunks = nullptr;
-    uint32_t   *d_cursor = nullptr;
-    if ((st = lalloc(L, &d_jobs, njobs))) return st;
-    if ((st = lalloc(L, &d_ts, njobs))) return st;
-    if ((st = lalloc(L, &d_segs, plan.segs.size()))) return st;
-    if ((st = lalloc(L, &d_chunks, plan.chunks.size()))) return st;
-    if ((st = lalloc(L, &d_cursor, 2))) return st;   // one per set: chunk k, then k + nsets, ...
     HIP_CHECK(hipMemcpyAsync(d_jobs, hj.data(), sizeof(JobDev) * njobs, hipMemcpyHostToDevice, s));
     HIP_CHECK(hipMemcpyAsync(d_ts, hts.data(), sizeof(TraceScene) * njobs, hipMemcpyHostToDevice, s));
     HIP_CHECK(hipMemcpyAsync(d_segs, plan.segs.data(), sizeof(BatchSeg) * plan.segs.size(), hipMemcpyHostToDevice, s));
