@@ -112,15 +112,11 @@ struct crt_context {
     uint32_t    stack  = kStackLds;   // LDS stack entries per traversal lane (8, 16, 32)
     uint32_t    refill = 0, park_min = 0, leaf_rounds = 0;   // traversal thresholds (0: defaults)
     uint32_t    batch_paths = 0;   // tuned wavefront size of crt_render_batch (0 = default)
-    // staging for crt_intersect / crt_occluded
-    uint32_t    stage_cap = 0;
-    float      *st_ray[8] = {};
-    float      *st_t = nullptr, *st_u = nullptr, *st_v = nullptr;
-    uint32_t   *st_tri = nullptr, *st_prim = nullptr, *st_geom = nullptr;
-    uint32_t   *st_inst = nullptr, *st_inst_out = nullptr;
-    float      *st_ng[3] = {};
-    uint8_t    *st_occ = nullptr;
-    uint32_t   *st_cnt = nullptr;   // kQcWords words: count, error flag, work counters
+    // staging for crt_intersect / crt_occluded / crt_cast_rays (QueryStage)
+    uint8_t    *stage = nullptr, *stage_pin = nullptr;
+    size_t      stage_bytes = 0, stage_pin_bytes = 0;
+    uint32_t   *q_cnt = nullptr;    // work counters and epilogue word of queries, 0 between launches
+    uint32_t   *q_err = nullptr;    // pinned: traversal error flag of queries
     uint8_t    *ws = nullptr;       // Workspace
     size_t      ws_bytes = 0;
     uint8_t    *noalloc = nullptr;  // this device's crt_intersect_noalloc scratch (noalloc.hip)
@@ -245,9 +241,17 @@ struct crt_renderer {
 
 namespace {
 
+// Launches of at most this many rays trace with eight lanes per ray (TraceQueue::group_rays).
+// A query alone on the GPU, us a call, a ray per lane against eight lanes per ray: diffuse rays
+// in 100k triangles, 4096: 246 / 120, 65,536: 264 / 207, 131,072: 284 / 307; camera rays in 1M
+// triangles, 65,536: 241 / 139, 131,072: 249 / 196.  A wavefront shares the GPU with another
+// one, where the work counts as well as the chain: within 1 % from 8192 to 98,304.
+constexpr uint32_t kGroupRaysQuery = 98304, kGroupRaysRender = 32768;
+
 TraceConfig trace_cfg(const crt_context *ctx)
 {
-    return TraceConfig{ctx->grid, ctx->stack, ctx->refill, ctx->park_min, ctx->leaf_rounds, ctx->spill_depth};
+    return TraceConfig{ctx->grid, ctx->stack, ctx->refill, ctx->park_min, ctx->leaf_rounds, kGroupRaysRender,
+                       ctx->spill_depth};
 }
 
 // Device memory for the length of one call, kept by the context between calls (an allocation
@@ -1127,35 +1131,136 @@ int reset_accum(crt_renderer *r)
     return CRT_OK;
 }
 
-int stage_reserve(crt_context *ctx, uint32_t n)
+// Memory of one query call of n rays: device arrays of n elements for the traversal, and, for
+// host callers, copies of their rays and results.  Host batches of up to kPinnedRays rays go
+// through pinned memory, gathered there into one block per direction: the runtime stages each
+// copy from or to pageable memory by itself, 8 to 15 us a copy, and a call had up to 20 of
+// them.  Up to kDirectRays the kernels read and write the pinned block itself; above, one copy
+// each way is faster than the bus reads of the traversal.  Larger arrays are copied one by one.
+// Everything is kept by the context, up to the largest call so far.
+constexpr uint32_t kPinnedRays = 131072, kDirectRays = 8192;
+
+struct QueryStage {
+    crt_context *ctx = nullptr;
+    uint32_t     n = 0;
+    size_t       stride = 0;           // bytes between arrays
+    bool         dev = false, pinned = false, direct = false;
+    uint32_t     nin = 0, nout = 0, ntmp = 0;
+    struct Out { void *user; size_t elem; } out[12];
+    uint8_t     *d = nullptr, *h = nullptr;
+    // device block: 8 inputs, 12 outputs, 8 temporaries; pinned block: 8 inputs, 12 outputs
+    static constexpr uint32_t kIn = 8, kOut = 12, kTmp = 8;
+
+    int open(crt_context *c, uint32_t rays, int memory)
+    {
+        ctx    = c;
+        n      = rays;
+        stride = ((size_t)n * 4 + 255) & ~(size_t)255;
+        dev    = memory == CRT_MEM_DEVICE;
+        pinned = !dev && n <= kPinnedRays;
+        direct = pinned && n <= kDirectRays;
+        auto grow = [&](uint8_t *&p, size_t &have, size_t want, bool host) -> int {
+            if (want <= have) return CRT_OK;
+            if (host && p) (void)hipHostFree(p);
+            if (!host) dfree(p);
+            p    = nullptr;
+            have = 0;
+            want = std::max<size_t>(want, 64 * 1024);
+            HIP_CHECK(host ? hipHostMalloc((void **)&p, want) : hipMalloc((void **)&p, want));
+            have = want;
+            return CRT_OK;
+        };
+        int st = grow(ctx->stage, ctx->stage_bytes, stride * (kIn + kOut + kTmp), false);
+        if (!st && pinned) st = grow(ctx->stage_pin, ctx->stage_pin_bytes, stride * (kIn + kOut), true);
+        if (st) return st;
+        if (!ctx->q_cnt) {
+            HIP_CHECK(dalloc(&ctx->q_cnt, (size_t)(kXcds + 1) * kCntLine));
+            HIP_CHECK(hipMemsetAsync(ctx->q_cnt, 0, sizeof(uint32_t) * (kXcds + 1) * kCntLine, ctx->stream));
+        }
+        if (!ctx->q_err) {
+            HIP_CHECK(hipHostMalloc((void **)&ctx->q_err, sizeof(uint32_t)));
+            *ctx->q_err = 0;
+        }
+        d = ctx->stage;
+        h = ctx->stage_pin;
+        return CRT_OK;
+    }
+    // device address of an input array
+    int input(const void *p, float **at)
+    {
+        const size_t off = stride * nin++;
+        if (dev) {
+            *at = static_cast<float *>(const_cast<void *>(p));
+            return CRT_OK;
+        }
+        *at = reinterpret_cast<float *>((direct ? h : d) + off);
+        if (pinned) std::memcpy(h + off, p, (size_t)n * 4);
+        else HIP_CHECK(hipMemcpyAsync(d + off, p, (size_t)n * 4, hipMemcpyHostToDevice, ctx->stream));
+        return CRT_OK;
+    }
+    // an input the caller left out: n times v
+    int fill(float v, float **at)
+    {
+        *at = temp<float>();
+        HIP_CHECK(launch_fill_f32(*at, n, v, ctx->stream));
+        return CRT_OK;
+    }
+    // after the inputs: one copy of the pinned block
+    int inputs_done()
+    {
+        if (pinned && !direct) HIP_CHECK(hipMemcpyAsync(d, h, stride * nin, hipMemcpyHostToDevice, ctx->stream));
+        return CRT_OK;
+    }
+    // device address of an output array, null where the caller wants none
+    template <class T>
+    T *output(T *user)
+    {
+        if (!user || dev) return user;
+        const size_t off = stride * (kIn + nout);
+        out[nout++] = Out{user, sizeof(T)};
+        return reinterpret_cast<T *>((direct ? h : d) + off);
+    }
+    template <class T>
+    T *temp()
+    {
+        return reinterpret_cast<T *>(d + stride * (kIn + kOut + ntmp++));
+    }
+    // the traversal's queue over the rays
+    TraceQueue queue(const RaySoA &rays, const HitSoA &hits, bool unit_dir)
+    {
+        TraceQueue q = make_queue(rays, hits, nullptr, ctx->q_cnt + kCntLine, ctx->q_err, unit_dir);
+        q.n    = n;
+        q.done = ctx->q_cnt;   // the epilogue leaves the counters at 0 for the next call
+        return q;
+    }
+    // copies the outputs to the caller and waits for them
+    int finish()
+    {
+        hipStream_t s = ctx->stream;
+        if (!dev && !pinned)
+            for (uint32_t k = 0; k < nout; ++k)
+                HIP_CHECK(hipMemcpyAsync(out[k].user, d + stride * (kIn + k), out[k].elem * n, hipMemcpyDeviceToHost, s));
+        if (pinned && !direct && nout)
+            HIP_CHECK(hipMemcpyAsync(h + stride * kIn, d + stride * kIn, stride * nout, hipMemcpyDeviceToHost, s));
+        HIP_CHECK(hipStreamSynchronize(s));
+        if (pinned)
+            for (uint32_t k = 0; k < nout; ++k) std::memcpy(out[k].user, h + stride * (kIn + k), out[k].elem * n);
+        if (*ctx->q_err) {
+            *ctx->q_err = 0;
+            return fail(CRT_ERR_HIP, "traversal stack overflow");
+        }
+        return CRT_OK;
+    }
+};
+
+int query_trace(crt_scene *scene, const TraceQueue &q, uint8_t *occ)
 {
-    if (n <= ctx->stage_cap && ctx->st_cnt) return CRT_OK;
-    for (float *&p : ctx->st_ray) dfree(p), p = nullptr;
-    dfree(ctx->st_t);
-    dfree(ctx->st_u);
-    dfree(ctx->st_v);
-    dfree(ctx->st_tri);
-    dfree(ctx->st_prim);
-    dfree(ctx->st_geom);
-    dfree(ctx->st_inst);
-    dfree(ctx->st_inst_out);
-    for (float *&p : ctx->st_ng) dfree(p), p = nullptr;
-    dfree(ctx->st_occ);
-    dfree(ctx->st_cnt);
-    const uint32_t cap = std::max<uint32_t>(n, 1024);
-    for (float *&p : ctx->st_ray) HIP_CHECK(dalloc(&p, cap));
-    HIP_CHECK(dalloc(&ctx->st_t, cap));
-    HIP_CHECK(dalloc(&ctx->st_u, cap));
-    HIP_CHECK(dalloc(&ctx->st_v, cap));
-    HIP_CHECK(dalloc(&ctx->st_tri, cap));
-    HIP_CHECK(dalloc(&ctx->st_prim, cap));
-    HIP_CHECK(dalloc(&ctx->st_geom, cap));
-    HIP_CHECK(dalloc(&ctx->st_inst, cap));
-    HIP_CHECK(dalloc(&ctx->st_inst_out, cap));
-    for (float *&p : ctx->st_ng) HIP_CHECK(dalloc(&p, cap));
-    HIP_CHECK(dalloc(&ctx->st_occ, cap));
-    HIP_CHECK(dalloc(&ctx->st_cnt, (size_t)kQcWords));
-    ctx->stage_cap = cap;
+    crt_context *ctx = scene->ctx;
+    if (int st = ensure_spill(ctx)) return st;
+    TraceConfig tc = trace_cfg(ctx);
+    tc.group_rays  = kGroupRaysQuery;
+    if (occ) HIP_CHECK(launch_trace_any(scene->dev, q, occ, ctx->spill, tc, ctx->stream));
+    else HIP_CHECK(launch_trace_closest(scene->dev, q, ctx->spill, tc, ctx->stream));
     return CRT_OK;
 }
 
@@ -1171,67 +1276,32 @@ int query(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_hits *hits, ui
     if (n == 0) return CRT_OK;
     crt_context *ctx = scene->ctx;
     std::lock_guard<std::mutex> lock(ctx->mu);
-    int st = stage_reserve(ctx, n);
+    QueryStage Q;
+    int st = Q.open(ctx, n, memory);
+    RaySoA  rs{};
+    float **dst[8] = {&rs.ox, &rs.oy, &rs.oz, &rs.dx, &rs.dy, &rs.dz, &rs.tn, &rs.tf};
+    for (int k = 0; k < 8 && !st; ++k) st = Q.input(in[k], dst[k]);
+    if (!st) st = Q.inputs_done();
     if (st) return st;
-    if ((st = ensure_spill(ctx))) return st;
-    hipStream_t s = ctx->stream;
-    RaySoA      rs;
-    float     **dst[8] = {&rs.ox, &rs.oy, &rs.oz, &rs.dx, &rs.dy, &rs.dz, &rs.tn, &rs.tf};
-    for (int k = 0; k < 8; ++k) {
-        if (memory == CRT_MEM_HOST) {
-            HIP_CHECK(hipMemcpyAsync(ctx->st_ray[k], in[k], sizeof(float) * n, hipMemcpyHostToDevice, s));
-            *dst[k] = ctx->st_ray[k];
-        } else {
-            *dst[k] = const_cast<float *>(in[k]);
-        }
+    if (!hits) {
+        if ((st = query_trace(scene, Q.queue(rs, HitSoA{}, false), Q.output(occluded)))) return st;
+        return Q.finish();
     }
-    HIP_CHECK(hipMemsetAsync(ctx->st_cnt, 0, sizeof(uint32_t) * kQcWords, s));
-    HIP_CHECK(hipMemcpyAsync(ctx->st_cnt, &n, sizeof n, hipMemcpyHostToDevice, s));
-    if (hits) {
-        HitSoA h{};
-        const bool dev = memory == CRT_MEM_DEVICE;
-        h.t    = dev ? hits->t : ctx->st_t;
-        h.u    = dev && hits->u ? hits->u : ctx->st_u;
-        h.v    = dev && hits->v ? hits->v : ctx->st_v;
-        h.tri  = ctx->st_tri;
-        h.inst = ctx->st_inst;
-        TraceQueue q = make_queue(rs, h, ctx->st_cnt, ctx->st_cnt + kQcWork, ctx->st_cnt + kQcErr, false);
-        HIP_CHECK(launch_trace_closest(scene->dev, q, ctx->spill, trace_cfg(ctx), s));
-        uint32_t *prim = dev ? hits->prim_id : ctx->st_prim;
-        uint32_t *geom = dev ? hits->geom_id : (hits->geom_id ? ctx->st_geom : nullptr);
-        float    *ng[3] = {hits->ng_x, hits->ng_y, hits->ng_z};
-        float    *ngd[3];
-        for (int k = 0; k < 3; ++k) ngd[k] = ng[k] ? (dev ? ng[k] : ctx->st_ng[k]) : nullptr;
-        uint32_t *inst = hits->inst_id ? (dev ? hits->inst_id : ctx->st_inst_out) : nullptr;
-        HIP_CHECK(launch_hits_to_api(scene->dev, h, n, prim, geom, ngd[0], ngd[1], ngd[2], inst, s));
-        if (!dev) {
-            HIP_CHECK(hipMemcpyAsync(hits->t, ctx->st_t, sizeof(float) * n, hipMemcpyDeviceToHost, s));
-            if (hits->u) HIP_CHECK(hipMemcpyAsync(hits->u, ctx->st_u, sizeof(float) * n, hipMemcpyDeviceToHost, s));
-            if (hits->v) HIP_CHECK(hipMemcpyAsync(hits->v, ctx->st_v, sizeof(float) * n, hipMemcpyDeviceToHost, s));
-            HIP_CHECK(hipMemcpyAsync(hits->prim_id, ctx->st_prim, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, s));
-            if (hits->geom_id)
-                HIP_CHECK(hipMemcpyAsync(hits->geom_id, ctx->st_geom, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, s));
-            if (hits->inst_id)
-                HIP_CHECK(hipMemcpyAsync(hits->inst_id, ctx->st_inst_out, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, s));
-            for (int k = 0; k < 3; ++k)
-                if (ng[k]) HIP_CHECK(hipMemcpyAsync(ng[k], ctx->st_ng[k], sizeof(float) * n, hipMemcpyDeviceToHost, s));
-        }
-    } else {
-        TraceQueue q = make_queue(rs, HitSoA{}, ctx->st_cnt, ctx->st_cnt + kQcWork, ctx->st_cnt + kQcErr, false);
-        uint8_t   *occ = memory == CRT_MEM_DEVICE ? occluded : ctx->st_occ;
-        HIP_CHECK(launch_trace_any(scene->dev, q, occ, ctx->spill, trace_cfg(ctx), s));
-        if (memory == CRT_MEM_HOST) HIP_CHECK(hipMemcpyAsync(occluded, ctx->st_occ, n, hipMemcpyDeviceToHost, s));
-    }
-    uint32_t err = 0;
-    HIP_CHECK(hipMemcpyAsync(&err, ctx->st_cnt + kQcErr, sizeof err, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    if (err) return fail(CRT_ERR_HIP, "traversal stack overflow");
-    return CRT_OK;
+    HitSoA h{};
+    h.t    = Q.output(hits->t);
+    h.u    = Q.output(hits->u);
+    h.v    = Q.output(hits->v);
+    h.tri  = Q.temp<uint32_t>();
+    h.inst = scene->dev.instanced ? Q.temp<uint32_t>() : nullptr;
+    uint32_t *prim = Q.output(hits->prim_id), *geom = Q.output(hits->geom_id);
+    float    *ng[3] = {Q.output(hits->ng_x), Q.output(hits->ng_y), Q.output(hits->ng_z)};
+    uint32_t *inst = Q.output(hits->inst_id);
+    if ((st = query_trace(scene, Q.queue(rs, h, false), nullptr))) return st;
+    HIP_CHECK(launch_hits_to_api(scene->dev, h, n, prim, geom, ng[0], ng[1], ng[2], inst, ctx->stream));
+    return Q.finish();
 }
 
-// scene::cast_ray over a batch (crt_cast_rays).  Host-memory calls stage the rays and reuse
-// the staging buffers for the records: the records kernel reads each element's inputs
-// before it writes that element's outputs.
+// scene::cast_ray over a batch (crt_cast_rays).
 int cast_records(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_records *rec, int memory)
 {
     if (!scene || !rays || !rec) return fail(CRT_ERR_INVALID_ARG, "null argument");
@@ -1244,69 +1314,40 @@ int cast_records(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_records
     if (n == 0) return CRT_OK;
     crt_context *ctx = scene->ctx;
     std::lock_guard<std::mutex> lock(ctx->mu);
-    int st = stage_reserve(ctx, n);
+    QueryStage Q;
+    int st = Q.open(ctx, n, memory);
+    RaySoA  rs{};
+    float **dst[8] = {&rs.ox, &rs.oy, &rs.oz, &rs.dx, &rs.dy, &rs.dz, &rs.tn, &rs.tf};
+    for (int k = 0; k < 8 && !st; ++k)
+        if (in[k]) st = Q.input(in[k], dst[k]);
+    if (!st) st = Q.inputs_done();
+    // a limit left out is the reference's (model.cpp:22-23): supplied by the traversal when both
+    // are, filled in when one is
+    if (!st && !in[6] && in[7]) st = Q.fill(kRayNear, &rs.tn);
+    if (!st && in[6] && !in[7]) st = Q.fill(std::numeric_limits<float>::infinity(), &rs.tf);
     if (st) return st;
-    if ((st = ensure_spill(ctx))) return st;
-    hipStream_t s   = ctx->stream;
-    const bool  dev = memory == CRT_MEM_DEVICE;
-    RaySoA      rs;
-    float     **dst[8] = {&rs.ox, &rs.oy, &rs.oz, &rs.dx, &rs.dy, &rs.dz, &rs.tn, &rs.tf};
-    const float dflt[2] = {1e-5f, std::numeric_limits<float>::infinity()};   // model.cpp:22-23
-    for (int k = 0; k < 8; ++k) {
-        if (!in[k]) {
-            HIP_CHECK(launch_fill_f32(ctx->st_ray[k], n, dflt[k - 6], s));
-            *dst[k] = ctx->st_ray[k];
-        } else if (!dev) {
-            HIP_CHECK(hipMemcpyAsync(ctx->st_ray[k], in[k], sizeof(float) * n, hipMemcpyHostToDevice, s));
-            *dst[k] = ctx->st_ray[k];
-        } else {
-            *dst[k] = const_cast<float *>(in[k]);
-        }
-    }
-    HIP_CHECK(hipMemsetAsync(ctx->st_cnt, 0, sizeof(uint32_t) * kQcWords, s));
-    HIP_CHECK(hipMemcpyAsync(ctx->st_cnt, &n, sizeof n, hipMemcpyHostToDevice, s));
     HitSoA h{};
-    h.t    = ctx->st_t;
-    h.u    = ctx->st_u;
-    h.v    = ctx->st_v;
-    h.tri  = ctx->st_tri;
-    h.inst = ctx->st_inst;
-    TraceQueue q = make_queue(rs, h, ctx->st_cnt, ctx->st_cnt + kQcWork, ctx->st_cnt + kQcErr, true);
-    HIP_CHECK(launch_trace_closest(scene->dev, q, ctx->spill, trace_cfg(ctx), s));
-    // where each field lands on the device, and where it goes on the host
-    struct Field {
-        void  *user;
-        void  *stage;
-        size_t elem;
-    };
-    Field f[12] = {{rec->distance, ctx->st_t, 4},     {rec->prim_id, ctx->st_prim, 4}, {rec->geom_id, ctx->st_geom, 4},
-                   {rec->material, ctx->st_inst_out, 4}, {rec->u, ctx->st_u, 4},        {rec->v, ctx->st_v, 4},
-                   {rec->n_x, ctx->st_ng[0], 4},      {rec->n_y, ctx->st_ng[1], 4},    {rec->n_z, ctx->st_ng[2], 4},
-                   {rec->p_x, ctx->st_ray[0], 4},     {rec->p_y, ctx->st_ray[1], 4},   {rec->p_z, ctx->st_ray[2], 4}};
-    void *o[12];
-    for (int k = 0; k < 12; ++k) o[k] = f[k].user ? (dev ? f[k].user : f[k].stage) : nullptr;
+    h.t    = Q.temp<float>();
+    h.u    = Q.temp<float>();
+    h.v    = Q.temp<float>();
+    h.tri  = Q.temp<uint32_t>();
+    h.inst = scene->dev.instanced ? Q.temp<uint32_t>() : nullptr;
+    if ((st = query_trace(scene, Q.queue(rs, h, true), nullptr))) return st;
     RecordsDev out;
-    out.dist = static_cast<float *>(o[0]);
-    out.prim = static_cast<uint32_t *>(o[1]);
-    out.geom = static_cast<uint32_t *>(o[2]);
-    out.mat  = static_cast<uint32_t *>(o[3]);
-    out.u    = static_cast<float *>(o[4]);
-    out.v    = static_cast<float *>(o[5]);
-    out.nx   = static_cast<float *>(o[6]);
-    out.ny   = static_cast<float *>(o[7]);
-    out.nz   = static_cast<float *>(o[8]);
-    out.px   = static_cast<float *>(o[9]);
-    out.py   = static_cast<float *>(o[10]);
-    out.pz   = static_cast<float *>(o[11]);
-    HIP_CHECK(launch_hit_records(scene->dev, rs, h, n, out, s));
-    if (!dev)
-        for (int k = 0; k < 12; ++k)
-            if (f[k].user) HIP_CHECK(hipMemcpyAsync(f[k].user, f[k].stage, f[k].elem * n, hipMemcpyDeviceToHost, s));
-    uint32_t err = 0;
-    HIP_CHECK(hipMemcpyAsync(&err, ctx->st_cnt + kQcErr, sizeof err, hipMemcpyDeviceToHost, s));
-    HIP_CHECK(hipStreamSynchronize(s));
-    if (err) return fail(CRT_ERR_HIP, "traversal stack overflow");
-    return CRT_OK;
+    out.dist = Q.output(rec->distance);
+    out.prim = Q.output(rec->prim_id);
+    out.geom = Q.output(rec->geom_id);
+    out.mat  = Q.output(rec->material);
+    out.u    = Q.output(rec->u);
+    out.v    = Q.output(rec->v);
+    out.nx   = Q.output(rec->n_x);
+    out.ny   = Q.output(rec->n_y);
+    out.nz   = Q.output(rec->n_z);
+    out.px   = Q.output(rec->p_x);
+    out.py   = Q.output(rec->p_y);
+    out.pz   = Q.output(rec->p_z);
+    HIP_CHECK(launch_hit_records(scene->dev, rs, h, n, out, ctx->stream));
+    return Q.finish();
 }
 
 }  // namespace
@@ -1383,18 +1424,10 @@ int crt_context_destroy(crt_context *ctx)
     (void)hipStreamSynchronize(ctx->stream2);
     dfree(ctx->spill);
     dfree(ctx->spill2);
-    for (float *p : ctx->st_ray) dfree(p);
-    dfree(ctx->st_t);
-    dfree(ctx->st_u);
-    dfree(ctx->st_v);
-    dfree(ctx->st_tri);
-    dfree(ctx->st_prim);
-    dfree(ctx->st_geom);
-    dfree(ctx->st_inst);
-    dfree(ctx->st_inst_out);
-    for (float *p : ctx->st_ng) dfree(p);
-    dfree(ctx->st_occ);
-    dfree(ctx->st_cnt);
+    dfree(ctx->stage);
+    dfree(ctx->q_cnt);
+    if (ctx->stage_pin) (void)hipHostFree(ctx->stage_pin);
+    if (ctx->q_err) (void)hipHostFree(ctx->q_err);
     dfree(ctx->ws);
     (void)hipStreamDestroy(ctx->stream);
     (void)hipStreamDestroy(ctx->stream2);

@@ -180,7 +180,8 @@ struct TraceQueue {
     // distances are in units of the unit direction; 0: the direction as given (rtcIntersect1
     // semantics of crt_intersect / crt_occluded).
     uint32_t        unit_dir;
-    const uint32_t *count;     // device: number of rays
+    const uint32_t *count;     // device: number of rays; null: n of them
+    uint32_t        n;
     uint32_t       *counters;  // device: work counters (kXcds of them, kCntLine words apart), 0 at launch
     uint32_t       *error;     // device: set to 1 if a traversal stack would overflow
     unsigned long long *tstats;  // device [5] or null: node visits, leaf visits, triangle tests,
@@ -204,6 +205,7 @@ struct TraceQueue {
     // set by the launcher from TraceConfig: idle lanes that trigger a refill, and the number
     // of lanes still able to park a leaf below which a wave leaves the inner-node phase
     uint32_t refill_idle, park_min;
+    uint32_t group_rays;    // launches of at most this many rays trace with eight lanes per ray
     uint32_t spill_depth;   // entries per lane of the spill area (multiple of 32)
     uint32_t leaf_rounds;   // leaf-loop iterations per leaf phase before the wave resumes the
                             // inner-node phase (0: until no lane holds a leaf)
@@ -216,6 +218,7 @@ struct TraceConfig {
     uint32_t refill = 0;
     uint32_t park_min = 0;
     uint32_t leaf_rounds = 0;
+    uint32_t group_rays  = 0;             // see TraceQueue
     uint32_t spill_depth = kSpillDepth;   // entries per lane of the spill area given to the launch
 };
 hipError_t launch_trace_closest(const SceneDev &sc, const TraceQueue &q, uint32_t *spill, const TraceConfig &tc,

@@ -837,8 +837,7 @@ __global__ void k_hits_to_api(SceneDev sc, HitSoA h, uint32_t n, uint32_t *prim,
 }
 
 // model.cpp:27-47, and model.cpp:114-118 for a hit on an instance: the intersection record
-// of each traced ray.  Every input of element i is read before any output is written, so the
-// outputs may alias the inputs of the same element (host-staged calls reuse the buffers).
+// of each traced ray.
 __global__ void k_hit_records(SceneDev sc, RaySoA rs, HitSoA h, uint32_t n, RecordsDev out)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;

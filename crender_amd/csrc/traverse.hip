@@ -412,6 +412,198 @@ struct RaySupply {
     }
 };
 
+// ---- few rays ---------------------------------------------------------------------------
+// Eight lanes per ray: lane j of a group tests child j of the group's node, so a node costs
+// one box test per lane instead of eight, its children are ranked by seven comparisons instead of
+// a 19-step network, and up to eight culled stack entries or leaf triangles go in one step.
+// A launch too small to fill the chip is bound by the chain of its longest ray, which this
+// makes about half as long; a full chip does more with a ray per lane (TraceQueue::group_rays).
+// The tests are those of the other mode, so are the hits.
+constexpr uint32_t kGroup     = 8;
+constexpr uint32_t kGroupRays = kTraceBlock / kGroup;   // rays of a block at a time
+
+// Value of lane (l ^ m) of the lane's group of eight, m = 1 .. 7: DPP quad permutations, and
+// the mirror of the half row (lane ^ 7) for the other quad.
+template <int m>
+__device__ __forceinline__ uint32_t group_xor(uint32_t v)
+{
+    constexpr int x    = m < 4 ? m : 7 - m;
+    constexpr int quad = (0 ^ x) | (1 ^ x) << 2 | (2 ^ x) << 4 | (3 ^ x) << 6;   // quad_perm of lane ^ x
+    if constexpr (m >= 4) v = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, 0x141, 0xF, 0xF, false);
+    if constexpr (x > 0) v = (uint32_t)__builtin_amdgcn_update_dpp((int)v, (int)v, quad, 0xF, 0xF, false);
+    return v;
+}
+
+// The group's eight bits of a ballot.
+__device__ __forceinline__ uint32_t group_ballot(bool b, uint32_t lane)
+{
+    return (uint32_t)(__ballot(b) >> (lane & ~(kGroup - 1u))) & 0xFFu;
+}
+
+// Keeps the lane's or its partner's candidate: the nearer hit, at equal distance the smaller
+// primID.
+template <int m>
+__device__ __forceinline__ void group_nearest(float &t, uint32_t &prim, uint32_t &who)
+{
+    const float    ot = __uint_as_float(group_xor<m>(__float_as_uint(t)));
+    const uint32_t op = group_xor<m>(prim), ow = group_xor<m>(who);
+    if (ot < t || (ot == t && op < prim)) {
+        t    = ot;
+        prim = op;
+        who  = ow;
+    }
+}
+
+// Writes the result of ray rid (one lane per ray calls it).
+template <bool kAny>
+__device__ __forceinline__ void store_ray(const TraceQueue &q, uint8_t *occ, uint32_t rid, const RayState &r)
+{
+    const bool h = r.best_tri != kInvalidRef;
+    if (!kAny) {
+        q.hits.t[rid]   = h ? r.tmax : kInf;
+        q.hits.tri[rid] = r.best_tri;
+        if (q.hits.u) q.hits.u[rid] = r.bu;
+        if (q.hits.v) q.hits.v[rid] = r.bv;
+    } else if (!q.res_rad) {
+        occ[rid] = h ? 1 : 0;
+    } else if (!h) {
+        const uint32_t p = q.res_path[rid];
+        const float4   c = q.res_contrib[rid];
+        float4         v = q.res_rad[p];
+        v.x += c.x;
+        v.y += c.y;
+        v.z += c.z;
+        q.res_rad[p] = v;
+    }
+}
+
+// Loads ray rid; false: it is degenerate and hits nothing (ntri: triangles of its scene).
+__device__ __forceinline__ bool load_ray(const TraceQueue &q, uint32_t rid, uint32_t ntri, RayState &r)
+{
+    r.o = mk3(q.rays.ox[rid], q.rays.oy[rid], q.rays.oz[rid]);
+    r.d = mk3(q.rays.dx[rid], q.rays.dy[rid], q.rays.dz[rid]);
+    if (q.unit_dir && (r.d.x != 0.0f || r.d.y != 0.0f || r.d.z != 0.0f)) r.d = normalize(r.d);
+    r.tn   = q.rays.tn ? q.rays.tn[rid] : kRayNear;
+    r.tmax = q.rays.tf ? q.rays.tf[rid] : kInf;
+    r.inv  = mk3(safe_rcp(r.d.x), safe_rcp(r.d.y), safe_rcp(r.d.z));
+    r.wt   = wt_setup(r.d);
+    r.best_tri = r.best_prim = kInvalidRef;
+    r.bu = r.bv = 0.0f;
+    return ntri > 0 && r.tn <= r.tmax && r.tmax == r.tmax && r.tn == r.tn &&
+           (r.d.x != 0.0f || r.d.y != 0.0f || r.d.z != 0.0f);
+}
+
+// The launch's n rays with a group per ray; lds: `depth` entries for each of the block's groups.
+template <bool kAny, bool kMulti>
+__device__ __forceinline__ void trace_groups(const SceneDev &sc, const TraceQueue &q, uint8_t *occ, uint32_t n,
+                                             uint2 *lds, uint32_t depth)
+{
+    const uint32_t lane = lane_id(), j = lane & (kGroup - 1u), slot = threadIdx.x / kGroup;
+    uint2 *stack = lds + slot;
+    for (uint32_t rid = blockIdx.x * kGroupRays + slot; rid < n; rid += gridDim.x * kGroupRays) {
+        const void   *nodes = sc.nodes;
+        const float4 *tris  = sc.tri;
+        uint32_t root = sc.root, ntri = sc.ntri;
+        if constexpr (kMulti) {
+            const TraceScene ts = q.scenes[q.path_job[q.ray_path[rid]]];
+            nodes = ts.nodes;
+            tris  = ts.tri;
+            root  = ts.root;
+            ntri  = ts.ntri;
+        }
+        RayState r;
+        uint32_t cur = load_ray(q, rid, ntri, r) ? root : kEmpty, sp = 0;
+        while (cur != kEmpty) {
+            if (ref_is_leaf(cur)) {
+                const uint32_t first = leaf_first(cur), cnt = leaf_count(cur);
+                for (uint32_t k0 = 0; k0 < cnt; k0 += kGroup) {   // leaves hold up to 16 triangles
+                    float    t = kInf, u = 0.0f, v = 0.0f;
+                    uint32_t prim = kInvalidRef, who = j;
+                    bool     hit = false;
+                    const size_t ti = (size_t)(first + k0 + j);
+                    if (k0 + j < cnt) {
+                        const float4 a = tris[3 * ti + 0], b = tris[3 * ti + 1], c = tris[3 * ti + 2];
+                        hit = wt_test(r.wt, mk3(a.x, a.y, a.z), mk3(b.x, b.y, b.z), mk3(c.x, c.y, c.z), r.o, r.tn, r.tmax,
+                                      t, u, v);
+                        if (hit) prim = __float_as_uint(a.w);
+                        else t = kInf;
+                    }
+                    if (group_ballot(hit, lane) == 0u) continue;
+                    group_nearest<1>(t, prim, who);
+                    group_nearest<2>(t, prim, who);
+                    group_nearest<7>(t, prim, who);
+                    if (t < r.tmax || prim < r.best_prim) {
+                        const int src = (int)((lane & ~(kGroup - 1u)) | who);
+                        r.tmax      = t;
+                        r.best_prim = prim;
+                        r.best_tri  = first + k0 + who;
+                        r.bu        = __shfl(u, src);
+                        r.bv        = __shfl(v, src);
+                    }
+                    if (kAny) break;
+                }
+                if (kAny && r.best_tri != kInvalidRef) break;
+            } else {
+                // child j of the node: NodeOps<8>::expand for one child
+                const Node8Q  &nd = static_cast<const Node8Q *>(nodes)[cur];
+                const uint4    h  = *reinterpret_cast<const uint4 *>(&nd);
+                const uint32_t ref = nd.child[j];
+                const uint32_t qlx = nd.qlox[j], qhx = nd.qhix[j], qly = nd.qloy[j], qhy = nd.qhiy[j], qlz = nd.qloz[j],
+                               qhz = nd.qhiz[j];
+                const float sx = __uint_as_float((h.w & 0xFFu) << 23) * r.inv.x;
+                const float sy = __uint_as_float(((h.w >> 8) & 0xFFu) << 23) * r.inv.y;
+                const float sz = __uint_as_float(((h.w >> 16) & 0xFFu) << 23) * r.inv.z;
+                const float bx = (__uint_as_float(h.x) - r.o.x) * r.inv.x;
+                const float by = (__uint_as_float(h.y) - r.o.y) * r.inv.y;
+                const float bz = (__uint_as_float(h.z) - r.o.z) * r.inv.z;
+                const float dx = 9.5367431640625e-07f * (fabsf(bx) + 255.0f * fabsf(sx));
+                const float dy = 9.5367431640625e-07f * (fabsf(by) + 255.0f * fabsf(sy));
+                const float dz = 9.5367431640625e-07f * (fabsf(bz) + 255.0f * fabsf(sz));
+                const bool  px = r.inv.x >= 0.0f, py = r.inv.y >= 0.0f, pz = r.inv.z >= 0.0f;
+                const float tnx = fmaf((float)(px ? qlx : qhx), sx, bx - dx), tfx = fmaf((float)(px ? qhx : qlx), sx, bx + dx);
+                const float tny = fmaf((float)(py ? qly : qhy), sy, by - dy), tfy = fmaf((float)(py ? qhy : qly), sy, by + dy);
+                const float tnz = fmaf((float)(pz ? qlz : qhz), sz, bz - dz), tfz = fmaf((float)(pz ? qhz : qlz), sz, bz + dz);
+                const float tmin = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, fmaxf(r.tn, 0.0f)));
+                const float tmax = fminf(fminf(tfx, tfy), fminf(tfz, r.tmax));
+                const bool  hit  = j < h.w >> 24 && tmin <= tmax;
+                const uint32_t key = hit ? make_key(tmin, (int)j) : kMissKey;
+                const uint32_t nh = (uint32_t)__popc(group_ballot(hit, lane));
+                if (nh > 0u) {
+                    // hits nearer than this one; misses compare equal among themselves only
+                    const uint32_t rank = (group_xor<1>(key) < key) + (group_xor<2>(key) < key) + (group_xor<3>(key) < key) +
+                                          (group_xor<4>(key) < key) + (group_xor<5>(key) < key) + (group_xor<6>(key) < key) +
+                                          (group_xor<7>(key) < key);
+                    if (sp + nh - 1u > depth) {   // cannot happen for the scenes admitted; never write beyond
+                        *q.error = 1u;
+                        break;
+                    }
+                    if (hit && rank > 0u) stack[(sp + nh - 1u - rank) * kGroupRays] = make_uint2(ref, key & ~7u);
+                    sp += nh - 1u;
+                    const uint32_t near = __builtin_ctz(group_ballot(hit && rank == 0u, lane));
+                    cur = __shfl(ref, (int)((lane & ~(kGroup - 1u)) | near));
+                    continue;
+                }
+            }
+            // next entry closer than the hit, eight entries at a time (the group's LDS accesses stay in
+            // order: its lanes are of one wave)
+            cur = kEmpty;
+            while (sp > 0u) {
+                uint2 e = make_uint2(kEmpty, 0u);
+                if (j < sp) e = stack[(sp - 1u - j) * kGroupRays];
+                const uint32_t m = group_ballot(j < sp && __uint_as_float(e.y) <= r.tmax, lane);
+                if (m) {
+                    const uint32_t i = __builtin_ctz(m);
+                    cur = __shfl(e.x, (int)((lane & ~(kGroup - 1u)) | i));
+                    sp -= i + 1u;
+                    break;
+                }
+                sp -= min(sp, kGroup);
+            }
+        }
+        if (j == 0u) store_ray<kAny>(q, occ, rid, r);
+    }
+}
+
 template <int W, bool kAny, bool kMulti, uint32_t S, bool kInst, bool kStats = false>
 __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev sc, TraceQueue q, uint8_t *occ,
                                                                       uint32_t *spill)
@@ -419,10 +611,19 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
     uint32_t c_nodes = 0, c_leaves = 0, c_tris = 0, c_wnode = 0, c_wleaf = 0;
     uint32_t c_noray = 0, c_empty = 0, c_leafwait = 0;   // idle lanes of node-loop iterations, by cause
     __shared__ uint2 s_stack[(S + 1) * kTraceBlock];
-    const uint32_t n = *q.count;
+    const uint32_t n = q.count ? *q.count : q.n;
     if (n == 0) {
         if (q.done && blockIdx.x == 0 && threadIdx.x == 0) trace_clear(q, n);
         return;
+    }
+    if constexpr (W == 8 && !kInst && !kStats) {
+        constexpr uint32_t kDepth = (S + 1) * kTraceBlock / kGroupRays;
+        if (n <= q.group_rays && q.spill_depth <= kDepth) {
+            if (blockIdx.x * kGroupRays >= n) return;
+            trace_groups<kAny, kMulti>(sc, q, occ, n, s_stack, kDepth);
+            trace_epilogue(q, n, min(gridDim.x, (n + kGroupRays - 1u) / kGroupRays));
+            return;
+        }
     }
     const uint32_t lane = lane_id();
     constexpr uint32_t kWaves = kTraceBlock / 64;
@@ -509,16 +710,6 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
             const uint32_t rank = __popcll(idle & ((1ull << lane) - 1ull));
             if (!active && rank < got) {
                 rid = base + rank;
-                r.o   = mk3(q.rays.ox[rid], q.rays.oy[rid], q.rays.oz[rid]);
-                r.d   = mk3(q.rays.dx[rid], q.rays.dy[rid], q.rays.dz[rid]);
-                if (q.unit_dir && (r.d.x != 0.0f || r.d.y != 0.0f || r.d.z != 0.0f)) r.d = normalize(r.d);
-                r.tn   = q.rays.tn ? q.rays.tn[rid] : kRayNear;
-                r.tmax = q.rays.tf ? q.rays.tf[rid] : kInf;
-                r.inv = mk3(safe_rcp(r.d.x), safe_rcp(r.d.y), safe_rcp(r.d.z));
-                r.wt  = wt_setup(r.d);
-                r.best_tri = kInvalidRef;
-                r.best_prim = kInvalidRef;
-                r.bu = r.bv = 0.0f;
                 st.sp = st.gsp = 0;
                 pend      = kEmpty;
                 pend2     = kEmpty;
@@ -532,8 +723,7 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
                     root  = ts.root;
                     ntri  = ts.ntri;
                 }
-                const bool valid = ntri > 0 && r.tn <= r.tmax && r.tmax == r.tmax && r.tn == r.tn &&
-                                   (r.d.x != 0.0f || r.d.y != 0.0f || r.d.z != 0.0f);
+                const bool valid = load_ray(q, rid, ntri, r);
                 cur    = valid ? root : kEmpty;
                 active = true;
             }
@@ -636,27 +826,8 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
             }
         }
         if (active && cur == kEmpty) {
-            if (kAny) {
-                const bool hit = r.best_tri != kInvalidRef;
-                if (!q.res_rad) {
-                    occ[rid] = hit ? 1 : 0;
-                } else if (!hit) {
-                    const uint32_t p = q.res_path[rid];
-                    const float4   c = q.res_contrib[rid];
-                    float4         v = q.res_rad[p];
-                    v.x += c.x;
-                    v.y += c.y;
-                    v.z += c.z;
-                    q.res_rad[p] = v;
-                }
-            } else {
-                const bool h = r.best_tri != kInvalidRef;
-                q.hits.t[rid]   = h ? r.tmax : kInf;
-                q.hits.tri[rid] = r.best_tri;
-                if (q.hits.u) q.hits.u[rid] = r.bu;
-                if (q.hits.v) q.hits.v[rid] = r.bv;
-                if (kInst && q.hits.inst) q.hits.inst[rid] = h ? best_inst : kInvalidRef;
-            }
+            store_ray<kAny>(q, occ, rid, r);
+            if (kInst && !kAny && q.hits.inst) q.hits.inst[rid] = r.best_tri != kInvalidRef ? best_inst : kInvalidRef;
             active = false;
         }
     }
@@ -714,6 +885,7 @@ hipError_t dispatch_trace(uint32_t width, const TraceConfig &tc, const SceneDev 
     q.refill_idle  = tc.refill ? std::min(tc.refill, 64u) : kRefillIdle;
     q.park_min     = tc.park_min ? std::min(tc.park_min, 64u) : kParkMin;
     q.spill_depth  = tc.spill_depth;
+    q.group_rays   = tc.group_rays;
     q.leaf_rounds  = tc.leaf_rounds ? (tc.leaf_rounds > 64u ? 0u : tc.leaf_rounds) : kLeafRounds;
     if (!kMulti && q.tstats) {
         // instrumented traversal: one stack depth (the counts do not depend on it)
