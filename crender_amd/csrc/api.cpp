@@ -56,16 +56,6 @@ void dfree(void *p)
     if (p) (void)hipFree(p);
 }
 
-uint64_t fnv1a(uint64_t h, const void *data, size_t n)
-{
-    const uint8_t *p = static_cast<const uint8_t *>(data);
-    for (size_t i = 0; i < n; ++i) {
-        h ^= p[i];
-        h *= 1099511628211ull;
-    }
-    return h;
-}
-
 struct ModelHost {
     std::string               name;
     std::vector<float>        corners;   // 9 per triangle
@@ -1568,9 +1558,22 @@ int crt_scene_add_model(crt_scene *scene, const crt_model_data *md, uint32_t *mo
     // registry.cpp:13-24,62-66: expand per corner, primID = triangle order
     m.corners.resize((size_t)n * 9);
     m.mat_idx.resize(n);
+    // Checked array by array first (three passes the compiler vectorises); where every index is
+    // in range and every vertex finite, as in any valid model, expanding is a gather without checks.
+    uint32_t vmax = 0, mmax = 0, wild = 0;
+    for (size_t i = 0; i < 3 * (size_t)n; ++i) vmax = std::max(vmax, md->vertex_indices[i]);
+    for (uint32_t t = 0; t < n; ++t) mmax = std::max(mmax, md->material_indices[t]);
+    const uint32_t *vbits = reinterpret_cast<const uint32_t *>(md->vertices);
+    for (size_t i = 0; n && i < 3 * (size_t)md->num_vertices; ++i) wild |= (vbits[i] & 0x7F800000u) == 0x7F800000u;
+    const bool clean = vmax < md->num_vertices && mmax < md->num_materials && !wild;
+    if (clean) {
+        for (size_t i = 0; i < 3 * (size_t)n; ++i)
+            std::memcpy(&m.corners[3 * i], md->vertices + 3 * (size_t)md->vertex_indices[i], 3 * sizeof(float));
+        std::memcpy(m.mat_idx.data(), md->material_indices, sizeof(uint32_t) * n);
+    }
     const bool has_uv = md->texture_coords && md->texture_indices && md->num_texture_coords;
     if (has_uv) m.uv.resize((size_t)n * 6);
-    for (uint32_t t = 0; t < n; ++t) {
+    for (uint32_t t = 0; t < n && !(clean && !has_uv); ++t) {
         for (int c = 0; c < 3; ++c) {
             const uint32_t vi = md->vertex_indices[3 * (size_t)t + c];
             if (vi >= md->num_vertices) return fail(CRT_ERR_INVALID_MESH, "vertex index out of range at triangle " + std::to_string(t));
@@ -1732,13 +1735,7 @@ int build_two_level(crt_scene *scene, const float *d_corners, const std::vector<
         max_depth = std::max(max_depth, blas[k].depth);
         ms += blas[k].ms;
         bvh2 += blas[k].bvh2_nodes;
-        float lo[3], hi[3];
-        for (int a = 0; a < 3; ++a) lo[a] = hi[a] = m.corners[a];
-        for (size_t i = 0; i < m.corners.size(); i += 3)
-            for (int a = 0; a < 3; ++a) {
-                lo[a] = std::min(lo[a], m.corners[i + a]);
-                hi[a] = std::max(hi[a], m.corners[i + a]);
-            }
+        const float *lo = blas[k].lo, *hi = blas[k].hi;
         for (size_t j = 0; j < m.instances.size() / 16; ++j) {
             const float *M = &m.instances[16 * j];
             double inv[12];
@@ -1871,20 +1868,21 @@ int crt_scene_commit(crt_scene *scene)
     // freed and the new ones built while none of them runs.
     std::lock_guard<std::mutex> ctx_lock(ctx->mu);
     free_scene_device(scene);
-    // concatenate models (scene.cpp:83-95 loops over them; one BVH over all here)
-    std::vector<float>       corners, uv;
-    std::vector<uint32_t>    mat_idx, model_first;
+    // one BVH over all models (scene.cpp:83-95 loops over them)
+    std::vector<float>       uv;
+    std::vector<uint32_t>    model_first;
     std::vector<MaterialDev> mats;
     std::vector<TextureDev>  texs;
     std::vector<float>       texels;
-    bool any_uv = false;
+    std::vector<uint32_t>    mat_base;
+    bool   any_uv = false, any_alpha = false;
+    size_t total = 0;
     for (auto &m : scene->models) any_uv |= !m.uv.empty();
-    bool any_alpha = false;
-    uint64_t h = 1469598103934665603ull;
     for (auto &m : scene->models) {
-        const uint32_t mat_base = (uint32_t)mats.size();
         const uint32_t tex_base = (uint32_t)texs.size();
-        model_first.push_back((uint32_t)mat_idx.size());
+        mat_base.push_back((uint32_t)mats.size());
+        model_first.push_back((uint32_t)total);
+        total += m.mat_idx.size();
         for (size_t i = 0; i < m.tex_data.size(); ++i) {
             TextureDev td;
             td.offset = texels.size() / 4;
@@ -1905,84 +1903,135 @@ int crt_scene_commit(crt_scene *scene)
             if (mt.tex >= 0 || mt.colour[3] == 0.0f) any_alpha = true;
             mats.push_back(d);
         }
-        corners.insert(corners.end(), m.corners.begin(), m.corners.end());
-        for (uint32_t t : m.mat_idx) mat_idx.push_back(mat_base + t);
         if (any_uv) {
-            if (m.uv.empty()) uv.insert(uv.end(), m.corners.size() / 9 * 6, 0.0f);
+            if (m.uv.empty()) uv.insert(uv.end(), m.mat_idx.size() * 6, 0.0f);
             else uv.insert(uv.end(), m.uv.begin(), m.uv.end());
         }
-        h = fnv1a(h, m.corners.data(), m.corners.size() * sizeof(float));
-        h = fnv1a(h, m.mat_idx.data(), m.mat_idx.size() * sizeof(uint32_t));
-        h = fnv1a(h, m.mats.data(), m.mats.size() * sizeof(crt_material));
     }
     int32_t sky_tex = -1;
+    size_t  sky_at  = 0;
     if (scene->has_sky) {
         TextureDev td;
         td.offset = texels.size() / 4;
         td.w      = scene->sky_w;
         td.h      = scene->sky_h;
         sky_tex   = (int32_t)texs.size();
+        sky_at    = texels.size();
         texs.push_back(td);
         texels.insert(texels.end(), scene->sky.begin(), scene->sky.end());
-        h = fnv1a(h, scene->sky.data(), scene->sky.size() * sizeof(float));
     }
-    const uint32_t ntri = (uint32_t)mat_idx.size();
-    if (corners.size() / 9 >= (1u << 27)) return fail(CRT_ERR_UNSUPPORTED, "more than 2^27 triangles");
+    if (total >= (1u << 27)) return fail(CRT_ERR_UNSUPPORTED, "more than 2^27 triangles");
+    const uint32_t ntri = (uint32_t)total;
+    const bool     two_level = scene_instanced(scene);
     float bmin[3] = {0, 0, 0}, bmax[3] = {1, 1, 1};
-    if (!corners.empty()) {
-        for (int k = 0; k < 3; ++k) {
-            bmin[k] = corners[k];
-            bmax[k] = corners[k];
-        }
-        for (size_t i = 0; i < corners.size(); i += 3)
-            for (int k = 0; k < 3; ++k) {
-                bmin[k] = std::min(bmin[k], corners[i + k]);
-                bmax[k] = std::max(bmax[k], corners[i + k]);
-            }
-    }
     hipStream_t s = ctx->stream;
     float *d_corners = nullptr;
-    HIP_CHECK(dalloc(&d_corners, corners.size()));
-    if (!corners.empty()) HIP_CHECK(hipMemcpyAsync(d_corners, corners.data(), sizeof(float) * corners.size(), hipMemcpyHostToDevice, s));
-    const uint32_t width = ctx->opt.bvh_width ? ctx->opt.bvh_width : 8u;
-    const uint32_t max_leaf = ctx->opt.max_leaf ? ctx->opt.max_leaf : 4u;
-    const bool     two_level = scene_instanced(scene);
-    BuildResult br{};
-    uint32_t    max_stack = 0;
-    if (!two_level) {
-        hipError_t be = build_bvh(d_corners, ntri, width, max_leaf, s, &br, ctx->opt.bvh_prim_cost);
-        dfree(d_corners);
-        if (br.invalid) return fail(CRT_ERR_HIP, "BVH build: the builder's consistency checks failed");
-        if (be != hipSuccess) return fail(CRT_ERR_HIP, std::string("BVH build: ") + hipGetErrorString(be));
-        scene->d_nodes = br.nodes;
-        scene->d_tri   = br.tri;
-        max_stack      = ntri ? (width - 1) * br.depth + 1 : 0;
-    } else {
-        const int st2 = build_two_level(scene, d_corners, model_first, width, max_leaf, s, br, bmin, bmax, max_stack);
-        dfree(d_corners);
-        if (st2) {
-            free_scene_device(scene);
-            return st2;
-        }
-        for (auto &m : scene->models) h = fnv1a(h, m.instances.data(), m.instances.size() * sizeof(float));
-    }
-    HIP_CHECK(dalloc(&scene->d_mat_idx, mat_idx.size()));
-    HIP_CHECK(dalloc(&scene->d_mats, std::max<size_t>(mats.size(), 1)));
-    if (!mat_idx.empty()) HIP_CHECK(hipMemcpyAsync(scene->d_mat_idx, mat_idx.data(), sizeof(uint32_t) * mat_idx.size(), hipMemcpyHostToDevice, s));
-    if (!mats.empty()) HIP_CHECK(hipMemcpyAsync(scene->d_mats, mats.data(), sizeof(MaterialDev) * mats.size(), hipMemcpyHostToDevice, s));
-    if (any_uv && !uv.empty()) {
-        HIP_CHECK(dalloc(&scene->d_uv, uv.size() / 2));
-        HIP_CHECK(hipMemcpyAsync(scene->d_uv, uv.data(), sizeof(float) * uv.size(), hipMemcpyHostToDevice, s));
-    }
+    HIP_CHECK(dalloc(&d_corners, total * 9));
+    HIP_CHECK(dalloc(&scene->d_mat_idx, total));
     if (!texs.empty()) {
         HIP_CHECK(dalloc(&scene->d_texs, texs.size()));
         HIP_CHECK(dalloc(&scene->d_texels, texels.size() / 4));
         HIP_CHECK(hipMemcpyAsync(scene->d_texs, texs.data(), sizeof(TextureDev) * texs.size(), hipMemcpyHostToDevice, s));
         HIP_CHECK(hipMemcpyAsync(scene->d_texels, texels.data(), sizeof(float) * texels.size(), hipMemcpyHostToDevice, s));
     }
+    // The scene hash of a checkpoint: per model its corners, material indices and materials, then
+    // the sky, then the instances of a two-level scene.  Hashed on the device, on the second
+    // stream beside the BVH build; the small arrays are gathered in one block for it.
+    std::vector<uint8_t> small;
+    for (auto &m : scene->models) {
+        const uint8_t *p = reinterpret_cast<const uint8_t *>(m.mats.data());
+        small.insert(small.end(), p, p + m.mats.size() * sizeof(crt_material));
+    }
+    const size_t inst_at = small.size();
+    for (auto &m : scene->models) {
+        const uint8_t *p = reinterpret_cast<const uint8_t *>(m.instances.data());
+        if (two_level) small.insert(small.end(), p, p + m.instances.size() * sizeof(float));
+    }
+    Workspace ws;
+    struct Drain {   // nothing runs on the workspace or the arrays when the call ends
+        hipStream_t s;
+        ~Drain() { (void)hipStreamSynchronize(s); }
+    } drain{ctx->stream2};
+    uint8_t  *hash_tmp = nullptr, *d_small = nullptr;
+    uint64_t *d_hash = nullptr;
+    for (int pass = 0; pass < 2; ++pass) {
+        Arena A{ws.base, 0};
+        A.get(&hash_tmp, hash_scratch_bytes(std::max({9 * total, scene->sky.size(), small.size() / 4})));
+        A.get(&d_hash, 1);
+        A.get(&d_small, small.size());
+        if (pass == 0)
+            if (int st = ws.open(ctx, A.used)) return st;
+    }
+    for (size_t k = 0; k < scene->models.size(); ++k) {
+        const ModelHost &m = scene->models[k];
+        const size_t     n = m.mat_idx.size(), at = model_first[k];
+        if (!n) continue;
+        HIP_CHECK(hipMemcpyAsync(d_corners + 9 * at, m.corners.data(), sizeof(float) * 9 * n, hipMemcpyHostToDevice, s));
+        HIP_CHECK(hipMemcpyAsync(scene->d_mat_idx + at, m.mat_idx.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice, s));
+    }
+    if (!small.empty()) HIP_CHECK(hipMemcpyAsync(d_small, small.data(), small.size(), hipMemcpyHostToDevice, s));
+    {
+        hipStream_t s2 = ctx->stream2;
+        hipEvent_t  uploaded;
+        HIP_CHECK(hipEventCreateWithFlags(&uploaded, hipEventDisableTiming));
+        hipError_t e = hipEventRecord(uploaded, s);
+        if (e == hipSuccess) e = hipStreamWaitEvent(s2, uploaded, 0);
+        (void)hipEventDestroy(uploaded);
+        HIP_CHECK(e);
+        HIP_CHECK(launch_hash_init(d_hash, s2));
+        size_t mat_at = 0;
+        for (size_t k = 0; k < scene->models.size(); ++k) {
+            const ModelHost &m = scene->models[k];
+            const size_t     n = m.mat_idx.size(), at = model_first[k], mw = m.mats.size() * sizeof(crt_material) / 4;
+            HIP_CHECK(launch_hash(d_corners + 9 * at, 9 * n, d_hash, hash_tmp, s2));
+            HIP_CHECK(launch_hash(scene->d_mat_idx + at, n, d_hash, hash_tmp, s2));
+            HIP_CHECK(launch_hash(d_small + mat_at, mw, d_hash, hash_tmp, s2));
+            // the model's materials follow those of the models before it
+            if (mat_base[k]) HIP_CHECK(launch_add_u32(scene->d_mat_idx + at, (uint32_t)n, mat_base[k], s2));
+            mat_at += 4 * mw;
+        }
+        if (scene->has_sky)
+            HIP_CHECK(launch_hash(reinterpret_cast<float *>(scene->d_texels) + sky_at, scene->sky.size(), d_hash, hash_tmp, s2));
+        HIP_CHECK(launch_hash(d_small + inst_at, (small.size() - inst_at) / 4, d_hash, hash_tmp, s2));
+    }
+    const uint32_t width = ctx->opt.bvh_width ? ctx->opt.bvh_width : 8u;
+    const uint32_t max_leaf = ctx->opt.max_leaf ? ctx->opt.max_leaf : 4u;
+    BuildResult br{};
+    uint32_t    max_stack = 0;
+    if (!two_level) {
+        hipError_t be = build_bvh(d_corners, ntri, width, max_leaf, s, &br, ctx->opt.bvh_prim_cost);
+        (void)hipStreamSynchronize(ctx->stream2);   // the hash reads the corners too
+        dfree(d_corners);
+        if (br.invalid) return fail(CRT_ERR_HIP, "BVH build: the builder's consistency checks failed");
+        if (be != hipSuccess) return fail(CRT_ERR_HIP, std::string("BVH build: ") + hipGetErrorString(be));
+        scene->d_nodes = br.nodes;
+        scene->d_tri   = br.tri;
+        max_stack      = ntri ? (width - 1) * br.depth + 1 : 0;
+        for (int k = 0; k < 3 && ntri; ++k) {
+            bmin[k] = br.lo[k];
+            bmax[k] = br.hi[k];
+        }
+    } else {
+        const int st2 = build_two_level(scene, d_corners, model_first, width, max_leaf, s, br, bmin, bmax, max_stack);
+        (void)hipStreamSynchronize(ctx->stream2);
+        dfree(d_corners);
+        if (st2) {
+            free_scene_device(scene);
+            return st2;
+        }
+    }
+    HIP_CHECK(dalloc(&scene->d_mats, std::max<size_t>(mats.size(), 1)));
+    if (!mats.empty()) HIP_CHECK(hipMemcpyAsync(scene->d_mats, mats.data(), sizeof(MaterialDev) * mats.size(), hipMemcpyHostToDevice, s));
+    if (any_uv && !uv.empty()) {
+        HIP_CHECK(dalloc(&scene->d_uv, uv.size() / 2));
+        HIP_CHECK(hipMemcpyAsync(scene->d_uv, uv.data(), sizeof(float) * uv.size(), hipMemcpyHostToDevice, s));
+    }
     HIP_CHECK(dalloc(&scene->d_model_first, std::max<size_t>(model_first.size(), 1)));
     if (!model_first.empty())
         HIP_CHECK(hipMemcpyAsync(scene->d_model_first, model_first.data(), sizeof(uint32_t) * model_first.size(), hipMemcpyHostToDevice, s));
+    uint64_t hash = 0;
+    HIP_CHECK(hipMemcpyAsync(&hash, d_hash, sizeof hash, hipMemcpyDeviceToHost, ctx->stream2));
+    HIP_CHECK(hipStreamSynchronize(ctx->stream2));
     HIP_CHECK(hipStreamSynchronize(s));
 
     if (max_stack > kSpillDepth + 8) {   // capacity of the smallest LDS stack configuration
@@ -2034,7 +2083,7 @@ int crt_scene_commit(crt_scene *scene)
     bi.bytes           = (uint64_t)br.node_count * 128u + (uint64_t)ntri * 48u;
     // a lane spills at most its deepest stack, a whole LDS stack (8 to 32 entries) at a time
     ctx->spill_depth = std::max(ctx->spill_depth, std::min(kSpillDepth, (max_stack + 31u) / 32u * 32u));
-    scene->hash      = h;
+    scene->hash      = hash;
     scene->committed = true;
     scene->dirty     = false;
     return ensure_spill(ctx);

@@ -1922,6 +1922,10 @@ hipError_t build_bvh(const float *d_tri, uint32_t ntri, uint32_t width, uint32_t
     out->node_count = nwide;
     out->bvh2_nodes = used_h;
     out->depth      = depth;
+    for (int k = 0; k < 3; ++k) {
+        out->lo[k] = root_node.lo[k];
+        out->hi[k] = root_node.hi[k];
+    }
     out->root       = 0;
     out->sah        = ra > 0.0 ? sah_h / ra : 0.0;
     out->ms         = ms;

@@ -154,6 +154,7 @@ struct BuildResult {
     uint32_t root;
     double   sah;
     float    ms;
+    float    lo[3], hi[3];  // box of all triangles
     uint32_t invalid = 0;   // 1: the builder's own consistency checks failed (hipErrorUnknown)
 };
 // Builds the BVH of ntri triangles (9 floats each, device memory) on stream s.
@@ -166,6 +167,13 @@ hipError_t bvh_rebase(void *nodes, uint32_t count, uint32_t width, uint32_t node
                       hipStream_t s);
 // Adds `base` to the primID stored in v0.w of every leaf-order triangle.
 hipError_t tri_add_prim_base(float4 *tri, uint32_t ntri, uint32_t base, hipStream_t s);
+
+// ---- scene hash (scene_hash.hip) --------------------------------------------------------
+// *h (device) = the FNV-1a hash of nwords 32-bit words (device) that continues from *h;
+// launch_hash_init: the empty hash.  scratch: hash_scratch_bytes(nwords) or more.
+size_t     hash_scratch_bytes(size_t nwords);
+hipError_t launch_hash_init(uint64_t *h, hipStream_t s);
+hipError_t launch_hash(const void *words, size_t nwords, uint64_t *h, void *scratch, hipStream_t s);
 
 // ---- traversal ----------------------------------------------------------------------
 constexpr uint32_t kXcds    = 8;
@@ -429,6 +437,7 @@ struct RecordsDev {
 hipError_t launch_hit_records(const SceneDev &sc, const RaySoA &rs, const HitSoA &h, uint32_t n, const RecordsDev &out,
                               hipStream_t s);
 hipError_t launch_fill_f32(float *p, uint32_t n, float v, hipStream_t s);
+hipError_t launch_add_u32(uint32_t *p, uint32_t n, uint32_t v, hipStream_t s);
 hipError_t launch_hits_to_api(const SceneDev &sc, const HitSoA &h, uint32_t n, uint32_t *prim, uint32_t *geom,
                               float *ngx, float *ngy, float *ngz, uint32_t *inst, hipStream_t s);
 

@@ -883,6 +883,12 @@ __global__ void k_fill_f32(float *p, uint32_t n, float v)
     if (i < n) p[i] = v;
 }
 
+__global__ void k_add_u32(uint32_t *p, uint32_t n, uint32_t v)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) p[i] += v;
+}
+
 // rad[path] += throughput * max(prediction, 0) for every cache query
 __global__ __launch_bounds__(256) void k_nrc_apply(PathBuffers b)
 {
@@ -1091,6 +1097,12 @@ hipError_t launch_hit_records(const SceneDev &sc, const RaySoA &rs, const HitSoA
 hipError_t launch_fill_f32(float *p, uint32_t n, float v, hipStream_t s)
 {
     if (n) k_fill_f32<<<blocks(n), 256, 0, s>>>(p, n, v);
+    return hipGetLastError();
+}
+
+hipError_t launch_add_u32(uint32_t *p, uint32_t n, uint32_t v, hipStream_t s)
+{
+    if (n) k_add_u32<<<blocks(n), 256, 0, s>>>(p, n, v);
     return hipGetLastError();
 }
 
