@@ -13,11 +13,11 @@
 //     start and takes further ones in chunks (RaySupply).
 //   * refill: when 16 or more lanes of a wave are idle, they take rays of the wave's chunk
 //     by ballot rank.
-//   * per-lane short stack in LDS (entry-major (ref, distance) pairs; 8, 16 or 32 entries), spilled
-//     a full stack at a time to a per-lane global region when full.  Entries carry the child's entry
-//     distance so popped nodes beyond the current hit are skipped.
+//   * per-lane short stack in LDS (entry-major (ref, distance) pairs; 8, 16 or 32 entries, growing
+//     downwards), spilled a full stack at a time to a per-lane global region when full.  Entries carry
+//     the child's entry distance so popped nodes beyond the current hit are skipped.
 //   * children are ordered by entry distance with a sorting network; the nearest is
-//     visited next and the others pushed far-to-near, with unconditional LDS writes.
+//     visited next and the others are written behind it, nearest on top.
 //   * leaf parking: a lane that reaches a leaf keeps it aside (up to two) and continues
 //     down the tree until most lanes of the wave hold their leaves (fewer than 16 can still
 //     park one), so the triangle phase runs with more lanes busy (Aila and Laine 2009,
@@ -31,7 +31,7 @@ namespace {
 
 constexpr float kInf = __builtin_huge_valf();
 constexpr uint32_t kEmpty = kInvalidRef;
-constexpr uint32_t kMissKey = 0xFFFFFFFFu;
+constexpr uint32_t kMissKey = 0x7FE00000u;   // behind every distance
 // default idle lanes that trigger a refill.  1080p soup 20 passes / terrain 8 passes with rays
 // from the wave's own chunk: 8 -> 26.4 / 12.5 ms, 16 -> 26.5 / 12.5, 24 -> 26.7 / 12.5, 32 -> 26.9 / 12.5
 constexpr uint32_t kRefillIdle = 16;
@@ -57,23 +57,38 @@ struct RayState {
     float  bu, bv;
 };
 
-// compare-exchange of (key, ref) pairs; refs travel with their keys so that every array
-// index stays static and the arrays live in registers
-__device__ __forceinline__ void cswap(uint32_t &a, uint32_t &b, uint32_t &ra, uint32_t &rb)
+// Child of a node to be sorted: entry distance bits above, ref below, read as one FP64 number.
+// Distances are non-negative floats and kMissKey is below the bits of an FP64 infinity, so the
+// order of the numbers is that of the distances (of the refs among equal ones) and none is a NaN.
+typedef double Child;
+
+__device__ __forceinline__ Child make_child(uint32_t key, uint32_t ref)
 {
-    const bool     sw = b < a;
-    const uint32_t ka = sw ? b : a, kb = sw ? a : b;
-    const uint32_t xa = sw ? rb : ra, xb = sw ? ra : rb;
-    a  = ka;
-    b  = kb;
-    ra = xa;
-    rb = xb;
+    return __builtin_bit_cast(double, make_uint2(ref, key));
+}
+__device__ __forceinline__ uint32_t child_key(Child c) { return __builtin_bit_cast(uint2, c).y; }
+__device__ __forceinline__ uint32_t child_ref(Child c) { return __builtin_bit_cast(uint2, c).x; }
+
+// compare-exchange: FP64 min and max move all 64 bits of the smaller and the larger one
+// (FP64 denormals are kept, and a distance of 0 gives one) at FP32 rate on gfx950: 2
+// instructions a comparator instead of a compare and four selects, 38 of the 95 for eight children.
+// With the pair pushed as it is and rows a constant apart a node step takes about 230 VALU
+// instructions instead of 300; the step is bound by these and by the latency of the node's
+// load.  1080p, before -> after: soup 8 passes 11.0 -> 10.2 ms, terrain 8 passes 12.5 -> 10.5 ms,
+// camera rays 694 -> 634 us.
+__device__ __forceinline__ void cswap(Child &a, Child &b)
+{
+    Child lo, hi;
+    asm("v_min_f64 %0, %1, %2" : "=v"(lo) : "v"(a), "v"(b));
+    asm("v_max_f64 %0, %1, %2" : "=v"(hi) : "v"(a), "v"(b));
+    a = lo;
+    b = hi;
 }
 
 template <int W>
-__device__ __forceinline__ void sort_pairs(uint32_t (&k)[W], uint32_t (&r)[W])
+__device__ __forceinline__ void sort_children(Child (&c)[W])
 {
-#define CS(i, j) cswap(k[i], k[j], r[i], r[j])
+#define CS(i, j) cswap(c[i], c[j])
     if constexpr (W == 4) {
         CS(0, 1); CS(2, 3);
         CS(0, 2); CS(1, 3);
@@ -119,22 +134,26 @@ __device__ __forceinline__ bool slab(float lx, float hx, float ly, float hy, flo
     return tmin <= fminf(tmax, r.tmax);
 }
 
+// Keeps a load where it is written (the compiler would sink one that only some lanes need below
+// the branch, behind the tests, and wait for memory a second time).  The child refs of a node:
+// soup 8 passes 10.2 -> 9.8 ms, terrain 10.5 -> 10.2 ms, camera rays 615 -> 596 us.
+__device__ __forceinline__ void keep_load(uint4 &v)
+{
+    asm volatile("" : "+v"(v.x), "+v"(v.y), "+v"(v.z), "+v"(v.w));
+}
+
 template <int W>
 struct NodeOps;
 
 template <>
 struct NodeOps<4> {
-    static __device__ __forceinline__ int expand(const void *nodes, uint32_t idx, const RayState &r, uint32_t (&key)[4],
-                                                 uint32_t (&ref)[4])
+    static __device__ __forceinline__ int expand(const void *nodes, uint32_t idx, const RayState &r, Child (&c)[4])
     {
         const float4 *p = reinterpret_cast<const float4 *>(static_cast<const Node4 *>(nodes) + idx);
         const float4  lx = p[0], hx = p[1], ly = p[2], hy = p[3], lz = p[4], hz = p[5];
         const uint4   ch = reinterpret_cast<const uint4 *>(p)[6];
         const uint32_t nc = reinterpret_cast<const uint4 *>(p)[7].x;
-        ref[0] = ch.x;
-        ref[1] = ch.y;
-        ref[2] = ch.z;
-        ref[3] = ch.w;
+        const uint32_t ref[4] = {ch.x, ch.y, ch.z, ch.w};
         const float LX[4] = {lx.x, lx.y, lx.z, lx.w}, HX[4] = {hx.x, hx.y, hx.z, hx.w};
         const float LY[4] = {ly.x, ly.y, ly.z, ly.w}, HY[4] = {hy.x, hy.y, hy.z, hy.w};
         const float LZ[4] = {lz.x, lz.y, lz.z, lz.w}, HZ[4] = {hz.x, hz.y, hz.z, hz.w};
@@ -143,7 +162,7 @@ struct NodeOps<4> {
         for (int j = 0; j < 4; ++j) {
             float t;
             const bool h = (uint32_t)j < nc && slab(LX[j], HX[j], LY[j], HY[j], LZ[j], HZ[j], r, t);
-            key[j] = h ? make_key(t, j) : kMissKey;
+            c[j] = make_child(h ? __float_as_uint(t) : kMissKey, ref[j]);
             nh += h ? 1 : 0;
         }
         return nh;
@@ -160,15 +179,15 @@ struct NodeOps<8> {
     // The entry plane of an axis is the low one for a positive direction and the high one for
     // a negative direction, so the byte words are picked once per node (lo <= hi holds for
     // every child slot below the child count) and a child costs no min/max per axis.
-    static __device__ __forceinline__ int expand(const void *nodes, uint32_t idx, const RayState &r, uint32_t (&key)[8],
-                                                 uint32_t (&ref)[8])
+    static __device__ __forceinline__ int expand(const void *nodes, uint32_t idx, const RayState &r, Child (&c)[8])
     {
         const uint4 *p  = reinterpret_cast<const uint4 *>(static_cast<const Node8Q *>(nodes) + idx);
         const uint4  h  = p[0];
-        const uint4  c0 = p[1], c1 = p[2];
+        uint4        c0 = p[1], c1 = p[2];
         const uint4  qx = p[3], qy = p[4], qz = p[5];
-        ref[0] = c0.x; ref[1] = c0.y; ref[2] = c0.z; ref[3] = c0.w;
-        ref[4] = c1.x; ref[5] = c1.y; ref[6] = c1.z; ref[7] = c1.w;
+        keep_load(c0);
+        keep_load(c1);
+        const uint32_t ref[8] = {c0.x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w};
         const float sx = __uint_as_float((h.w & 0xFFu) << 23) * r.inv.x;
         const float sy = __uint_as_float(((h.w >> 8) & 0xFFu) << 23) * r.inv.y;
         const float sz = __uint_as_float(((h.w >> 16) & 0xFFu) << 23) * r.inv.z;
@@ -199,7 +218,7 @@ struct NodeOps<8> {
             const float tmin = fmaxf(fmaxf(tnx, tny), fmaxf(tnz, tn0));
             const float tmax = fminf(fminf(tfx, tfy), fminf(tfz, r.tmax));
             const bool hit = (uint32_t)j < nc && tmin <= tmax;
-            key[j] = hit ? make_key(tmin, j) : kMissKey;
+            c[j] = make_child(hit ? __float_as_uint(tmin) : kMissKey, ref[j]);
             nh += hit ? 1 : 0;
         }
         return nh;
@@ -208,52 +227,62 @@ struct NodeOps<8> {
 
 template <uint32_t S>
 struct Stack {
-    uint2    *s;        // LDS [S + 1][kTraceBlock] of (ref, entry distance bits); row S absorbs
-                        // the writes of children that missed
+    uint2    *s;        // this lane's column of the LDS stack, [S][kTraceBlock] of (ref, entry distance
+                        // bits), filled from row S - 1 downwards
     uint4    *g;        // this lane's global spill: `depth` (ref, distance) entries, contiguous, so
                         // that a spill of S entries writes S * 8 bytes of whole lines (uint4 = 2 entries)
-    uint32_t  tid;
-    uint32_t  sp, gsp, depth;
+    uint32_t  top, gsp, depth;   // row of the top entry (S: none in LDS), entries spilled
 
     uint32_t *err;
 
-    __device__ __forceinline__ void push(uint32_t ref, float dist)
+    __device__ __forceinline__ void clear()
     {
-        if (sp == S) {
+        top = S;
+        gsp = 0;
+    }
+    __device__ __forceinline__ void push(uint2 e)
+    {
+        if (top == 0) {
             if (gsp + S > depth) {
                 // cannot happen for trees admitted at commit; never write out of bounds
                 *err = 1u;
                 return;
             }
             for (uint32_t k = 0; k < S; k += 2) {
-                const uint2 a = s[k * kTraceBlock + tid], b = s[(k + 1) * kTraceBlock + tid];
+                const uint2 a = s[k * kTraceBlock], b = s[(k + 1) * kTraceBlock];
                 g[(gsp + k) / 2] = make_uint4(a.x, a.y, b.x, b.y);
             }
             gsp += S;
-            sp = 0;
+            top = S;
         }
-        s[sp * kTraceBlock + tid] = make_uint2(ref, __float_as_uint(dist));
-        ++sp;
+        --top;
+        s[top * kTraceBlock] = e;
     }
-    // Pushes the hit children of a node, keys sorted ascending with the nh - 1 hits behind
-    // the nearest in slots 1..nh-1, so that slot 1 ends on top.  When they fit, every slot
-    // is written unconditionally (misses into row S), which keeps the node step free of
-    // per-child branches.
+    // Writes c[K .. W - 1] to the rows from p on, up to the last hit: rows a constant apart, one
+    // compare per child, and no further ones once no lane has any left.
+    template <int W, int K>
+    static __device__ __forceinline__ void store_children(uint2 *p, const Child (&c)[W], int nh)
+    {
+        if constexpr (K < W) {
+            if (K < nh) {
+                p[(K - 1) * kTraceBlock] = __builtin_bit_cast(uint2, c[K]);
+                store_children<W, K + 1>(p, c, nh);
+            }
+        }
+    }
+    // Pushes the hit children of a node, sorted ascending with the nh - 1 hits behind the nearest
+    // in slots 1..nh-1, so that slot 1 ends on top.
     template <int W>
-    __device__ __forceinline__ void push_children(const uint32_t (&key)[W], const uint32_t (&ref)[W], int nh)
+    __device__ __forceinline__ void push_children(const Child (&c)[W], int nh)
     {
         const uint32_t m = (uint32_t)nh - 1u;
-        if (sp + m <= S) {
-#pragma unroll
-            for (int k = 1; k < W; ++k) {
-                const uint32_t pos = k < nh ? sp + m - (uint32_t)k : S;
-                s[pos * kTraceBlock + tid] = make_uint2(ref[k], key[k] & ~7u);
-            }
-            sp += m;
+        if (m <= top) {
+            top -= m;
+            store_children<W, 1>(s + top * kTraceBlock, c, nh);
         } else {
 #pragma unroll
             for (int k = W - 1; k >= 1; --k) {
-                if (key[k] != kMissKey) push(ref[k], __uint_as_float(key[k] & ~7u));
+                if (k < nh) push(__builtin_bit_cast(uint2, c[k]));
             }
         }
     }
@@ -261,18 +290,18 @@ struct Stack {
     __device__ __forceinline__ uint32_t pop(float tmax)
     {
         for (;;) {
-            if (sp == 0) {
+            if (top == S) {
                 if (gsp == 0) return kEmpty;
                 gsp -= S;
                 for (uint32_t k = 0; k < S; k += 2) {
                     const uint4 v = g[(gsp + k) / 2];
-                    s[k * kTraceBlock + tid]       = make_uint2(v.x, v.y);
-                    s[(k + 1) * kTraceBlock + tid] = make_uint2(v.z, v.w);
+                    s[k * kTraceBlock]       = make_uint2(v.x, v.y);
+                    s[(k + 1) * kTraceBlock] = make_uint2(v.z, v.w);
                 }
-                sp = S;
+                top = 0;
             }
-            --sp;
-            const uint2 v = s[sp * kTraceBlock + tid];
+            const uint2 v = s[top * kTraceBlock];
+            ++top;
             if (__uint_as_float(v.y) <= tmax) return v.x;
         }
     }
@@ -610,14 +639,14 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
 {
     uint32_t c_nodes = 0, c_leaves = 0, c_tris = 0, c_wnode = 0, c_wleaf = 0;
     uint32_t c_noray = 0, c_empty = 0, c_leafwait = 0;   // idle lanes of node-loop iterations, by cause
-    __shared__ uint2 s_stack[(S + 1) * kTraceBlock];
+    __shared__ uint2 s_stack[S * kTraceBlock];
     const uint32_t n = q.count ? *q.count : q.n;
     if (n == 0) {
         if (q.done && blockIdx.x == 0 && threadIdx.x == 0) trace_clear(q, n);
         return;
     }
     if constexpr (W == 8 && !kInst && !kStats) {
-        constexpr uint32_t kDepth = (S + 1) * kTraceBlock / kGroupRays;
+        constexpr uint32_t kDepth = S * kTraceBlock / kGroupRays;
         if (n <= q.group_rays && q.spill_depth <= kDepth) {
             if (blockIdx.x * kGroupRays >= n) return;
             trace_groups<kAny, kMulti>(sc, q, occ, n, s_stack, kDepth);
@@ -635,12 +664,11 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
     if (!sup.dynamic && blockIdx.x / kXcds * kWaves * kStatic >= sup.slice_len(blockIdx.x % kXcds)) return;
 
     Stack<S> st;
-    st.s      = s_stack;
+    st.s      = s_stack + threadIdx.x;
     st.g      = reinterpret_cast<uint4 *>(spill) + (size_t)(blockIdx.x * blockDim.x + threadIdx.x) * (q.spill_depth / 2);
     st.depth  = q.spill_depth;
-    st.tid    = threadIdx.x;
-    st.sp = st.gsp = 0;
-    st.err = q.error;
+    st.err    = q.error;
+    st.clear();
 
     RayState r;
     const void   *nodes = sc.nodes;
@@ -671,7 +699,7 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
         level    = 1;
         cur_inst = inst;
         inst_hit = false;
-        st.push(kInstExit, -kInf);
+        st.push(make_uint2(kInstExit, __float_as_uint(-kInf)));
         return I.root;
     };
     auto exit_instance = [&]() {
@@ -710,7 +738,7 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
             const uint32_t rank = __popcll(idle & ((1ull << lane) - 1ull));
             if (!active && rank < got) {
                 rid = base + rank;
-                st.sp = st.gsp = 0;
+                st.clear();
                 pend      = kEmpty;
                 pend2     = kEmpty;
                 level     = 0;
@@ -756,15 +784,15 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
                 c_leafwait += active && cur != kEmpty && ref_is_leaf(cur);
             }
             if (inner) {
-                uint32_t key[W], ref[W];
-                const int nh = NodeOps<W>::expand(nodes, cur, r, key, ref);
+                Child c[W];
+                const int nh = NodeOps<W>::expand(nodes, cur, r, c);
                 if constexpr (kStats) ++c_nodes;
                 if (nh == 0) {
                     cur = next();
                 } else {
-                    sort_pairs<W>(key, ref);
-                    cur = ref[0];
-                    st.template push_children<W>(key, ref, nh);
+                    sort_children<W>(c);
+                    cur = child_ref(c[0]);
+                    st.template push_children<W>(c, nh);
                 }
             }
         }
@@ -779,7 +807,7 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
             if (kInst && leaf && level == 0) {
                 // instance leaf: enter the first instance, keep the rest for later
                 const uint32_t first = leaf_first(cur), cnt = leaf_count(cur);
-                if (cnt > 1) st.push(ref_leaf(first + 1, cnt - 1), -kInf);
+                if (cnt > 1) st.push(make_uint2(ref_leaf(first + 1, cnt - 1), __float_as_uint(-kInf)));
                 cur = enter_instance(sc.tlas_inst[first]);
             } else if (leaf) {
                 const uint32_t lf = parked ? pend : cur;
