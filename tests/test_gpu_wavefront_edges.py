@@ -41,3 +41,11 @@ def test_more_paths_than_shading_threads(oracle):
     got = _render(spec, w, h, 2, 1, 0)
     ref = oracle.render(spec, res=(w, h), spp=1, seed=11, trav=oracle.BRUTE32)["raw"]
     assert np.isclose(got, ref, rtol=1e-5, atol=1e-7).all(axis=2).mean() >= 0.999
+
+
+@pytest.mark.parametrize("spp", [7, 8])
+def test_lone_wavefront_in_halves(spp):
+    spec = scenes.sunlit(4, mode=1)
+    w, h = 1536, 1024   # 8 passes are 12,582,912 paths, the fewest that are split
+    got = _render(spec, w, h, 2, spp, 1)
+    assert np.array_equal(got, _render(spec, w, h, 2, spp, 1, wavefront_paths=w * h))   # a pass at a time
