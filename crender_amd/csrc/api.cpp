@@ -410,9 +410,8 @@ struct Arena {
 };
 
 // Path buffers of a batch: P path slots of queue, hit and path state.  uv: some scene has
-// texture coordinates, sun: some scene has its sun on, alpha: shadow rays pass transparent
-// texels (their continuations are staged behind the queue).
-void carve_batch_paths(Arena &A, PathBuffers &b, size_t P, bool uv, bool sun, bool alpha)
+// texture coordinates, sun: some scene has its sun on.
+void carve_batch_paths(Arena &A, PathBuffers &b, size_t P, bool uv, bool sun)
 {
     auto rays = [&](RaySoA &q, size_t n) {
         for (float **f : {&q.ox, &q.oy, &q.oz, &q.dx, &q.dy, &q.dz}) A.get(f, n);
@@ -429,11 +428,9 @@ void carve_batch_paths(Arena &A, PathBuffers &b, size_t P, bool uv, bool sun, bo
     }
     hits(b.hits, uv);
     if (sun) {
-        const size_t n = alpha ? 2 * P : P;
-        rays(b.sq, n);
-        A.get(&b.spath, n);
-        A.get(&b.scontrib, n);
-        if (alpha) hits(b.shits, true);
+        rays(b.sq, P);
+        A.get(&b.spath, P);
+        A.get(&b.scontrib, P);
     }
     A.get(&b.thr, P);
     A.get(&b.rad, P);
@@ -473,7 +470,7 @@ int alloc_path_set(crt_renderer *r, PathBuffers &b, bool image)
     if ((st = ralloc(r, ptr, n)) != CRT_OK) return st
     if ((st = alloc_rays(r, b.q[0], P))) return st;
     if ((st = alloc_rays(r, b.q[1], P))) return st;
-    if ((st = alloc_rays(r, b.sq, 2 * P))) return st;
+    if ((st = alloc_rays(r, b.sq, P))) return st;
     RA(&b.qpath[0], P);
     RA(&b.qpath[1], P);
     RA(&b.hits.t, P);
@@ -481,13 +478,8 @@ int alloc_path_set(crt_renderer *r, PathBuffers &b, bool image)
     RA(&b.hits.v, P);
     RA(&b.hits.tri, P);
     RA(&b.hits.inst, P);
-    RA(&b.shits.inst, P);
-    RA(&b.shits.t, P);
-    RA(&b.shits.u, P);
-    RA(&b.shits.v, P);
-    RA(&b.shits.tri, P);
-    RA(&b.spath, 2 * P);
-    RA(&b.scontrib, 2 * P);
+    RA(&b.spath, P);
+    RA(&b.scontrib, P);
     RA(&b.thr, P);
     RA(&b.rad, P);
     if (image) {
@@ -705,25 +697,16 @@ int run_paths(crt_renderer *r, const PathBuffers &b, const RenderParams &rp, hip
         if (tm) HIP_CHECK(mark(t.ev_shade[i]));
         if (tm) t.ev_shadow[i] = -1;
         if (sc.sun_enabled) {
+            TraceQueue qs = make_queue(b.sq, HitSoA{}, b.cnt + kCntShadow, b.cnt + kCntWorkShadow, b.cnt + kCntErr);
+            qs.done       = b.cnt + kCntDoneShadow;
+            qs.stat       = b.stats + 1;
+            resolve_into(qs, b);
             if (!sc.any_alpha) {
-                TraceQueue qs = make_queue(b.sq, HitSoA{}, b.cnt + kCntShadow, b.cnt + kCntWorkShadow, b.cnt + kCntErr);
-                qs.tstats     = b.tstats;
-                qs.done       = b.cnt + kCntDoneShadow;
-                qs.stat       = b.stats + 1;
-                resolve_into(qs, b);
+                qs.tstats = b.tstats;
                 HIP_CHECK(launch_trace_any(sc, qs, nullptr, spill, tc, s));
             } else {
-                // closest hit + alpha pass-through, renderer.cpp:330-345 (bounded at 64 steps)
-                HIP_CHECK(launch_shadow_prep(b, s));
-                for (int step = 0; step < 64; ++step) {
-                    TraceQueue qs = make_queue(b.sq, b.shits, b.cnt + kCntShadow, b.cnt + kCntWorkShadow, b.cnt + kCntErr);
-                    HIP_CHECK(launch_trace_closest(sc, qs, spill, tc, s));
-                    HIP_CHECK(launch_shadow_alpha_step(sc, b, s));
-                    uint32_t left = 0;
-                    HIP_CHECK(hipMemcpyAsync(&left, b.cnt + kCntShadow, sizeof left, hipMemcpyDeviceToHost, s));
-                    HIP_CHECK(hipStreamSynchronize(s));
-                    if (left == 0) break;
-                }
+                qs.alpha_stat = b.stats + 1;
+                HIP_CHECK(launch_trace_alpha(sc, qs, spill, tc, s));
             }
             if (tm) HIP_CHECK(mark(t.ev_shadow[i]));
         }
@@ -2962,27 +2945,17 @@ int record_trace(const PathBuffers &b, const BatchDev &bd, const TraceScene *tsc
         HIP_CHECK(launch_shade_multi(bd, b, i, cur, s));
         if (any_sun) {
             HIP_CHECK(launch_shadow_prep(b, s));
+            TraceQueue qs = make_queue(b.sq, HitSoA{}, b.cnt + kCntShadow, b.cnt + kCntWorkShadow, b.cnt + kCntErr);
+            qs.ray_path = b.spath;
+            qs.path_job = b.pjob;
+            qs.scenes   = tscenes;
+            resolve_into(qs, b);
             if (!any_alpha) {
-                TraceQueue qs = make_queue(b.sq, HitSoA{}, b.cnt + kCntShadow, b.cnt + kCntWorkShadow, b.cnt + kCntErr);
-                qs.ray_path = b.spath;
-                qs.path_job = b.pjob;
-                qs.scenes   = tscenes;
-                resolve_into(qs, b);
                 HIP_CHECK(launch_trace_any_multi(width, qs, nullptr, spill, tc, s));
             } else {
-                // alpha pass-through (renderer.cpp:330-345): host-driven, never captured
-                for (int step = 0; step < 64; ++step) {
-                    TraceQueue qs = make_queue(b.sq, b.shits, b.cnt + kCntShadow, b.cnt + kCntWorkShadow, b.cnt + kCntErr);
-                    qs.ray_path = b.spath;
-                    qs.path_job = b.pjob;
-                    qs.scenes   = tscenes;
-                    HIP_CHECK(launch_trace_closest_multi(width, qs, spill, tc, s));
-                    HIP_CHECK(launch_shadow_alpha_step_multi(bd, b, s));
-                    uint32_t left = 0;
-                    HIP_CHECK(hipMemcpyAsync(&left, b.cnt + kCntShadow, sizeof left, hipMemcpyDeviceToHost, s));
-                    HIP_CHECK(hipStreamSynchronize(s));
-                    if (left == 0) break;
-                }
+                qs.jobs       = bd.jobs;
+                qs.alpha_stat = b.stats + 1;
+                HIP_CHECK(launch_trace_alpha_multi(width, qs, spill, tc, s));
             }
         }
         cur ^= 1u;
@@ -3081,7 +3054,7 @@ int crt_render_batch(crt_context *ctx, const crt_job *jobs, uint32_t njobs, cons
     uint32_t   *d_cursor = nullptr;   // one per set: chunk k, then k + nsets, ...
     for (int pass = 0; pass < 2; ++pass) {   // sizes, then addresses
         arena = Arena{ws.base, 0};
-        for (uint32_t k = 0; k < nsets; ++k) carve_batch_paths(arena, b[k], P, any_uv, any_sun, any_alpha);
+        for (uint32_t k = 0; k < nsets; ++k) carve_batch_paths(arena, b[k], P, any_uv, any_sun);
         for (uint32_t j = 0; j < njobs; ++j) {
             if (jobs[j].memory == CRT_MEM_DEVICE) dev_out[j] = jobs[j].rgb_sum;
             else arena.get(&dev_out[j], (size_t)jobs[j].width * jobs[j].height * 3);

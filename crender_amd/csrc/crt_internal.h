@@ -180,6 +180,7 @@ constexpr uint32_t kXcds    = 8;
 constexpr uint32_t kCntLine = 32;   // words per 128-byte line
 constexpr uint32_t kSpillDepth = 256;   // most global spill entries per lane (multiple of 32)
 struct TraceScene;
+struct JobDev;
 struct TraceQueue {
     RaySoA          rays;
     HitSoA          hits;
@@ -198,7 +199,10 @@ struct TraceQueue {
     const uint32_t   *ray_path;
     const uint32_t   *path_job;
     const TraceScene *scenes;
-    // any-hit launches: where rad is set, an unoccluded ray i adds contrib[i] to rad[path[i]]
+    // alpha launches: the batch's jobs (whose materials decide), and the count of passes
+    const JobDev       *jobs;
+    unsigned long long *alpha_stat;
+    // any-hit and alpha launches: where rad is set, an unoccluded ray i adds contrib[i] to rad[path[i]]
     // (a path has at most one ray in the queue) instead of storing its occlusion byte
     const uint32_t *res_path;
     const float4   *res_contrib;
@@ -231,12 +235,16 @@ struct TraceConfig {
 };
 hipError_t launch_trace_closest(const SceneDev &sc, const TraceQueue &q, uint32_t *spill, const TraceConfig &tc,
                                 hipStream_t s);
+hipError_t launch_trace_alpha(const SceneDev &sc, const TraceQueue &q, uint32_t *spill, const TraceConfig &tc,
+                              hipStream_t s);
 hipError_t launch_trace_any(const SceneDev &sc, const TraceQueue &q, uint8_t *occ, uint32_t *spill,
                             const TraceConfig &tc, hipStream_t s);
 // batched: every ray carries its scene (q.ray_path / q.path_job / q.scenes); all scenes
 // share one BVH width
 hipError_t launch_trace_closest_multi(uint32_t width, const TraceQueue &q, uint32_t *spill, const TraceConfig &tc,
                                       hipStream_t s);
+hipError_t launch_trace_alpha_multi(uint32_t width, const TraceQueue &q, uint32_t *spill, const TraceConfig &tc,
+                                    hipStream_t s);
 hipError_t launch_trace_any_multi(uint32_t width, const TraceQueue &q, uint8_t *occ, uint32_t *spill,
                                   const TraceConfig &tc, hipStream_t s);
 // Ray-queue reordering (raysort.hip): keys, values and radix-sort temporary storage.
@@ -313,7 +321,6 @@ struct PathBuffers {
     RaySoA    sq;               // shadow queue
     uint32_t *spath;
     float4   *scontrib;         // radiance added if the shadow ray escapes
-    HitSoA    shits;            // closest hits of shadow rays (alpha pass-through)
     float4   *thr, *rad;
     float    *raw;              // W*H*3 running sum, flipped as renderer.cpp:358-365
     float4   *aov_alb, *aov_nrm, *aov_dep;
@@ -341,7 +348,7 @@ constexpr uint32_t kStatSlots = 64;
 // flight together use, lie kCntLine words (one 128-byte line) apart: atomics on one line from
 // the whole chip are served one after the other.
 enum : uint32_t {
-    kCntQ0 = 0, kCntQ1 = kCntQ0 + kCntLine, kCntShadow = 2 * kCntLine, kCntShadow2 = 3 * kCntLine,
+    kCntQ0 = 0, kCntQ1 = kCntQ0 + kCntLine, kCntShadow = 2 * kCntLine,
     kCntNrcQ = 4 * kCntLine, kCntTrain = 5 * kCntLine, kCntErr = 6 * kCntLine,
     kCntNrcBad = kCntErr + 1,   // a cache prediction of the wavefront was not finite: its accumulation is skipped
     kCntDoneExt = 7 * kCntLine, kCntDoneShadow = 8 * kCntLine,
@@ -414,7 +421,6 @@ hipError_t launch_shade(const SceneDev &sc, const PathBuffers &b, const RenderPa
 constexpr uint32_t kShadeClasses = 4;
 hipError_t launch_shade_sort(const SceneDev &sc, const PathBuffers &b, uint32_t cur, hipStream_t s);
 hipError_t launch_shadow_prep(const PathBuffers &b, hipStream_t s);
-hipError_t launch_shadow_alpha_step(const SceneDev &sc, const PathBuffers &b, hipStream_t s);
 hipError_t launch_accumulate(const PathBuffers &b, uint32_t nsamp, hipStream_t s);
 hipError_t launch_display(const float *raw, uint64_t n, uint32_t npix, float4 *out, hipStream_t s);
 hipError_t launch_fill(float4 *p, uint64_t n, float v, hipStream_t s);
@@ -425,7 +431,6 @@ hipError_t nrc_launch_infer_dev(const float *q, float *out, const uint32_t *n_de
                                 hipStream_t s);
 hipError_t launch_batch_generate(const BatchDev &bd, const PathBuffers &b, hipStream_t s);
 hipError_t launch_shade_multi(const BatchDev &bd, const PathBuffers &b, uint32_t bounce, uint32_t cur, hipStream_t s);
-hipError_t launch_shadow_alpha_step_multi(const BatchDev &bd, const PathBuffers &b, hipStream_t s);
 hipError_t launch_batch_accumulate(const BatchDev &bd, const PathBuffers &b, uint32_t max_acc, hipStream_t s);
 hipError_t launch_batch_advance(uint32_t *cursor, uint32_t step, hipStream_t s);
 // Intersection records (crt_records): every output pointer may be null except dist.

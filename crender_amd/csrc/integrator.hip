@@ -15,6 +15,7 @@
 #include <hip/hip_runtime.h>
 #include <float.h>
 #include "crt_internal.h"
+#include "material.h"
 
 namespace crt {
 
@@ -62,22 +63,6 @@ __device__ __forceinline__ void block_add_stat(unsigned long long *stats, uint32
     __syncthreads();
 }
 
-// image.h:104-109: nearest texel, static_cast<uint64_t>(u * width) % width.  The cast of a
-// negative product is undefined in C++; this follows what x86-64 code without AVX-512 does
-// (the signed truncation reinterpreted as uint64), so u * width in (-1, 0] maps to column 0
-// and -1.5 to (2^64 - 1) % width.  For power-of-two sizes that is the positive modulo.
-__device__ __forceinline__ uint64_t texel_index(float u, uint32_t size)
-{
-    return (uint64_t)(int64_t)(u * (float)size) % (uint64_t)size;
-}
-
-__device__ __forceinline__ float4 tex_uv(const SceneDev &sc, int32_t t, float u, float v)
-{
-    const TextureDev td = sc.texs[t];
-    const uint64_t   x = texel_index(u, td.w), y = texel_index(v, td.h);
-    return sc.texels[td.offset + x + y * (uint64_t)td.w];
-}
-
 // renderer.cpp:277-289, scene.cpp:67-77
 __device__ __forceinline__ f3 sky(const SceneDev &sc, f3 d)
 {
@@ -92,12 +77,6 @@ __device__ __forceinline__ f3 sky(const SceneDev &sc, f3 d)
     const float v  = 0.5f - asin_cr(dy) * kInvPi;
     const float4 c = tex_uv(sc, sc.sky_tex, u + sc.sky_rot[0], v + sc.sky_rot[1]);
     return mk3(c.x, c.y, c.z);
-}
-
-__device__ __forceinline__ float4 mat_colour(const SceneDev &sc, const MaterialDev &m, float u, float v)
-{
-    if (m.tex >= 0 && (uint32_t)m.tex < sc.ntex) return tex_uv(sc, m.tex, u, v);
-    return make_float4(m.colour[0], m.colour[1], m.colour[2], m.colour[3]);
 }
 
 // sampling.h:53-57
@@ -202,10 +181,7 @@ __global__ void k_shadow_prep(PathBuffers b)
 {
     const uint32_t t = threadIdx.x;
     if (t < 8) b.cnt[kCntWorkShadow + t * kCntLine] = 0;
-    if (t == 0) {
-        b.cnt[kCntShadow2] = 0;
-        atomicAdd(&b.stats[1], (unsigned long long)b.cnt[kCntShadow]);
-    }
+    if (t == 0) atomicAdd(&b.stats[1], (unsigned long long)b.cnt[kCntShadow]);
 }
 
 struct HitRec {
@@ -652,88 +628,6 @@ __global__ __launch_bounds__(256, 5) void k_shade(ShadeArgs args)
     if (blockIdx.x * blockDim.x < n) block_add_stat(kp->b.stats, 2, seg);
 }
 
-// True if the shadow ray k stopped on a transparent texel (colour.w == 0); o2 = where it continues.
-__device__ __forceinline__ bool alpha_passes(const SceneDev &sc, const PathBuffers &b, uint32_t k, f3 o, f3 d,
-                                             uint32_t tri, f3 &o2)
-{
-    const HitRec       h   = hit_record(sc, o, d, b.shits.t[k], tri, b.shits.u[k], b.shits.v[k]);
-    const MaterialDev &m   = sc.mats[sc.mat_idx[h.prim]];
-    const float4       col = mat_colour(sc, m, h.u, h.v);
-    o2 = h.point + d * 0.1f;
-    return col.w == 0.0f;
-}
-
-// Alpha-aware shadow step (renderer.cpp:330-345): after a closest-hit trace of the shadow
-// queue, escaped rays add their contribution, rays stopped by an alpha surface continue
-// from hit + 0.1*dir (compacted into the front of the same queue), others are blocked.
-template <bool kMulti>
-__global__ __launch_bounds__(256) void k_shadow_alpha(SceneDev sc_one, PathBuffers b, const JobDev *jobs)
-{
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    const uint32_t n = b.cnt[kCntShadow];
-    bool     cont = false;
-    f3       o2 = mk3(0, 0, 0), d = mk3(0, 0, 0);
-    uint32_t p = 0;
-    float4   c = make_float4(0, 0, 0, 0);
-    if (k < n) {
-        p = b.spath[k];
-        c = b.scontrib[k];
-        const uint32_t tri = b.shits.tri[k];
-        const f3 o = mk3(b.sq.ox[k], b.sq.oy[k], b.sq.oz[k]);
-        d = mk3(b.sq.dx[k], b.sq.dy[k], b.sq.dz[k]);
-        if (tri == kInvalidRef) {
-            float4 r = b.rad[p];
-            r.x += c.x;
-            r.y += c.y;
-            r.z += c.z;
-            b.rad[p] = r;
-        } else {
-            if constexpr (kMulti) cont = alpha_passes(jobs[b.pjob[p]].sc, b, k, o, d, tri, o2);
-            else cont = alpha_passes(sc_one, b, k, o, d, tri, o2);
-        }
-    }
-    // continuation rays go to a staging count, then the host swaps them in
-    const uint32_t slot = block_append(&b.cnt[kCntShadow2], cont);
-    if (cont) {
-        // staged after the live entries; k_shadow_compact moves them to the front
-        const uint32_t dst = n + slot;
-        if (dst < b.P * 2u) {
-            put_ray(b.sq, dst, o2, d);
-            b.spath[dst]    = p;
-            b.scontrib[dst] = c;
-        }
-    }
-}
-
-__global__ __launch_bounds__(256) void k_shadow_compact(PathBuffers b)
-{
-    const uint32_t n = b.cnt[kCntShadow];
-    const uint32_t m = b.cnt[kCntShadow2];
-    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k < m) {
-        const uint32_t s = n + k;
-        const RaySoA  &q = b.sq;
-        const float ox = q.ox[s], oy = q.oy[s], oz = q.oz[s], dx = q.dx[s], dy = q.dy[s], dz = q.dz[s];
-        const uint32_t pp = b.spath[s];
-        const float4   cc = b.scontrib[s];
-        // source indices >= n and destinations < m <= n never overlap
-        q.ox[k] = ox; q.oy[k] = oy; q.oz[k] = oz; q.dx[k] = dx; q.dy[k] = dy; q.dz[k] = dz;
-        b.spath[k]    = pp;
-        b.scontrib[k] = cc;
-    }
-}
-
-__global__ void k_shadow_swap(PathBuffers b)
-{
-    if (threadIdx.x == 0) {
-        const uint32_t m = b.cnt[kCntShadow2];
-        b.cnt[kCntShadow]  = m;
-        b.cnt[kCntShadow2] = 0;
-        atomicAdd(&b.stats[1], (unsigned long long)m);
-    }
-    if (threadIdx.x < 8) b.cnt[kCntWorkShadow + threadIdx.x * kCntLine] = 0;
-}
-
 // raw[pixel] += the radiance of each of the wavefront's samples of the pixel, in sample
 // order: the same sums as one accumulation per pass.  A pixel's nsamp slots lie side by side,
 // so the block reads its 256 pixels' slots in order (a wave 1 KB at a time) and passes them
@@ -1045,13 +939,6 @@ hipError_t launch_shadow_prep(const PathBuffers &b, hipStream_t s)
     k_shadow_prep<<<1, 64, 0, s>>>(b);
     return hipGetLastError();
 }
-hipError_t launch_shadow_alpha_step(const SceneDev &sc, const PathBuffers &b, hipStream_t s)
-{
-    k_shadow_alpha<false><<<blocks(b.P), 256, 0, s>>>(sc, b, nullptr);
-    k_shadow_compact<<<blocks(b.P), 256, 0, s>>>(b);
-    k_shadow_swap<<<1, 64, 0, s>>>(b);
-    return hipGetLastError();
-}
 hipError_t launch_accumulate(const PathBuffers &b, uint32_t nsamp, hipStream_t s)
 {
     k_accumulate<<<blocks(b.npix), 256, 0, s>>>(b, nsamp);
@@ -1119,13 +1006,6 @@ hipError_t launch_shade_multi(const BatchDev &bd, const PathBuffers &b, uint32_t
     return hipGetLastError();
 }
 
-hipError_t launch_shadow_alpha_step_multi(const BatchDev &bd, const PathBuffers &b, hipStream_t s)
-{
-    k_shadow_alpha<true><<<blocks(b.P), 256, 0, s>>>(SceneDev{}, b, bd.jobs);
-    k_shadow_compact<<<blocks(b.P), 256, 0, s>>>(b);
-    k_shadow_swap<<<1, 64, 0, s>>>(b);
-    return hipGetLastError();
-}
 
 hipError_t launch_batch_accumulate(const BatchDev &bd, const PathBuffers &b, uint32_t max_acc, hipStream_t s)
 {

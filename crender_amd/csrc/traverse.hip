@@ -24,6 +24,7 @@
 //     "speculative traversal").
 #include <hip/hip_runtime.h>
 #include "crt_internal.h"
+#include "material.h"
 
 namespace crt {
 
@@ -522,6 +523,32 @@ __device__ __forceinline__ bool load_ray(const TraceQueue &q, uint32_t rid, uint
            (r.d.x != 0.0f || r.d.y != 0.0f || r.d.z != 0.0f);
 }
 
+// Shadow rays of scenes with transparent texels (renderer.cpp:330-345): a ray that stops on one
+// (colour.w == 0) goes on from the hit + 0.1 * direction, up to kAlphaSteps traces, and adds its
+// contribution if it escapes.  The lane restarts the ray itself, in the same launch: with a
+// launch per step, its material test, compaction and counters as kernels of their own and the host
+// reading the count between the steps, 640x360 with cut-outs took 950 us where it now takes 511.
+constexpr uint32_t kAlphaSteps = 64;
+
+// True if ray rid, stopped at r's hit, passes; o2 = where it goes on.
+template <bool kMulti>
+__device__ __forceinline__ bool alpha_passes(const SceneDev &sc_one, const TraceQueue &q, uint32_t rid,
+                                             const RayState &r, f3 &o2)
+{
+#pragma clang fp contract(off)
+    const SceneDev &sc = kMulti ? q.jobs[q.path_job[q.ray_path[rid]]].sc : sc_one;
+    float u = 0.0f, v = 0.0f;
+    if (sc.uv) {
+        const float2 w0 = sc.uv[3 * (size_t)r.best_prim + 0], w1 = sc.uv[3 * (size_t)r.best_prim + 1],
+                     w2 = sc.uv[3 * (size_t)r.best_prim + 2];
+        const float b0 = 1.0f - r.bu - r.bv;
+        u = b0 * w0.x + r.bu * w1.x + r.bv * w2.x;
+        v = b0 * w0.y + r.bu * w1.y + r.bv * w2.y;
+    }
+    o2 = r.o + r.d * r.tmax + mk3(q.rays.dx[rid], q.rays.dy[rid], q.rays.dz[rid]) * 0.1f;
+    return mat_colour(sc, sc.mats[sc.mat_idx[r.best_prim]], u, v).w == 0.0f;
+}
+
 // The launch's n rays with a group per ray; lds: `depth` entries for each of the block's groups.
 template <bool kAny, bool kMulti>
 __device__ __forceinline__ void trace_groups(const SceneDev &sc, const TraceQueue &q, uint8_t *occ, uint32_t n,
@@ -633,7 +660,7 @@ __device__ __forceinline__ void trace_groups(const SceneDev &sc, const TraceQueu
     }
 }
 
-template <int W, bool kAny, bool kMulti, uint32_t S, bool kInst, bool kStats = false>
+template <int W, bool kAny, bool kMulti, uint32_t S, bool kInst, bool kStats = false, bool kAlpha = false>
 __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev sc, TraceQueue q, uint8_t *occ,
                                                                       uint32_t *spill)
 {
@@ -645,7 +672,7 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
         if (q.done && blockIdx.x == 0 && threadIdx.x == 0) trace_clear(q, n);
         return;
     }
-    if constexpr (W == 8 && !kInst && !kStats) {
+    if constexpr (W == 8 && !kInst && !kStats && !kAlpha) {
         constexpr uint32_t kDepth = S * kTraceBlock / kGroupRays;
         if (n <= q.group_rays && q.spill_depth <= kDepth) {
             if (blockIdx.x * kGroupRays >= n) return;
@@ -674,6 +701,7 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
     const void   *nodes = sc.nodes;
     const float4 *tris  = sc.tri;
     uint32_t rid = 0, cur = kEmpty;
+    uint32_t aroot = sc.root, steps = 0, passed = 0;   // kAlpha: the ray's root, traces of it, passes of the lane
     // instance state (kInst): world ray while inside an instance, scale, instance ids
     f3       wo = mk3(0, 0, 0), wd = mk3(0, 0, 0);
     float    wtmax = 0.0f, ilen = 1.0f;
@@ -754,6 +782,10 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
                 const bool valid = load_ray(q, rid, ntri, r);
                 cur    = valid ? root : kEmpty;
                 active = true;
+                if constexpr (kAlpha) {
+                    aroot = root;
+                    steps = 1;
+                }
             }
             idle  = __ballot(!active);
             nidle = __popcll(idle);
@@ -853,8 +885,22 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
                 }
             }
         }
+        if constexpr (kAlpha) {
+            f3 o2;
+            if (active && cur == kEmpty && r.best_tri != kInvalidRef && alpha_passes<kMulti>(sc, q, rid, r, o2)) {
+                ++passed;
+                if (steps < kAlphaSteps) {
+                    ++steps;
+                    r.o    = o2;
+                    r.tmax = kInf;
+                    r.best_tri = r.best_prim = kInvalidRef;
+                    st.clear();
+                    cur = aroot;
+                }
+            }
+        }
         if (active && cur == kEmpty) {
-            store_ray<kAny>(q, occ, rid, r);
+            store_ray<kAny || kAlpha>(q, occ, rid, r);
             if (kInst && !kAny && q.hits.inst) q.hits.inst[rid] = r.best_tri != kInvalidRef ? best_inst : kInvalidRef;
             active = false;
         }
@@ -880,6 +926,10 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
             atomicAdd(q.tstats + 7, f);
         }
     }
+    if constexpr (kAlpha) {
+        for (int o = 32; o > 0; o >>= 1) passed += __shfl_xor(passed, o);
+        if (lane == 0 && passed != 0u) atomicAdd(q.alpha_stat, (unsigned long long)passed);
+    }
     trace_epilogue(q, n, sup.active_blocks(gridDim.x, kWaves));
 }
 
@@ -904,7 +954,7 @@ uint64_t trace_spill_bytes(uint32_t grid, uint32_t spill_depth)
 namespace {
 
 // Instantiates k_trace for the BVH width and LDS stack depth of the launch.
-template <bool kAny, bool kMulti, bool kInst>
+template <bool kAny, bool kMulti, bool kInst, bool kAlpha = false>
 hipError_t dispatch_trace(uint32_t width, const TraceConfig &tc, const SceneDev &sc, const TraceQueue &qin, uint8_t *occ,
                           uint32_t *spill, hipStream_t s)
 {
@@ -915,13 +965,13 @@ hipError_t dispatch_trace(uint32_t width, const TraceConfig &tc, const SceneDev 
     q.spill_depth  = tc.spill_depth;
     q.group_rays   = tc.group_rays;
     q.leaf_rounds  = tc.leaf_rounds ? (tc.leaf_rounds > 64u ? 0u : tc.leaf_rounds) : kLeafRounds;
-    if (!kMulti && q.tstats) {
+    if (!kMulti && !kAlpha && q.tstats) {
         // instrumented traversal: one stack depth (the counts do not depend on it)
         if (width == 4) k_trace<4, kAny, false, 32, kInst, true><<<g, b, 0, s>>>(sc, q, occ, spill);
         else k_trace<8, kAny, false, 32, kInst, true><<<g, b, 0, s>>>(sc, q, occ, spill);
         return hipGetLastError();
     }
-#define CRT_TRACE(Wd, Sd) k_trace<Wd, kAny, kMulti, Sd, kInst><<<g, b, 0, s>>>(sc, q, occ, spill)
+#define CRT_TRACE(Wd, Sd) k_trace<Wd, kAny, kMulti, Sd, kInst, false, kAlpha><<<g, b, 0, s>>>(sc, q, occ, spill)
     if (width == 4) {
         if (tc.stack == 8) CRT_TRACE(4, 8);
         else if (tc.stack == 32) CRT_TRACE(4, 32);
@@ -951,12 +1001,27 @@ hipError_t launch_trace_any(const SceneDev &sc, const TraceQueue &q, uint8_t *oc
     return dispatch_trace<true, false, false>(sc.width, tc, sc, q, occ, spill, s);
 }
 
+hipError_t launch_trace_alpha(const SceneDev &sc, const TraceQueue &q, uint32_t *spill, const TraceConfig &tc,
+                              hipStream_t s)
+{
+    if (sc.instanced) return dispatch_trace<false, false, true, true>(sc.width, tc, sc, q, nullptr, spill, s);
+    return dispatch_trace<false, false, false, true>(sc.width, tc, sc, q, nullptr, spill, s);
+}
+
 hipError_t launch_trace_closest_multi(uint32_t width, const TraceQueue &q, uint32_t *spill, const TraceConfig &tc,
                                       hipStream_t s)
 {
     SceneDev none{};
     none.ntri = 1;   // per-ray scenes decide
     return dispatch_trace<false, true, false>(width, tc, none, q, nullptr, spill, s);
+}
+
+hipError_t launch_trace_alpha_multi(uint32_t width, const TraceQueue &q, uint32_t *spill, const TraceConfig &tc,
+                                    hipStream_t s)
+{
+    SceneDev none{};
+    none.ntri = 1;
+    return dispatch_trace<false, true, false, true>(width, tc, none, q, nullptr, spill, s);
 }
 
 hipError_t launch_trace_any_multi(uint32_t width, const TraceQueue &q, uint8_t *occ, uint32_t *spill,
