@@ -124,10 +124,11 @@ def cpu_baseline(spec, res, bounces, seconds_target: float) -> dict:
 # Sources that decide what the closest-hit traversal reads and writes: HBM traffic measured
 # with profiler counters holds only for the build they were measured on.
 TRAVERSAL_SOURCES = ("crender_amd/csrc/traverse.hip", "crender_amd/csrc/crt_math.h", "crender_amd/csrc/crt_internal.h",
-                     "crender_amd/csrc/bvh_build.hip", "crender_amd/csrc/integrator.hip")
+                     "crender_amd/csrc/material.h", "crender_amd/csrc/bvh_build.hip",
+                     "crender_amd/csrc/integrator.hip")
 PMC_FILE = ROOT / "profiles" / "trace_closest_soup1m_1080p_pmc.json"
 # the closest-hit traversal the headline workload launches (default width, stack, no instances)
-TRACE_KERNEL = "k_trace<8, false, false, 16u, false, false>"
+TRACE_KERNEL = "k_trace<8, false, false, 16u, false, false, false>"
 
 
 def traversal_source_hash() -> str:

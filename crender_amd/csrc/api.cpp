@@ -234,10 +234,11 @@ namespace {
 
 // Launches of at most this many rays trace with eight lanes per ray (TraceQueue::group_rays).
 // A query alone on the GPU, us a call, a ray per lane against eight lanes per ray: diffuse rays
-// in 100k triangles, 4096: 246 / 120, 65,536: 264 / 207, 131,072: 284 / 307; camera rays in 1M
-// triangles, 65,536: 241 / 139, 131,072: 249 / 196.  A wavefront shares the GPU with another
-// one, where the work counts as well as the chain: within 1 % from 8192 to 98,304.
-constexpr uint32_t kGroupRaysQuery = 98304, kGroupRaysRender = 32768;
+// in 100k triangles, 4096: 222 / 122, 65,536: 239 / 208, 81,920: 247 / 258, 98,304: 242 / 302;
+// in 1M triangles, 65,536: 277 / 261, 81,920: 302 / 334; camera rays in 1M triangles, 65,536:
+// 213 / 178, 98,304: 224 / 219.  A wavefront shares the GPU with another one, where the work
+// counts as well as the chain: within 1 % from 8192 to 98,304.
+constexpr uint32_t kGroupRaysQuery = 65536, kGroupRaysRender = 32768;
 
 TraceConfig trace_cfg(const crt_context *ctx)
 {
@@ -652,15 +653,10 @@ int run_paths(crt_renderer *r, const PathBuffers &b, const RenderParams &rp, hip
     }
     const uint32_t timed = t.timing ? std::min<uint32_t>(nb, crt_renderer::kTimedBounces) : 0u;
     const bool sort = (ctx->opt.flags & CRT_FLAG_SORT_RAYS) && r->sort.keys;
-    // While the cache trains beside the traversal, the traversal leaves room in a CU's LDS for
-    // a training block (31.7 KB): a stack of at most 16 entries and, at the default grid, three
-    // blocks (3 x 34.8 KB) instead of four.
+    // While the cache trains beside the traversal, its training blocks (41 KB of LDS) must find
+    // room between the traversal's: a stack of at most 16 entries (32 KB per block).
     TraceConfig tc = trace_cfg(ctx);
-    if (rp.nrc.enabled && r->nopt.train) {
-        tc.stack = std::min<uint32_t>(tc.stack, 16u);
-        if (ctx->opt.trace_waves_per_cu == 0)
-            tc.grid = tc.grid / (kXcds * kTraceBlocksPerCu) * kXcds * kTraceBlocksPerCuTraining;
-    }
+    if (rp.nrc.enabled && r->nopt.train) tc.stack = std::min<uint32_t>(tc.stack, 16u);
     for (uint32_t i = 0; i < nb; ++i) {
         const bool tm = i < timed;
         if (sort && i > 0) {

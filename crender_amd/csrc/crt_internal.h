@@ -274,18 +274,16 @@ hipError_t launch_atrous(const float4 *colour, const float4 *normal, const float
 uint32_t trace_grid(int device, uint32_t blocks_per_cu);
 uint64_t trace_spill_bytes(uint32_t grid, uint32_t spill_depth);
 constexpr uint32_t kTraceBlock = 256;
-// default LDS stack entries per lane: 16 entries (34.8 KB per 256-lane block) let a CU hold
-// four blocks (139 of 160 KB), where 32 entries (67.6 KB per block) admit two
+// default LDS stack entries per lane: 16 entries (32 KB per 256-lane block) let a CU hold
+// four blocks (128 of 160 KB), where 32 entries (64 KB per block) admit two
 constexpr uint32_t kStackLds   = 16;
-// Default traversal blocks per CU: as many as fit with the default stack.  One launch then
-// fills the chip by itself, and a second wavefront's blocks start as the first one's end.
-// Two blocks (16 resident with both launches in flight) against four, 1080p: soup 8 passes
-// 16.4 -> 11.4 ms, 20 passes 28.1 -> 26.5, terrain 8 passes 16.1 -> 12.5, 2.07M camera rays
-// 0.83 -> 0.66 ms; three 13.0 / 27.8 / 13.6 / 0.70, eight (they queue) 12.2 / 29.0 / 13.1 / 0.79.
+// Default traversal blocks per CU.  One launch then fills the chip by itself, and a second
+// wavefront's blocks start as the first one's end.  1080p, soup 8 passes / 20 passes / terrain 8
+// passes / 2.07M camera rays, ms: three 11.02 / 22.95 / 11.14 / 0.62, four 9.78 / 21.87 / 10.16 /
+// 0.60, five (as many as fit) 10.13 / 22.52 / 10.64 / 0.64: more waves share each CU's cache.
 constexpr uint32_t kTraceBlocksPerCu = 4;
-// ... and while the radiance cache trains beside the traversal, so that a training block
-// (31.7 KB) still fits next to the traversal's (3 x 34.8 KB)
-constexpr uint32_t kTraceBlocksPerCuTraining = 3;
+// The same where a radiance cache trains beside it: a training block (41 KB) fits in as soon as
+// one of the four ends, and a grid of three per CU took 22.0 ms for 16 passes against 21.1.
 
 // ---- allocation-free queries (noalloc.hip) ---------------------------------------------
 // Layout of the per-device scratch array (byte offsets): counters (query_cnt words), leaf-order triangle and instance indices, u and v for callers that

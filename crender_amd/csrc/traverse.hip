@@ -34,7 +34,7 @@ constexpr float kInf = __builtin_huge_valf();
 constexpr uint32_t kEmpty = kInvalidRef;
 constexpr uint32_t kMissKey = 0x7FE00000u;   // behind every distance
 // default idle lanes that trigger a refill.  1080p soup 20 passes / terrain 8 passes with rays
-// from the wave's own chunk: 8 -> 26.4 / 12.5 ms, 16 -> 26.5 / 12.5, 24 -> 26.7 / 12.5, 32 -> 26.9 / 12.5
+// from the wave's own chunk: 8 -> 22.1 / 10.2 ms, 16 -> 21.9-22.1 / 10.2 (24 and 32 1 to 2 % more)
 constexpr uint32_t kRefillIdle = 16;
 // default: a wave leaves the inner-node phase for its parked leaves once fewer than 16 lanes
 // can still park one.  Measured on the 1M soup / 14.8M terrain at 1080p with two wavefronts in
@@ -316,7 +316,7 @@ __device__ __forceinline__ uint32_t lane_id() { return __lane_id(); }
 // one transforms the lane's ray into the instance's object space (direction renormalised,
 // distances scaled by |inv * d|, model.cpp:107-113) and pushes kInstExit, whose pop
 // restores the world ray; closest-hit distances are compared in world units.
-// The 8-entry stack variant is also the high-occupancy one: its 18 KB of LDS per block
+// The 8-entry stack variant is also the high-occupancy one: its 16 KB of LDS per block
 // leaves room for 8 waves per SIMD, so the register budget is capped to match (64 VGPRs).
 // kStats: the instrumented variant; counts each lane's inner-node tests, leaf visits and
 // triangle tests, each wave's iterations of the node and leaf loops, and the lanes idle in

@@ -1,5 +1,5 @@
 """Small batches, traced with eight lanes per ray, against the same rays as part of a batch large
-enough for a ray per lane (more than 98,304 rays): every field is equal.  Scenes with leaves of
+enough for a ray per lane (more than 65,536 rays): every field is equal.  Scenes with leaves of
 up to 16 triangles, coincident triangles (ties go to the smaller primID) and deep trees; rays
 with limits that cut hits off, degenerate and non-finite rays."""
 import numpy as np

@@ -4,7 +4,7 @@ The queue is cut into 8 slices; a wave owns 64 rays of its slice by position and
 a slice is handed out in chunks.  The counts cover slices that are empty, not full or one ray
 long, blocks without rays, exactly the rays owned by position, one ray more or less (one chunk
 of one ray per slice, slices of unequal length), and several chunks per wave, for the grid of
-crt_intersect (256 CUs x 4 blocks x 4 waves x 64 = 262,144 rays owned; it traces up to 98,304
+crt_intersect (256 CUs x 4 blocks x 4 waves x 64 = 262,144 rays owned; it traces up to 65,536
 rays with eight lanes per ray instead) and that of crt_intersect_noalloc (64 blocks, 16,384
 rays owned, a ray per lane at every count).  Every ray's hit equals the FP32 oracle's, bit for bit.
 """
@@ -38,7 +38,7 @@ def _rays(n):
     return o, d
 
 
-@pytest.mark.parametrize("n", [1, 7, 8, 9, 63, 64, 65, 511, 513, 98_304, 98_305, OWNED - 1, OWNED, OWNED + 1,
+@pytest.mark.parametrize("n", [1, 7, 8, 9, 63, 64, 65, 511, 513, 65_536, 65_537, 98_304, 98_305, OWNED - 1, OWNED, OWNED + 1,
                                OWNED + 9, 2 * OWNED + 5])
 def test_every_ray_is_traced_once(oracle, n):
     spec = scenes.cornell(1)
