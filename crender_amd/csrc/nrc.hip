@@ -12,15 +12,14 @@
 //   A: lane supplies row r, eight reduction elements j = 0 .. 7 of its group g
 //   B: lane supplies column r, the same reduction elements
 //   D: lane holds rows 4g .. 4g + 3 of column r
-// A and B name their reduction elements alike, so any assignment of the 32 elements to
-// (g, j) gives the same sums.  Every product is formed transposed: A = weights (rows =
-// output features), B = activations (columns = samples).  The result then has a sample per
-// lane and four consecutive features in its registers, and two result tiles together are,
-// converted to bf16, the B operand of the next layer with reduction element (g, j) =
-// feature 32 c + 16 (j / 4) + 4 g + j % 4.  Activations never leave the registers; the
-// weights are stored in that order instead, so a fragment is one 16-byte load per lane.
-// The 96 input features are assigned to (g, j) so that every lane group computes nine sin/cos
-// pairs and up to six other inputs (kmap0).
+// Reduction element (g, j) of 32-deep chunk c is feature 32 c + 8 g + j in every product.  (Another
+// assignment would give sums that differ in their FP32 roundings and, through the rounding to
+// bf16, predictions that differ by 2e-4.)  Every product is formed transposed: A = weights
+// (rows = output features), B = activations (columns = samples), and row 4 g + i of row tile
+// 2 c + h is output feature 32 c + 8 g + 4 h + i (feature_of).  The result then has a sample per
+// lane, and two result tiles together are, converted to bf16, the B operand of chunk c of the
+// next layer.  Activations never leave the registers; the weights are stored in that order
+// instead, so a fragment is one 16-byte load per lane.
 //
 // A product with the identity turns a tile with a sample per lane into one with a feature per
 // lane (exact: one term per sum), the operand form of dW = X^T G.
@@ -69,92 +68,94 @@ __host__ __device__ constexpr int fwd_frag(int l) { return l == 0 ? 0 : 12 + 8 *
 // first backward fragment of layer l >= 1: 4 x 8 + 4 = 36
 __host__ __device__ constexpr int bwd_frag(int l) { return 8 * (l - 1); }
 
-// input row (0 .. 95) of reduction element (chunk, g, j) of the first layer
-__device__ __forceinline__ int kmap0(int chunk, int g, int j)
-{
-    const int s = 8 * chunk + j;   // the lane group's feature 0 .. 23
-    if (s < 18) return 18 * g + s;                          // sin / cos pairs 9 g .. 9 g + 8
-    if (s < 21) return g < 3 ? 72 + 3 * g + (s - 18) : 81 + (s - 18);   // direction, normal, albedo | roughness, 1, 0
-    return 84 + 3 * g + (s - 21);                           // zero padding
-}
+// feature of row (or column) r of the 16-wide tile t of a layer's outputs
+__device__ __forceinline__ int feature_of(int t, int r) { return 32 * (t >> 1) + 8 * (r >> 2) + 4 * (t & 1) + (r & 3); }
+// and back: feature f is row tile_row(f) of tile tile_of(f)
+__device__ __forceinline__ int tile_of(int f) { return 2 * (f >> 5) + ((f >> 2) & 1); }
+__device__ __forceinline__ int tile_row(int f) { return 4 * ((f >> 3) & 3) + (f & 3); }
+// element of a fragment: row r, reduction feature k
+__device__ __forceinline__ int frag_elem(int r, int k) { return (((k >> 3) & 3) * 16 + r) * 8 + (k & 7); }
 
 // position of weight (k, c) of layer l among the forward fragments
 __device__ __forceinline__ int fwd_pos(int l, int k, int c)
 {
-    int kc, g, j;
-    if (l > 0) {
-        kc = k >> 5;
-        g  = (k >> 2) & 3;
-        j  = ((k >> 4) & 1) * 4 + (k & 3);
-    } else {
-        int s;
-        if (k < 72) {
-            g = k / 18;
-            s = k - 18 * g;
-        } else if (k < 84) {
-            g = (k - 72) / 3;
-            s = 18 + (k - 72) % 3;
-        } else {
-            g = (k - 84) / 3;
-            s = 21 + (k - 84) % 3;
-        }
-        kc = s >> 3;
-        j  = s & 7;
-    }
-    const int nk = layer_k(l) / 32;
-    return (fwd_frag(l) + (c >> 4) * nk + kc) * kFrag + (g * 16 + (c & 15)) * 8 + j;
+    return (fwd_frag(l) + tile_of(c) * (layer_k(l) / 32) + (k >> 5)) * kFrag + frag_elem(tile_row(c), k);
 }
 
 // position of weight (k, c) of layer l >= 1 among the backward fragments (rows = input
 // features, reduction over the output features)
 __device__ __forceinline__ int bwd_pos(int l, int k, int c)
 {
-    const int nc = layer_n(l) / 32, g = (c >> 2) & 3, j = ((c >> 4) & 1) * 4 + (c & 3);
-    return (bwd_frag(l) + (k >> 4) * nc + (c >> 5)) * kFrag + (g * 16 + (k & 15)) * 8 + j;
+    return (bwd_frag(l) + tile_of(k) * (layer_n(l) / 32) + (c >> 5)) * kFrag + frag_elem(tile_row(k), c);
+}
+
+// two features in one register
+__device__ __forceinline__ uint32_t pack2(float lo, float hi)
+{
+    typedef bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(uint32_t, bf16x2{to_bf16(lo), to_bf16(hi)});
+}
+
+// sin and cos of x times the FP32 number 2^freq pi.  sincosf on that product: the features are FP32
+// sines and cosines before they become bf16 ones, for any x (the hardware's v_sin and v_cos take
+// revolutions, and one known to 2^-25 leaves few correct bits near a zero crossing and none
+// far outside the unit box).  kNear: the product is below 2^17 in magnitude, where sincosf needs
+// no table for its reduction; told so, the compiler leaves that part out, 100 of 150 instructions.
+template <bool kNear>
+__device__ __forceinline__ uint32_t sincos_pair(float x, int freq)
+{
+    const float a = x * __uint_as_float(0x40490FDBu + ((uint32_t)freq << 23));
+    if (kNear) __builtin_assume(__builtin_fabsf(a) < 131072.0f);
+    float s, c;
+    sincosf(a, &s, &c);
+    return pack2(s, c);
 }
 
 // The lane's 24 input features of its sample (three B operands).  q: the sample's query (any
-// query of the batch for the lanes beyond it, whose results are not used).  Pair p = 9 g + m is sin and cos of a 2^f with a the
-// FP32 product of pi and x_c, c = p / 12, f = p % 12.  a / 2 pi is formed once per component
-// as a sum of two floats; scaling both by 2^f and taking the fraction of the first are exact,
-// so the hardware sine and cosine (which take revolutions) see an argument within 2^-25 of a
-// revolution, with no reduction of the argument per feature.
+// query of the batch for the lanes beyond it, whose results are not used).  Features 2 p and
+// 2 p + 1 are the pair of component p / 12 and frequency p % 12: pairs 16 c + 4 g .. in chunks
+// c = 0 and 1, whose four belong to one component; the pairs 32 .. 35 of chunk 2 are all lane
+// group 0's, so every group computes one of them and group 0 gathers them.
 __device__ __forceinline__ void encode(const float *q, int g, bf16x8 (&f)[3])
 {
-    const int   c0 = 9 * g / 12, c1 = min(c0 + 1, 2);
-    const float x0 = q[c0], x1 = q[c1];
-    float e[3];
-    e[0] = q[g < 3 ? 3 + 3 * g : 12];
-    e[1] = q[g < 3 ? 4 + 3 * g : 12];
-    e[2] = q[g < 3 ? 5 + 3 * g : 12];
-    if (g == 3) {
-        e[1] = 1.0f;
-        e[2] = 0.0f;
+    typedef float    f4 __attribute__((ext_vector_type(4), aligned(4)));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    const float x0 = q[g < 3 ? 0 : 1], x1 = q[g < 2 ? 1 : 2], x2 = q[2];
+    // direction, normal, albedo and roughness: features 72 .. 79 are group 1's, 80 and 81 group 2's
+    const f4  ea = *reinterpret_cast<const f4 *>(q + (g == 1 ? 3 : 9));
+    const f4  eb = *reinterpret_cast<const f4 *>(q + (g == 1 ? 7 : 9));
+    const int f0 = g < 3 ? 4 * g : 0, f1 = g < 2 ? 4 + 4 * g : 4 * g - 8;
+    uint32_t  v[9];
+    // 16 * 2^11 pi < 2^17; a NaN is not near
+    if (__all(fabsf(x0) <= 16.0f && fabsf(x1) <= 16.0f && fabsf(x2) <= 16.0f)) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            v[m]     = sincos_pair<true>(x0, f0 + m);
+            v[4 + m] = sincos_pair<true>(x1, f1 + m);
+        }
+        v[8] = sincos_pair<true>(x2, 8 + g);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 9; ++k) v[k] = 0u;
+#pragma unroll 1
+        for (int m = 0; m < 9; ++m) {
+            const uint32_t p = sincos_pair<false>(m < 4 ? x0 : m < 8 ? x1 : x2, m < 4 ? f0 + m : m < 8 ? f1 + m - 4 : 8 + g);
+#pragma unroll
+            for (int k = 0; k < 9; ++k) v[k] = k == m ? p : v[k];
+        }
     }
-    const int f0 = 9 * g - 12 * c0;   // first frequency: 0, 9, 6, 3
-    constexpr double kInv2Pi = 0.15915494309189533577;
-    constexpr float  kHi = (float)kInv2Pi, kLo = (float)(kInv2Pi - (double)kHi);
-    const float a0 = x0 * 3.14159265358979323846f, a1 = x1 * 3.14159265358979323846f;
-    const float h0 = a0 * kHi, h1 = a1 * kHi;
-    const float l0 = fmaf(a0, kHi, -h0) + a0 * kLo, l1 = fmaf(a1, kHi, -h1) + a1 * kLo;
-    float v[24];
+    const int   r    = __lane_id() & 15;
+    const u32x4 mid  = {pack2(ea[0], ea[1]), pack2(ea[2], ea[3]), pack2(eb[0], eb[1]), pack2(eb[2], eb[3])};
+    const u32x4 last = {pack2(ea[2], ea[3]), pack2(1.0f, 0.0f), 0u, 0u};
+    u32x4 c2;
 #pragma unroll
-    for (int m = 0; m < 9; ++m) {
-        const bool  own = f0 + m < 12;
-        const float sc  = __uint_as_float((uint32_t)(127 + (own ? f0 + m : f0 + m - 12)) << 23);
-        const float rev = fmaf(own ? l0 : l1, sc, __builtin_amdgcn_fractf((own ? h0 : h1) * sc));
-        v[2 * m]     = __builtin_amdgcn_sinf(rev);
-        v[2 * m + 1] = __builtin_amdgcn_cosf(rev);
+    for (int m = 0; m < 4; ++m) {
+        const uint32_t p = (uint32_t)__shfl((int)v[8], 16 * m + r);
+        c2[m] = g == 0 ? p : g == 1 ? mid[m] : g == 2 ? last[m] : 0u;
     }
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        v[18 + k] = e[k];
-        v[21 + k] = 0.0f;
-    }
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) f[c][j] = to_bf16(v[8 * c + j]);
+    f[0] = __builtin_bit_cast(bf16x8, u32x4{v[0], v[1], v[2], v[3]});
+    f[1] = __builtin_bit_cast(bf16x8, u32x4{v[4], v[5], v[6], v[7]});
+    f[2] = __builtin_bit_cast(bf16x8, c2);
 }
 
 // max(x, 0), 0 for NaN, in one instruction where fmaxf takes two (it first quiets its operand).
@@ -201,13 +202,14 @@ __device__ __forceinline__ void activate(const f32x4 (&acc)[4][CT], bf16x8 (&b)[
         for (int ct = 0; ct < CT; ++ct) b[c][ct] = pack<true>(acc[2 * c][ct], acc[2 * c + 1][ct]);
 }
 
-// Inference.  Bound by vector instructions (conversion, ReLU and the encoding: about 1000 and 72
-// transcendental ones per 64 samples, 65 us for 2.07M samples) beside the matrix pipe (184
-// products of 16 cycles, 39 us) and the query bytes (133 MB).  A block of four waves keeps the
-// 46 used weight fragments in LDS (46 KB: three blocks, 12 waves per CU, which 159 registers
-// a lane also allow) and loops over tiles of 256 samples; a wave owns 64 samples, so a
-// fragment read from LDS serves four products.  2,073,600 queries: 409 us with activations
-// passed through LDS, weights re-read from L2 by every wave and sincosf; 110 us like this.
+// Inference.  Bound by vector instructions (conversion, ReLU and, the larger part, the 36 sines
+// and cosines of a sample: about 1550 per 64 samples, 81 us for 2.07M samples) beside the matrix
+// pipe (184 products of 16 cycles, 39 us) and the query bytes (133 MB).  A block of four waves
+// keeps the 46 used weight fragments in LDS (46 KB: three blocks, 12 waves per CU, which 160
+// registers a lane also allow) and loops over tiles of 256 samples; a wave owns 64 samples, so
+// a fragment read from LDS serves four products.  2,073,600 queries: 409 us with activations
+// passed through LDS, weights re-read from L2 by every wave and the sines with their reduction
+// for any argument inline; 147 us like this, with the same predictions bit for bit.
 constexpr int kInferWaves = 4, kInferBlocks = 768;
 constexpr int kInferFrags = 46;   // 44 of the hidden layers, row tile 0 of the output
 
@@ -271,12 +273,12 @@ __global__ __launch_bounds__(64 * kInferWaves, 3) void k_nrc_infer(const float *
 // forms the column tile w of the layer's dW over all 64 samples.  The dW tiles accumulate in
 // registers over all the block's tiles (92 registers a lane), so a batch writes one gradient
 // partial per block, at most kNrcMaxParts of them, instead of one per 64 samples.  Two exchange
-// buffers alternate, so a layer costs one barrier.  40 KB of LDS leave room beside three
-// traversal blocks on a CU.  Bound by the chain of 12 products of one tile (a few microseconds)
+// buffers alternate, so a layer costs one barrier.  40 KB of LDS fit in beside three
+// traversal blocks on a CU, that is once one of the four has ended.  Bound by the chain of 12 products of one tile (a few microseconds)
 // for batches below 16,384; for larger ones by the weight fragments from L2 (82 KB per wave and
 // tile).  16,384 samples: 28 us with the activations saved to HBM and gathered from there by 2
-// bytes, 22 us like this; with the partials' sum (60 -> 6 us) and one pinned copy of gradient and
-// loss a gradient call went from 131 to 46 us.
+// bytes, 23 us like this; with the partials' sum (60 -> 5 us) and one pinned copy of gradient and
+// loss a gradient call went from 131 to 50 us.
 constexpr int kXt = 6 * 4 * 64, kGt = 4 * 4 * 64;   // exchanged fragments of 4 elements
 
 __global__ __launch_bounds__(256, 1) void k_nrc_train(const float *__restrict__ q, const float *__restrict__ target,
@@ -416,13 +418,13 @@ __global__ __launch_bounds__(256, 1) void k_nrc_train(const float *__restrict__ 
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
-        for (int k = 0; k < 6; ++k) P[kmap0(k >> 1, g, 4 * (k & 1) + i) * kNrcHid + wv * 16 + r] = dw0[k][i];
+        for (int k = 0; k < 6; ++k) P[feature_of(k, 4 * g + i) * kNrcHid + feature_of(wv, r)] = dw0[k][i];
 #pragma unroll
         for (int l = 0; l < 4; ++l)
 #pragma unroll
             for (int k = 0; k < 4; ++k)
-                P[nrc_w_off(l + 1) + (k * 16 + 4 * g + i) * kNrcHid + wv * 16 + r] = dwh[l][k][i];
-        float *p5 = P + nrc_w_off(5) + (wv * 16 + 4 * g + i) * kNrcOut + r;
+                P[nrc_w_off(l + 1) + feature_of(k, 4 * g + i) * kNrcHid + feature_of(wv, r)] = dwh[l][k][i];
+        float *p5 = P + nrc_w_off(5) + feature_of(wv, 4 * g + i) * kNrcOut + r;
         p5[0]  = dw5[i];
         p5[16] = 0.0f;
     }
