@@ -558,6 +558,19 @@ int alloc_renderer_buffers(crt_renderer *r)
     return CRT_OK;
 }
 
+// The sun with what the shading derives from its size.
+SunDev sun_dev(const crt_sun &sun)
+{
+    SunDev d{};
+    d.size      = sun.size;
+    d.cos_size  = (float)std::cos((double)sun.size);
+    d.cos_in    = sun_cos_in(sun.size);
+    d.intensity = sun.intensity;
+    d.dir       = mk3(sun.direction[0], sun.direction[1], sun.direction[2]);
+    d.colour    = mk3(sun.colour[0], sun.colour[1], sun.colour[2]);
+    return d;
+}
+
 camera_dev to_camera_dev(const crt_camera &c)
 {
     camera_dev d{};
@@ -1662,10 +1675,7 @@ int crt_scene_set_sun(crt_scene *scene, const crt_sun *sun)
     if (!scene || !sun) return fail(CRT_ERR_INVALID_ARG, "null argument");
     if (!(sun->size > 0.0f)) return fail(CRT_ERR_INVALID_ARG, "sun size must be positive");
     scene->sun = *sun;
-    scene->dev.sun.size      = sun->size;
-    scene->dev.sun.intensity = sun->intensity;
-    scene->dev.sun.dir       = mk3(sun->direction[0], sun->direction[1], sun->direction[2]);
-    scene->dev.sun.colour    = mk3(sun->colour[0], sun->colour[1], sun->colour[2]);
+    scene->dev.sun = sun_dev(*sun);
     return CRT_OK;
 }
 
@@ -1824,24 +1834,6 @@ int build_two_level(crt_scene *scene, const float *d_corners, const std::vector<
 }  // namespace
 
 extern "C" {
-
-namespace {
-
-// Least float c in [-1, 1] with acos_cr(c) < size, 2 if there is none: acos falls, so the
-// shading's test "the angle to the sun is below its size" (sampling.h:53-57) is c >= this.
-float sun_cos_in(float size)
-{
-    if (!(acos_cr(1.0f) < size)) return 2.0f;
-    int lo = f2ord(-1.0f), hi = f2ord(1.0f);   // acos_cr(hi) < size
-    while (lo < hi) {
-        const int mid = lo + (hi - lo) / 2;
-        if (acos_cr(ord2f(mid)) < size) hi = mid;
-        else lo = mid + 1;
-    }
-    return ord2f(hi);
-}
-
-}  // namespace
 
 int crt_scene_commit(crt_scene *scene)
 {
@@ -2042,12 +2034,7 @@ int crt_scene_commit(crt_scene *scene)
     d.sky_rot[0]  = scene->sky_rot[0];
     d.sky_rot[1]  = scene->sky_rot[1];
     d.sun_enabled = scene->sun_enabled;
-    d.sun.size      = scene->sun.size;
-    d.sun.cos_size  = (float)std::cos((double)scene->sun.size);
-    d.sun.cos_in    = sun_cos_in(scene->sun.size);
-    d.sun.intensity = scene->sun.intensity;
-    d.sun.dir       = mk3(scene->sun.direction[0], scene->sun.direction[1], scene->sun.direction[2]);
-    d.sun.colour    = mk3(scene->sun.colour[0], scene->sun.colour[1], scene->sun.colour[2]);
+    d.sun         = sun_dev(scene->sun);
     d.any_alpha   = any_alpha ? 1 : 0;
     d.model_first = scene->d_model_first;
     d.nmodels     = (uint32_t)model_first.size();

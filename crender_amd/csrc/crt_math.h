@@ -295,4 +295,18 @@ CRT_HD int f2ord(float f)
 }
 CRT_HD float ord2f(int i) { return __builtin_bit_cast(float, i >= 0 ? i : i ^ 0x7FFFFFFF); }
 
+// Least float c in [-1, 1] with acos_cr(c) < size, 2 if there is none: acos falls, so the
+// shading's test "the angle to the sun is below its size" (sampling.h:53-57) is c >= this.
+inline float sun_cos_in(float size)
+{
+    if (!(acos_cr(1.0f) < size)) return 2.0f;
+    int lo = f2ord(-1.0f), hi = f2ord(1.0f);   // acos_cr(hi) < size
+    while (lo < hi) {
+        const int mid = lo + (hi - lo) / 2;
+        if (acos_cr(ord2f(mid)) < size) hi = mid;
+        else lo = mid + 1;
+    }
+    return ord2f(hi);
+}
+
 }  // namespace crt

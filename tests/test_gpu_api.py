@@ -273,3 +273,25 @@ def test_cpp_host_example_runs():
     assert "cast_ray: distance 4.4000 material 2 normal 0.0 0.0 -1.0 point 0.00 1.00 1.00" in out.stdout
     mean = float(out.stdout.strip().split("mean display ")[-1])
     assert 0.05 < mean < 1.0
+
+
+@pytest.mark.parametrize("size", [0.4, 1e-3, 2.0])
+def test_sun_set_after_commit(size):
+    """A sun set on a committed scene counts at once and as a whole: the next image is that of
+    a scene committed with it."""
+    spec = scenes.sunlit(4, mode=1)
+    sun = dict(size=size, intensity=40.0, direction=(0.3, -1.0, 0.2), colour=(1.0, 0.9, 0.7))
+    ctx = Context(0)
+    raw = []
+    for after in (True, False):
+        sc = scene_from_spec(ctx, spec, commit=after)
+        sc.set_sun(**sun)
+        if not after:
+            sc.commit()
+        r = Renderer(ctx, sc, 48, 32, 4)
+        r.set_resolution(48, 32)
+        r.set_options(mode=1, seed=5)
+        r.render(4)
+        raw.append(r.raw())
+    assert np.array_equal(*raw)
+    ctx.close()
