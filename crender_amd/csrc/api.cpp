@@ -108,6 +108,11 @@ struct crt_context {
     size_t      stage_bytes = 0, stage_pin_bytes = 0;
     uint32_t   *q_cnt = nullptr;    // work counters and epilogue word of queries, 0 between launches
     uint32_t   *q_err = nullptr;    // pinned: traversal error flag of queries
+    // crt_render_batch's own streams.  The others are used under other locks as well (images are
+    // read, caches called, renderers created and reset while a batch runs): a launch or a wait
+    // of another thread on a stream that is being captured would become part of the batch's
+    // graph, or break it, and a reader would wait for the whole batch.
+    hipStream_t batch_stream[2] = {nullptr, nullptr};
     uint8_t    *ws = nullptr;       // Workspace
     size_t      ws_bytes = 0;
     uint8_t    *noalloc = nullptr;  // this device's crt_intersect_noalloc scratch (noalloc.hip)
@@ -1417,6 +1422,8 @@ int crt_context_destroy(crt_context *ctx)
     if (ctx->stage_pin) (void)hipHostFree(ctx->stage_pin);
     if (ctx->q_err) (void)hipHostFree(ctx->q_err);
     dfree(ctx->ws);
+    for (hipStream_t s : ctx->batch_stream)
+        if (s) (void)hipStreamDestroy(s);
     (void)hipStreamDestroy(ctx->stream);
     (void)hipStreamDestroy(ctx->stream2);
     delete ctx;
@@ -2887,8 +2894,8 @@ void plan_batch(const crt_job *jobs, uint32_t njobs, uint32_t P, BatchPlan &plan
 // Two sets of path buffers replay alternate chunks on two streams (set k renders chunks k,
 // k + 2, ...), so one chunk's traversal overlaps the other's; each chunk's accumulation
 // waits for the previous chunk's, so the job sums are added in chunk order.  Per set: one of
-// the context's streams and spill areas, a chunk cursor and, with graphs, one graph for the traversal part of
-// a replay and one for its accumulation.
+// the context's batch streams and spill areas, a chunk cursor and, with graphs, one graph for
+// the traversal part of a replay and one for its accumulation.
 struct BatchRun {
     hipStream_t         stream[2] = {nullptr, nullptr};
     hipGraph_t          graph[2][2] = {};      // [set][0: generate + bounces, 1: accumulate + advance]
@@ -2998,7 +3005,7 @@ int crt_render_batch(crt_context *ctx, const crt_job *jobs, uint32_t njobs, cons
         }
         work += (uint64_t)J.width * J.height * J.spp;
     }
-    // one stream and one spill area per context: batches, queries, autotuning and renderer
+    // the spill areas and the workspace are shared: batches, queries, autotuning and renderer
     // passes on a context run one at a time
     std::lock_guard<std::mutex> ctx_lock(ctx->mu);
     uint64_t P64 = o.max_paths ? o.max_paths : (ctx->batch_paths ? ctx->batch_paths : (4u << 20));
@@ -3051,8 +3058,9 @@ int crt_render_batch(crt_context *ctx, const crt_job *jobs, uint32_t njobs, cons
     }
     for (uint32_t k = 0; k < nsets; ++k) {
         if ((st = ensure_spill(ctx, (int)k))) return st;
-        spill[k]      = k ? ctx->spill2 : ctx->spill;
-        run.stream[k] = k ? ctx->stream2 : ctx->stream;
+        spill[k] = k ? ctx->spill2 : ctx->spill;
+        if (!ctx->batch_stream[k]) HIP_CHECK(hipStreamCreateWithFlags(&ctx->batch_stream[k], hipStreamNonBlocking));
+        run.stream[k] = ctx->batch_stream[k];
         b[k].P    = P;
         b[k].npix = P;   // no cache-training paths in batches
         b[k].ncam = P;

@@ -8,9 +8,10 @@
  * last failure on the calling thread.
  *
  * Threading: a scene is immutable after crt_scene_commit.  Calls on distinct renderers
- * are thread-safe.  Each context owns one HIP stream; every renderer and query of a
- * context is ordered on it.  Mutating a scene or renderer requires the renderer to be
- * paused, mirroring cr::renderer::update (renderer.cpp:185-192).
+ * are thread-safe.  Each context owns its HIP streams: two for the passes of renderers (queries
+ * and everything else use the first), two that only crt_render_batch uses; passes, queries,
+ * batches and commits of a context take turns.  Mutating a scene or renderer requires the
+ * renderer to be paused, mirroring cr::renderer::update (renderer.cpp:185-192).
  *
  * Memory: buffers passed to crt_scene_* are copied at commit; the caller may free them
  * after the call returns (the reference shares them with Embree instead,

@@ -142,3 +142,51 @@ def test_autotune_beside_a_background_renderer():
         box.close()
     finally:
         ctx.close()
+
+
+def test_other_calls_beside_batches():
+    """Batches on one thread, images read, cache calls and new renderers on another, all on one
+    context: every result is the one of the calls alone."""
+    import threading
+
+    from crender_amd import Nrc, Renderer
+
+    ctx = Context(0)
+    specs = [scenes.cornell(1), scenes.sunlit(4, mode=0)]
+    scs = [scene_from_spec(ctx, s) for s in specs]
+    jobs = [dict(scene=s, width=96, height=64, spp=6, max_bounces=4, seed=k) for k, s in enumerate(scs)]
+    want = render_batch(ctx, jobs, max_paths=8192)[0]
+    r = Renderer(ctx, scs[0], 64, 48, 3)
+    r.set_resolution(64, 48)
+    r.render(4)
+    image = r.raw()
+    cache = Nrc(ctx, max_batch=1024)
+    q = np.random.default_rng(1).random((1000, 13)).astype(np.float32)
+    pred, grad = cache.infer(q), cache.gradient(q, q[:, :3])
+    wrong, stop = [], threading.Event()
+
+    def poll():
+        try:
+            while not stop.is_set():
+                r.current_progress()
+                if not np.array_equal(r.raw(), image):
+                    wrong.append("image")
+                if not np.array_equal(cache.infer(q), pred) or not np.array_equal(cache.gradient(q, q[:, :3])[1], grad[1]):
+                    wrong.append("cache")
+                other = Renderer(ctx, scs[1], 32, 32, 2)
+                other.set_resolution(24, 16)
+                other.close()
+        except Exception as e:   # noqa: BLE001 - reported below, with the batches' results
+            wrong.append(repr(e))
+
+    t = threading.Thread(target=poll)
+    t.start()
+    try:
+        for _ in range(20):
+            for a, b in zip(render_batch(ctx, jobs, max_paths=8192)[0], want):
+                assert np.array_equal(a, b)
+    finally:
+        stop.set()
+        t.join(60)
+    assert not wrong, wrong[:3]
+    ctx.close()
