@@ -477,6 +477,10 @@ __device__ __forceinline__ uint32_t group_ballot(bool b, uint32_t lane)
     return (uint32_t)(__ballot(b) >> (lane & ~(kGroup - 1u))) & 0xFFu;
 }
 
+// Between stack accesses of different lanes of a group.  One wave's LDS accesses stay in order, so it
+// costs no instruction; it keeps the compiler from moving them across each other.
+__device__ __forceinline__ void group_fence() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local"); }
+
 // Keeps the lane's or its partner's candidate: the nearer hit, at equal distance the smaller
 // primID.
 template <int m>
@@ -640,6 +644,7 @@ __device__ __forceinline__ void trace_groups(const SceneDev &sc, const TraceQueu
                         *q.error = 1u;
                         break;
                     }
+                    group_fence();   // behind the loads that emptied these entries
                     if (hit && rank > 0u) stack[(sp + nh - 1u - rank) * kGroupRays] = make_uint2(ref, key & ~7u);
                     sp += nh - 1u;
                     const uint32_t near = __builtin_ctz(group_ballot(hit && rank == 0u, lane));
@@ -647,8 +652,8 @@ __device__ __forceinline__ void trace_groups(const SceneDev &sc, const TraceQueu
                     continue;
                 }
             }
-            // next entry closer than the hit, eight entries at a time (the group's LDS accesses stay in
-            // order: its lanes are of one wave)
+            // next entry closer than the hit, eight entries at a time
+            group_fence();   // behind the stores of the other lanes
             cur = kEmpty;
             while (sp > 0u) {
                 uint2 e = make_uint2(kEmpty, 0u);
