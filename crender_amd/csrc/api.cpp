@@ -97,9 +97,9 @@ struct crt_context {
     // fills the GPU while the other's launches drain; the second has its own spill area
     hipStream_t stream2 = nullptr;
     uint32_t   *spill2  = nullptr;
-    // spill entries per lane the committed scenes can need (grows with the deepest), and the
-    // number each of the two areas was allocated with
-    uint32_t    spill_depth = 32, spill_alloc[2] = {0, 0};
+    // entries of the deepest stack of the committed scenes, the spill entries per lane that it
+    // needs (both grow only), and the number each of the two areas was allocated with
+    uint32_t    stack_need = 0, spill_depth = 32, spill_alloc[2] = {0, 0};
     uint32_t    stack  = kStackLds;   // LDS stack entries per traversal lane (8, 16, 32)
     uint32_t    refill = 0, park_min = 0, leaf_rounds = 0;   // traversal thresholds (0: defaults)
     uint32_t    batch_paths = 0;   // tuned wavefront size of crt_render_batch (0 = default)
@@ -248,7 +248,7 @@ constexpr uint32_t kGroupRaysQuery = 65536, kGroupRaysRender = 32768;
 TraceConfig trace_cfg(const crt_context *ctx)
 {
     return TraceConfig{ctx->grid, ctx->stack, ctx->refill, ctx->park_min, ctx->leaf_rounds, kGroupRaysRender,
-                       ctx->spill_depth};
+                       ctx->stack_need, ctx->spill_depth};
 }
 
 // Device memory for the length of one call, kept by the context between calls (an allocation
@@ -2018,7 +2018,7 @@ int crt_scene_commit(crt_scene *scene)
     HIP_CHECK(hipStreamSynchronize(ctx->stream2));
     HIP_CHECK(hipStreamSynchronize(s));
 
-    if (max_stack > kSpillDepth + 8) {   // capacity of the smallest LDS stack configuration
+    if (max_stack > kStackMax) {
         free_scene_device(scene);
         return fail(CRT_ERR_UNSUPPORTED, "BVH too deep for the traversal stack");
     }
@@ -2060,8 +2060,8 @@ int crt_scene_commit(crt_scene *scene)
     bi.sah_cost        = br.sah;
     bi.build_ms        = br.ms;
     bi.bytes           = (uint64_t)br.node_count * 128u + (uint64_t)ntri * 48u;
-    // a lane spills at most its deepest stack, a whole LDS stack (8 to 32 entries) at a time
-    ctx->spill_depth = std::max(ctx->spill_depth, std::min(kSpillDepth, (max_stack + 31u) / 32u * 32u));
+    ctx->stack_need  = std::max(ctx->stack_need, max_stack);
+    ctx->spill_depth = std::max(ctx->spill_depth, spill_entries(max_stack));
     scene->hash      = hash;
     scene->committed = true;
     scene->dirty     = false;

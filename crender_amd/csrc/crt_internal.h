@@ -179,6 +179,16 @@ hipError_t launch_hash(const void *words, size_t nwords, uint64_t *h, void *scra
 constexpr uint32_t kXcds    = 8;
 constexpr uint32_t kCntLine = 32;   // words per 128-byte line
 constexpr uint32_t kSpillDepth = 256;   // most global spill entries per lane (multiple of 32)
+// deepest stack of an admitted scene: the smallest LDS stack (8 entries) and the spill area
+constexpr uint32_t kStackMax   = kSpillDepth + 8;
+// Spill entries per lane for a deepest stack of `need` entries: all of them where they fit, as a
+// lane spills a whole LDS stack (8 to 32 entries) at a time.  The LDS stack itself holds the rest.
+constexpr uint32_t spill_entries(uint32_t need)
+{
+    return (need + 31u) / 32u * 32u < kSpillDepth ? (need + 31u) / 32u * 32u : kSpillDepth;
+}
+// Eight lanes per ray use a block's LDS stacks alone: 8 times a lane's entries for each ray.
+constexpr bool group_stack_fits(uint32_t need, uint32_t stack_lds) { return need <= 8u * stack_lds; }
 struct TraceScene;
 struct JobDev;
 struct TraceQueue {
@@ -217,7 +227,8 @@ struct TraceQueue {
     // set by the launcher from TraceConfig: idle lanes that trigger a refill, and the number
     // of lanes still able to park a leaf below which a wave leaves the inner-node phase
     uint32_t refill_idle, park_min;
-    uint32_t group_rays;    // launches of at most this many rays trace with eight lanes per ray
+    uint32_t group_rays;    // launches of at most this many rays trace with eight lanes per ray (0
+                            // where a scene's deepest stack does not fit, group_stack_fits)
     uint32_t spill_depth;   // entries per lane of the spill area (multiple of 32)
     uint32_t leaf_rounds;   // leaf-loop iterations per leaf phase before the wave resumes the
                             // inner-node phase (0: until no lane holds a leaf)
@@ -231,6 +242,7 @@ struct TraceConfig {
     uint32_t park_min = 0;
     uint32_t leaf_rounds = 0;
     uint32_t group_rays  = 0;             // see TraceQueue
+    uint32_t stack_need  = 0;             // entries of the deepest stack of the scenes (with group_rays)
     uint32_t spill_depth = kSpillDepth;   // entries per lane of the spill area given to the launch
 };
 hipError_t launch_trace_closest(const SceneDev &sc, const TraceQueue &q, uint32_t *spill, const TraceConfig &tc,

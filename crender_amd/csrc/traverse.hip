@@ -686,7 +686,8 @@ __global__ __launch_bounds__(kTraceBlock, S == 8 ? 8 : 1) void k_trace(SceneDev 
     }
     if constexpr (W == 8 && !kInst && !kStats && !kAlpha) {
         constexpr uint32_t kDepth = S * kTraceBlock / kGroupRays;
-        if (n <= q.group_rays && q.spill_depth <= kDepth) {
+        static_assert(group_stack_fits(kDepth, S) && !group_stack_fits(kDepth + 1u, S), "the host's rule is this depth");
+        if (n <= q.group_rays) {
             if (blockIdx.x * kGroupRays >= n) return;
             trace_groups<kAny, kMulti>(sc, q, occ, n, s_stack, kDepth);
             trace_epilogue(q, n, min(gridDim.x, (n + kGroupRays - 1u) / kGroupRays));
@@ -975,7 +976,7 @@ hipError_t dispatch_trace(uint32_t width, const TraceConfig &tc, const SceneDev 
     q.refill_idle  = tc.refill ? std::min(tc.refill, 64u) : kRefillIdle;
     q.park_min     = tc.park_min ? std::min(tc.park_min, 64u) : kParkMin;
     q.spill_depth  = tc.spill_depth;
-    q.group_rays   = tc.group_rays;
+    q.group_rays   = group_stack_fits(tc.stack_need, tc.stack) ? tc.group_rays : 0u;
     q.leaf_rounds  = tc.leaf_rounds ? (tc.leaf_rounds > 64u ? 0u : tc.leaf_rounds) : kLeafRounds;
     if (!kMulti && !kAlpha && q.tstats) {
         // instrumented traversal: one stack depth (the counts do not depend on it)
