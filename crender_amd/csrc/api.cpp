@@ -1130,7 +1130,9 @@ int reset_accum(crt_renderer *r)
 // copy from or to pageable memory by itself, 8 to 15 us a copy, and a call had up to 20 of
 // them.  Up to kDirectRays the kernels read and write the pinned block itself; above, one copy
 // each way is faster than the bus reads of the traversal.  Larger arrays are copied one by one.
-// Everything is kept by the context, up to the largest call so far.
+// Everything is kept by the context, up to the largest call so far; a call takes the arrays it
+// uses and no more: callers with device memory at most 6 (24 bytes a ray), host callers at most
+// 19 above kPinnedRays (76 bytes a ray).
 constexpr uint32_t kPinnedRays = 131072, kDirectRays = 8192;
 
 struct QueryStage {
@@ -1138,13 +1140,15 @@ struct QueryStage {
     uint32_t     n = 0;
     size_t       stride = 0;           // bytes between arrays
     bool         dev = false, pinned = false, direct = false;
-    uint32_t     nin = 0, nout = 0, ntmp = 0;
-    struct Out { void *user; size_t elem; } out[12];
+    uint32_t     nin = 0, nout = 0, ntmp = 0, ncopy = 0;   // arrays handed out, results to copy
+    uint32_t     cap_in = 0, cap_out = 0, cap_tmp = 0;     // arrays of the call
+    struct Out { void *user; uint8_t *at; size_t elem; } out[12];
     uint8_t     *d = nullptr, *h = nullptr;
-    // device block: 8 inputs, 12 outputs, 8 temporaries; pinned block: 8 inputs, 12 outputs
-    static constexpr uint32_t kIn = 8, kOut = 12, kTmp = 8;
+    // pinned block: inputs, outputs; device block: the same where the kernels do not use the
+    // pinned one, then temporaries.  A device caller's inputs and outputs are its own arrays.
 
-    int open(crt_context *c, uint32_t rays, int memory)
+    // in, outs: arrays the caller gives and wants; tmp: temporaries of the call
+    int open(crt_context *c, uint32_t rays, int memory, uint32_t in, uint32_t outs, uint32_t tmp)
     {
         ctx    = c;
         n      = rays;
@@ -1152,6 +1156,9 @@ struct QueryStage {
         dev    = memory == CRT_MEM_DEVICE;
         pinned = !dev && n <= kPinnedRays;
         direct = pinned && n <= kDirectRays;
+        cap_in  = dev ? 0 : in;
+        cap_out = dev ? 0 : outs;
+        cap_tmp = tmp;
         auto grow = [&](uint8_t *&p, size_t &have, size_t want, bool host) -> int {
             if (want <= have) return CRT_OK;
             if (host && p) (void)hipHostFree(p);
@@ -1163,8 +1170,8 @@ struct QueryStage {
             have = want;
             return CRT_OK;
         };
-        int st = grow(ctx->stage, ctx->stage_bytes, stride * (kIn + kOut + kTmp), false);
-        if (!st && pinned) st = grow(ctx->stage_pin, ctx->stage_pin_bytes, stride * (kIn + kOut), true);
+        int st = grow(ctx->stage, ctx->stage_bytes, stride * ((direct ? 0 : cap_in + cap_out) + cap_tmp), false);
+        if (!st && pinned) st = grow(ctx->stage_pin, ctx->stage_pin_bytes, stride * (cap_in + cap_out), true);
         if (st) return st;
         if (!ctx->q_cnt) {
             HIP_CHECK(dalloc(&ctx->q_cnt, (size_t)(kXcds + 1) * kCntLine));
@@ -1204,19 +1211,24 @@ struct QueryStage {
         if (pinned && !direct) HIP_CHECK(hipMemcpyAsync(d, h, stride * nin, hipMemcpyHostToDevice, ctx->stream));
         return CRT_OK;
     }
-    // device address of an output array, null where the caller wants none
+    // Device address of an output array, null where the caller wants none.  over: an array of the
+    // call whose element the kernel reads before it writes the output's, taken for it where
+    // outputs are copied one by one (shares).
     template <class T>
-    T *output(T *user)
+    T *output(T *user, T *over = nullptr)
     {
         if (!user || dev) return user;
-        const size_t off = stride * (kIn + nout);
-        out[nout++] = Out{user, sizeof(T)};
-        return reinterpret_cast<T *>((direct ? h : d) + off);
+        uint8_t *at = over && shares() ? reinterpret_cast<uint8_t *>(over)
+                                       : (direct ? h : d) + stride * (cap_in + nout++);
+        out[ncopy++] = Out{user, at, sizeof(T)};
+        return reinterpret_cast<T *>(at);
     }
+    bool shares() const { return !dev && !pinned; }
+    static bool shares(uint32_t rays, int memory) { return memory != CRT_MEM_DEVICE && rays > kPinnedRays; }
     template <class T>
     T *temp()
     {
-        return reinterpret_cast<T *>(d + stride * (kIn + kOut + ntmp++));
+        return reinterpret_cast<T *>(d + stride * ((direct ? 0 : cap_in + cap_out) + ntmp++));
     }
     // the traversal's queue over the rays
     TraceQueue queue(const RaySoA &rays, const HitSoA &hits, bool unit_dir)
@@ -1231,13 +1243,13 @@ struct QueryStage {
     {
         hipStream_t s = ctx->stream;
         if (!dev && !pinned)
-            for (uint32_t k = 0; k < nout; ++k)
-                HIP_CHECK(hipMemcpyAsync(out[k].user, d + stride * (kIn + k), out[k].elem * n, hipMemcpyDeviceToHost, s));
+            for (uint32_t k = 0; k < ncopy; ++k)
+                HIP_CHECK(hipMemcpyAsync(out[k].user, out[k].at, out[k].elem * n, hipMemcpyDeviceToHost, s));
         if (pinned && !direct && nout)
-            HIP_CHECK(hipMemcpyAsync(h + stride * kIn, d + stride * kIn, stride * nout, hipMemcpyDeviceToHost, s));
+            HIP_CHECK(hipMemcpyAsync(h + stride * cap_in, d + stride * cap_in, stride * nout, hipMemcpyDeviceToHost, s));
         HIP_CHECK(hipStreamSynchronize(s));
-        if (pinned)
-            for (uint32_t k = 0; k < nout; ++k) std::memcpy(out[k].user, h + stride * (kIn + k), out[k].elem * n);
+        if (pinned)   // one array after the other in both blocks
+            for (uint32_t k = 0; k < ncopy; ++k) std::memcpy(out[k].user, h + stride * (cap_in + k), out[k].elem * n);
         if (*ctx->q_err) {
             *ctx->q_err = 0;
             return fail(CRT_ERR_HIP, "traversal stack overflow");
@@ -1269,8 +1281,15 @@ int query(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_hits *hits, ui
     if (n == 0) return CRT_OK;
     crt_context *ctx = scene->ctx;
     std::lock_guard<std::mutex> lock(ctx->mu);
+    const uint32_t tmp = hits ? 1u + (scene->dev.instanced ? 1u : 0u) : 0u;
+    uint32_t       wanted = occluded ? 1u : 0u;
+    if (hits)
+        for (const void *p : {(const void *)hits->t, (const void *)hits->u, (const void *)hits->v, (const void *)hits->prim_id,
+                              (const void *)hits->geom_id, (const void *)hits->ng_x, (const void *)hits->ng_y,
+                              (const void *)hits->ng_z, (const void *)hits->inst_id})
+            wanted += p != nullptr;
     QueryStage Q;
-    int st = Q.open(ctx, n, memory);
+    int st = Q.open(ctx, n, memory, 8, wanted, tmp);
     RaySoA  rs{};
     float **dst[8] = {&rs.ox, &rs.oy, &rs.oz, &rs.dx, &rs.dy, &rs.dz, &rs.tn, &rs.tf};
     for (int k = 0; k < 8 && !st; ++k) st = Q.input(in[k], dst[k]);
@@ -1307,8 +1326,15 @@ int cast_records(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_records
     if (n == 0) return CRT_OK;
     crt_context *ctx = scene->ctx;
     std::lock_guard<std::mutex> lock(ctx->mu);
+    // six results can take the place of the traversal's and of the staged origins
+    const void *wants[12] = {rec->distance, rec->u,   rec->v,   rec->p_x, rec->p_y, rec->p_z,
+                             rec->prim_id,  rec->geom_id, rec->material, rec->n_x, rec->n_y, rec->n_z};
+    uint32_t given = 0, wanted = 0;
+    for (const float *p : in) given += p != nullptr;
+    for (int k = QueryStage::shares(n, memory) ? 6 : 0; k < 12; ++k) wanted += wants[k] != nullptr;
+    const uint32_t tmp = 4u + (scene->dev.instanced ? 1u : 0u) + (!in[6] != !in[7] ? 1u : 0u);
     QueryStage Q;
-    int st = Q.open(ctx, n, memory);
+    int st = Q.open(ctx, n, memory, given, wanted, tmp);
     RaySoA  rs{};
     float **dst[8] = {&rs.ox, &rs.oy, &rs.oz, &rs.dx, &rs.dy, &rs.dz, &rs.tn, &rs.tf};
     for (int k = 0; k < 8 && !st; ++k)
@@ -1327,18 +1353,18 @@ int cast_records(crt_scene *scene, const crt_rays *rays, uint32_t n, crt_records
     h.inst = scene->dev.instanced ? Q.temp<uint32_t>() : nullptr;
     if ((st = query_trace(scene, Q.queue(rs, h, true), nullptr))) return st;
     RecordsDev out;
-    out.dist = Q.output(rec->distance);
+    out.dist = Q.output(rec->distance, h.t);
     out.prim = Q.output(rec->prim_id);
     out.geom = Q.output(rec->geom_id);
     out.mat  = Q.output(rec->material);
-    out.u    = Q.output(rec->u);
-    out.v    = Q.output(rec->v);
+    out.u    = Q.output(rec->u, h.u);
+    out.v    = Q.output(rec->v, h.v);
     out.nx   = Q.output(rec->n_x);
     out.ny   = Q.output(rec->n_y);
     out.nz   = Q.output(rec->n_z);
-    out.px   = Q.output(rec->p_x);
-    out.py   = Q.output(rec->p_y);
-    out.pz   = Q.output(rec->p_z);
+    out.px   = Q.output(rec->p_x, rs.ox);
+    out.py   = Q.output(rec->p_y, rs.oy);
+    out.pz   = Q.output(rec->p_z, rs.oz);
     HIP_CHECK(launch_hit_records(scene->dev, rs, h, n, out, ctx->stream));
     return Q.finish();
 }

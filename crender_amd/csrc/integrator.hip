@@ -731,7 +731,8 @@ __global__ void k_hits_to_api(SceneDev sc, HitSoA h, uint32_t n, uint32_t *prim,
 }
 
 // model.cpp:27-47, and model.cpp:114-118 for a hit on an instance: the intersection record
-// of each traced ray.
+// of each traced ray.  A thread reads its ray and hit before it writes: outputs may share the
+// arrays of either.
 __global__ void k_hit_records(SceneDev sc, RaySoA rs, HitSoA h, uint32_t n, RecordsDev out)
 {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;

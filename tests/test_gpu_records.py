@@ -144,3 +144,30 @@ def test_instanced_records_consistent_with_hits(ctx):
     assert np.all(rec["material"][both] == a.material_indices[rec["prim_id"][both]])
     assert np.all(np.isinf(rec["distance"][~hit]))
     sc.close()
+
+
+@pytest.mark.parametrize("instanced", [False, True])
+def test_records_of_each_staging(ctx, instanced):
+    """Host batches on both sides of the sizes at which their arrays go another way (8192 rays:
+    pinned memory read by the kernels; 131,072: copied through it; above: array by array, results
+    over the staged rays and hits) hold the records of the same rays in small batches."""
+    sc = scene_from_spec(ctx, scenes.soup(5_000, seed=4, sigma=0.05), commit=False)
+    if instanced:
+        sc.set_instances(0, np.eye(4, dtype=np.float32).reshape(1, 16))
+    sc.commit()
+    o, d = scenes.diffuse_rays(4_001, seed=12)
+    tf = np.where(np.arange(len(o)) % 3 == 0, 0.3, np.inf).astype(np.float32)
+    for lim in ({}, {"tfar": tf}, {"tnear": np.full(len(o), 0.01, np.float32), "tfar": tf}):
+        want = sc.cast_ray_records(o, d, **lim)
+        hits = sc.cast_rays(o, d, **lim, normals=True)
+        assert (want["prim_id"] != MISS).mean() > 0.2
+        for n in (8_192, 8_193, 131_072, 131_073):
+            k = np.arange(n) % len(o)
+            big = {key: v[k] for key, v in lim.items()}
+            got = sc.cast_ray_records(o[k], d[k], **big)
+            for key, v in want.items():
+                assert np.array_equal(got[key], v[k], equal_nan=True), (key, n)
+            got = sc.cast_rays(o[k], d[k], **big, normals=True)
+            for key, v in hits.items():
+                assert np.array_equal(got[key], v[k], equal_nan=True), (key, n)
+    sc.close()
