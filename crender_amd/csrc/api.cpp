@@ -1935,8 +1935,16 @@ int crt_scene_commit(crt_scene *scene)
     const bool     two_level = scene_instanced(scene);
     float bmin[3] = {0, 0, 0}, bmax[3] = {1, 1, 1};
     hipStream_t s = ctx->stream;
-    float *d_corners = nullptr;
-    HIP_CHECK(dalloc(&d_corners, total * 9));
+    struct Corners {   // freed as soon as the tree is built, and on every way out
+        float *p = nullptr;
+        void   free()
+        {
+            dfree(p);
+            p = nullptr;
+        }
+        ~Corners() { free(); }
+    } d_corners;
+    HIP_CHECK(dalloc(&d_corners.p, total * 9));
     HIP_CHECK(dalloc(&scene->d_mat_idx, total));
     if (!texs.empty()) {
         HIP_CHECK(dalloc(&scene->d_texs, texs.size()));
@@ -1976,7 +1984,7 @@ int crt_scene_commit(crt_scene *scene)
         const ModelHost &m = scene->models[k];
         const size_t     n = m.mat_idx.size(), at = model_first[k];
         if (!n) continue;
-        HIP_CHECK(hipMemcpyAsync(d_corners + 9 * at, m.corners.data(), sizeof(float) * 9 * n, hipMemcpyHostToDevice, s));
+        HIP_CHECK(hipMemcpyAsync(d_corners.p + 9 * at, m.corners.data(), sizeof(float) * 9 * n, hipMemcpyHostToDevice, s));
         HIP_CHECK(hipMemcpyAsync(scene->d_mat_idx + at, m.mat_idx.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice, s));
     }
     if (!small.empty()) HIP_CHECK(hipMemcpyAsync(d_small, small.data(), small.size(), hipMemcpyHostToDevice, s));
@@ -1993,7 +2001,7 @@ int crt_scene_commit(crt_scene *scene)
         for (size_t k = 0; k < scene->models.size(); ++k) {
             const ModelHost &m = scene->models[k];
             const size_t     n = m.mat_idx.size(), at = model_first[k], mw = m.mats.size() * sizeof(crt_material) / 4;
-            HIP_CHECK(launch_hash(d_corners + 9 * at, 9 * n, d_hash, hash_tmp, s2));
+            HIP_CHECK(launch_hash(d_corners.p + 9 * at, 9 * n, d_hash, hash_tmp, s2));
             HIP_CHECK(launch_hash(scene->d_mat_idx + at, n, d_hash, hash_tmp, s2));
             HIP_CHECK(launch_hash(d_small + mat_at, mw, d_hash, hash_tmp, s2));
             // the model's materials follow those of the models before it
@@ -2009,9 +2017,9 @@ int crt_scene_commit(crt_scene *scene)
     BuildResult br{};
     uint32_t    max_stack = 0;
     if (!two_level) {
-        hipError_t be = build_bvh(d_corners, ntri, width, max_leaf, s, &br, ctx->opt.bvh_prim_cost);
+        hipError_t be = build_bvh(d_corners.p, ntri, width, max_leaf, s, &br, ctx->opt.bvh_prim_cost);
         (void)hipStreamSynchronize(ctx->stream2);   // the hash reads the corners too
-        dfree(d_corners);
+        d_corners.free();
         if (br.invalid) return fail(CRT_ERR_HIP, "BVH build: the builder's consistency checks failed");
         if (be != hipSuccess) return fail(CRT_ERR_HIP, std::string("BVH build: ") + hipGetErrorString(be));
         scene->d_nodes = br.nodes;
@@ -2022,9 +2030,9 @@ int crt_scene_commit(crt_scene *scene)
             bmax[k] = br.hi[k];
         }
     } else {
-        const int st2 = build_two_level(scene, d_corners, model_first, width, max_leaf, s, br, bmin, bmax, max_stack);
+        const int st2 = build_two_level(scene, d_corners.p, model_first, width, max_leaf, s, br, bmin, bmax, max_stack);
         (void)hipStreamSynchronize(ctx->stream2);
-        dfree(d_corners);
+        d_corners.free();
         if (st2) {
             free_scene_device(scene);
             return st2;

@@ -1654,10 +1654,29 @@ hipError_t build_bvh(const float *d_tri, uint32_t ntri, uint32_t width, uint32_t
     if (dev < 0 || dev >= kMaxDevices) return hipErrorInvalidDevice;
     ScratchArena               &sa = device_arena(dev);
     std::lock_guard<std::mutex> arena_lock(sa.mu);
-    hipEvent_t ev0, ev1;
-    HIP_TRY(hipEventCreate(&ev0));
-    HIP_TRY(hipEventCreate(&ev1));
-    HIP_TRY(hipEventRecord(ev0, s));
+    // What the build creates, given back on every way out; the result's buffers only if it fails,
+    // and nothing before the kernels that may still run on them have ended.
+    struct Owned {
+        hipStream_t s;
+        hipEvent_t  ev0 = nullptr, ev1 = nullptr;
+        void       *arena = nullptr, *wide = nullptr;
+        float4     *tri   = nullptr;   // the triangles in leaf order: part of the result
+        bool        done  = false;
+        ~Owned()
+        {
+            if (!done) {
+                (void)hipStreamSynchronize(s);
+                if (tri) (void)hipFree(tri);
+                if (wide) (void)hipFree(wide);
+            }
+            if (arena) (void)hipFree(arena);
+            if (ev0) (void)hipEventDestroy(ev0);
+            if (ev1) (void)hipEventDestroy(ev1);
+        }
+    } own{s};
+    HIP_TRY(hipEventCreate(&own.ev0));
+    HIP_TRY(hipEventCreate(&own.ev1));
+    HIP_TRY(hipEventRecord(own.ev0, s));
 
     const uint32_t nslots = 2 * ntri;
     float4 *plo, *phi, *cen;
@@ -1714,9 +1733,9 @@ hipError_t build_bvh(const float *d_tri, uint32_t ntri, uint32_t width, uint32_t
     A.add(&fb, sizeof(Frontier) * max_wide);
     A.add(&fcnt, sizeof(uint32_t) * ((size_t)max_wide + 6));
     void *arena     = nullptr;
-    bool  own_arena = A.bytes > kKeepBytes;   // too large to keep: this build's own
-    if (own_arena) {
-        HIP_TRY(hipMalloc(&arena, A.bytes));
+    if (A.bytes > kKeepBytes) {   // too large to keep: this build's own
+        HIP_TRY(hipMalloc(&own.arena, A.bytes));
+        arena = own.arena;
     } else {
         if (sa.bytes < A.bytes) {   // the previous build on this device has completed
             if (sa.base) HIP_TRY(hipFree(sa.base));
@@ -1729,7 +1748,6 @@ hipError_t build_bvh(const float *d_tri, uint32_t ntri, uint32_t width, uint32_t
         arena = sa.base;
     }
     A.place(arena);
-    float4 *tri_out = nullptr;   // the triangles in leaf order: part of the result
 
     // root bounds start empty (order-preserving integer images of +inf / -inf); small
     // constants are set with memsets, not copied from pageable host memory, which would wait
@@ -1769,7 +1787,7 @@ hipError_t build_bvh(const float *d_tri, uint32_t ntri, uint32_t width, uint32_t
         }
         HIP_TRY(hipGetLastError());
         // the result's triangle buffer is allocated while the first levels run
-        if (!tri_out) HIP_TRY(hipMalloc((void **)&tri_out, sizeof(float4) * 3 * (size_t)ntri));
+        if (!own.tri) HIP_TRY(hipMalloc((void **)&own.tri, sizeof(float4) * 3 * (size_t)ntri));
         HIP_TRY(hipMemcpyAsync(hc, counts, sizeof hc, hipMemcpyDeviceToHost, s));
         HIP_TRY(hipStreamSynchronize(s));
         if (hc[8 + L % kRing] == 0u) break;
@@ -1815,11 +1833,6 @@ hipError_t build_bvh(const float *d_tri, uint32_t ntri, uint32_t width, uint32_t
             HIP_TRY(hipStreamSynchronize(s));
             if (first && hc[5] != 0u) {
                 // a node slot or child range fell outside the tree: nothing past this point is safe
-                HIP_TRY(hipStreamSynchronize(s));
-                if (own_arena) hipFree(arena);
-                hipFree(tri_out);
-                hipEventDestroy(ev0);
-                hipEventDestroy(ev1);
                 out->invalid = 1;
                 return hipErrorUnknown;
             }
@@ -1885,12 +1898,11 @@ hipError_t build_bvh(const float *d_tri, uint32_t ntri, uint32_t width, uint32_t
     const uint32_t nwide = hc[4];
     if (width == 4) k_check_wide<4><<<(nwide + 255) / 256, 256, 0, s>>>(wide_tmp, nwide, ntri, counts + 5);
     else k_check_wide<8><<<(nwide + 255) / 256, 256, 0, s>>>(wide_tmp, nwide, ntri, counts + 5);
-    k_reorder<<<(ntri + 255) / 256, 256, 0, s>>>(idx, ntri, d_tri, tri_out);
+    k_reorder<<<(ntri + 255) / 256, 256, 0, s>>>(idx, ntri, d_tri, own.tri);
     HIP_TRY(hipGetLastError());
-    void *wide;   // allocated while the two kernels above run
-    HIP_TRY(hipMalloc(&wide, node_bytes * nwide));
-    HIP_TRY(hipMemcpyAsync(wide, wide_tmp, node_bytes * nwide, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipEventRecord(ev1, s));
+    HIP_TRY(hipMalloc(&own.wide, node_bytes * nwide));   // while the two kernels above run
+    HIP_TRY(hipMemcpyAsync(own.wide, wide_tmp, node_bytes * nwide, hipMemcpyDeviceToDevice, s));
+    HIP_TRY(hipEventRecord(own.ev1, s));
 
     double   sah_h = 0.0;
     uint32_t used_h = 0;
@@ -1902,23 +1914,19 @@ hipError_t build_bvh(const float *d_tri, uint32_t ntri, uint32_t width, uint32_t
     HIP_TRY(hipStreamSynchronize(s));
     const bool invalid = hc[5] != 0u;   // the structure check of the wide tree failed
     float ms = 0.0f;
-    HIP_TRY(hipEventElapsedTime(&ms, ev0, ev1));
-    hipEventDestroy(ev0);
-    hipEventDestroy(ev1);
+    HIP_TRY(hipEventElapsedTime(&ms, own.ev0, own.ev1));
     const float rdx = root_node.hi[0] - root_node.lo[0], rdy = root_node.hi[1] - root_node.lo[1],
                 rdz = root_node.hi[2] - root_node.lo[2];
     const double ra = 2.0 * ((double)rdx * rdy + (double)rdy * rdz + (double)rdz * rdx);
 
-    if (own_arena) HIP_TRY(hipFree(arena));
     if (invalid) {
-        hipFree(wide);
-        hipFree(tri_out);
         out->invalid = 1;
         return hipErrorUnknown;
     }
 
-    out->nodes      = wide;
-    out->tri        = tri_out;
+    own.done        = true;
+    out->nodes      = own.wide;
+    out->tri        = own.tri;
     out->node_count = nwide;
     out->bvh2_nodes = used_h;
     out->depth      = depth;

@@ -18,8 +18,8 @@ stub = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)   # ahead of libcrt.so and the ru
 stub.stub_log.restype = C.c_char_p
 stub.stub_phase.argtypes = [C.c_char_p]
 stub.stub_fail.argtypes = [C.c_long]
-for f in (stub.stub_live, stub.stub_peak):
-    f.restype = C.c_size_t
+stub.stub_handles.restype = C.c_long
+stub.stub_live.restype = C.c_size_t
 sys.path[:0] = [%r, %r]
 import numpy as np
 from crender_amd import Context, CrtError, Nrc, Renderer, render_batch, scene_from_spec, scenes

@@ -14,8 +14,8 @@ namespace {
 std::mutex               mu;
 std::string              phase = "-", text;
 std::map<void *, size_t> live;
-size_t                   live_bytes = 0, peak_bytes = 0;
-long                     calls = 0, fail_at = -1;
+size_t                   live_bytes = 0;
+long                     calls = 0, fail_at = -1, handles = 0;
 hipError_t               last = hipSuccess;
 uintptr_t                next_handle = 0x1000;
 
@@ -36,7 +36,6 @@ hipError_t take(void **p, size_t n)
     *p = std::calloc(1, n ? n : 1);
     live[*p] = n;
     live_bytes += n;
-    if (live_bytes > peak_bytes) peak_bytes = live_bytes;
     return hipSuccess;
 }
 
@@ -56,6 +55,14 @@ hipError_t handle(T *h)
 {
     std::lock_guard<std::mutex> g(mu);
     *h = reinterpret_cast<T>(next_handle += 16);
+    ++handles;
+    return hipSuccess;
+}
+
+hipError_t drop()
+{
+    std::lock_guard<std::mutex> g(mu);
+    --handles;
     return hipSuccess;
 }
 
@@ -69,12 +76,13 @@ void        stub_clear() { text.clear(); }
 // the k-th call from now on that can fail does (-1: none)
 void        stub_fail(long k)
 {
-    calls   = 0;
+    if (k >= 0) calls = 0;
     fail_at = k;
+    last    = hipSuccess;
 }
+int         stub_reached(long k) { return calls > k; }   // whether the call chosen last was made
 size_t      stub_live() { return live_bytes; }
-size_t      stub_peak() { return peak_bytes; }
-void        stub_reset_peak() { peak_bytes = live_bytes; }
+long        stub_handles() { return handles; }   // streams, events and graphs
 
 #define TRY(...)                                            \
     do {                                                    \
@@ -127,7 +135,11 @@ hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned)
     TRY();
     return handle(s);
 }
-hipError_t hipStreamDestroy(hipStream_t s) { return call(__func__, s, false); }
+hipError_t hipStreamDestroy(hipStream_t s)
+{
+    (void)call(__func__, s, false);
+    return drop();
+}
 hipError_t hipStreamSynchronize(hipStream_t s) { return call(__func__, s); }
 hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t, unsigned) { return call(__func__, s); }
 hipError_t hipStreamBeginCapture(hipStream_t s, hipStreamCaptureMode) { return call(__func__, s); }
@@ -142,8 +154,8 @@ hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, 
     return handle(e);
 }
 hipError_t hipGraphLaunch(hipGraphExec_t, hipStream_t s) { return call(__func__, s); }
-hipError_t hipGraphDestroy(hipGraph_t) { return hipSuccess; }
-hipError_t hipGraphExecDestroy(hipGraphExec_t) { return hipSuccess; }
+hipError_t hipGraphDestroy(hipGraph_t) { return drop(); }
+hipError_t hipGraphExecDestroy(hipGraphExec_t) { return drop(); }
 hipError_t hipEventCreate(hipEvent_t *e)
 {
     TRY();
@@ -154,7 +166,7 @@ hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned)
     TRY();
     return handle(e);
 }
-hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return drop(); }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t s) { return call(__func__, s); }
 hipError_t hipEventSynchronize(hipEvent_t) { return call(__func__); }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t)
