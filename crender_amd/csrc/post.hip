@@ -22,6 +22,7 @@
 // 5 levels of a 5x5 B3-spline kernel with hole spacing 2^level, each tap weighted by
 // exp(-|dc|^2/sc^2) exp(-|dn|^2/sn^2) exp(-|da|^2/sa^2).
 #include <hip/hip_runtime.h>
+#include <float.h>
 #include <math.h>
 
 #include "crt_internal.h"
@@ -356,9 +357,12 @@ hipError_t launch_atrous(const float4 *colour, const float4 *normal, const float
         // the colour tolerance halves per level (finer detail survives at coarse scales)
         const float scl = sc * exp2f(-(float)l);
         const int     step = 1 << l;
-        const float   le   = 1.4426950408889634f;   // log2 e
-        const AtrousArgs a = {src, normal, albedo, (int)w, (int)h, step, le / (scl * scl), le / (sn * sn),
-                              le / (sa * sa)};
+        // log2 e / sigma^2; finite where 1 / sigma^2 is, so that taps of equal values keep their weight
+        auto coeff = [](float sigma) {
+            const float v = 1.4426950408889634f / (sigma * sigma);
+            return 1.0f / (sigma * sigma) <= FLT_MAX ? fminf(v, FLT_MAX) : v;
+        };
+        const AtrousArgs a = {src, normal, albedo, (int)w, (int)h, step, coeff(scl), coeff(sn), coeff(sa)};
         // groups of rows that are `step` apart, in every residue class
         auto groups = [&](uint32_t rows) { return step * ((h + rows * step - 1) / (rows * step)); };
         auto tiles = [&](auto *kernel, uint32_t tw) {

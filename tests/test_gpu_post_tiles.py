@@ -52,3 +52,13 @@ def test_atrous_infinite_pixel_stays_local(ctx):
     same = np.ones((h, w), bool)
     same[:3, :3] = False
     assert np.array_equal(got[same], want[same])
+
+
+@pytest.mark.parametrize("which", ["colour", "normal", "albedo"])
+def test_atrous_smallest_tolerances(ctx, which):
+    """A tolerance whose inverse square is just finite lets no tap but the pixel's own and its equals
+    through: an image without equal neighbours stays as it is."""
+    h, w = 20, 70
+    c, n, a = (_image(s, h, w) for s in (7, 8, 9))
+    got = denoise(ctx, c, n, a, levels=1, **{f"sigma_{which}": 6e-20})
+    np.testing.assert_allclose(got[..., :3], c[..., :3], rtol=3e-7)
