@@ -2951,8 +2951,7 @@ struct BatchRun {
 };
 
 // The traversal part of one replay: generate the chunk's paths, trace / shade / shadow for
-// max_bounces bounces.  Only kernel launches (capturable) unless some job's scene has alpha
-// materials under the sun.
+// max_bounces bounces.  Kernel launches only, so all of it can be captured.
 int record_trace(const PathBuffers &b, const BatchDev &bd, const TraceScene *tscenes, uint32_t width,
                  uint32_t max_bounces, bool any_sun, bool any_alpha, uint32_t *spill, const TraceConfig &tc,
                  hipStream_t s)
@@ -3057,6 +3056,7 @@ int crt_render_batch(crt_context *ctx, const crt_job *jobs, uint32_t njobs, cons
     const uint32_t P = (uint32_t)((P64 + 255) / 256 * 256);
     BatchPlan plan;
     plan_batch(jobs, njobs, P, plan);
+    // batches with transparent texels under a sun are launched directly, and say so (used_graph)
     const bool use_graph = o.use_graph && !any_alpha;
 
     HIP_CHECK(hipSetDevice(ctx->device));

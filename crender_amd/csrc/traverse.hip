@@ -33,17 +33,18 @@ namespace {
 constexpr float kInf = __builtin_huge_valf();
 constexpr uint32_t kEmpty = kInvalidRef;
 constexpr uint32_t kMissKey = 0x7FE00000u;   // behind every distance
-// default idle lanes that trigger a refill.  1080p soup 20 passes / terrain 8 passes with rays
-// from the wave's own chunk: 8 -> 22.1 / 10.2 ms, 16 -> 21.9-22.1 / 10.2 (24 and 32 1 to 2 % more)
+// The defaults of the three thresholds, at 1080p: soup of 1M triangles 8 passes / 20 passes, terrain
+// of 1M triangles 8 passes, ms; 9.40 / 22.13 / 9.92 with all of them.
+// Idle lanes that trigger a refill: 8 -> 9.34 / 22.08 / 9.89, 24 -> 9.37 / 22.40 / 9.91, 32 -> 9.68 /
+// 22.68 / 9.89.
 constexpr uint32_t kRefillIdle = 16;
-// default: a wave leaves the inner-node phase for its parked leaves once fewer than 16 lanes
-// can still park one.  Measured on the 1M soup / 14.8M terrain at 1080p with two wavefronts in
-// flight: 4 -> 2690 / 3031 Mrays/s, 8 -> 2814 / 3090, 16 -> 2852-2861 / 3079, 32 -> 2758 / 2979.
+// A wave leaves the inner-node phase for its parked leaves once fewer lanes than this can still
+// park one: 4 -> 9.79 / 23.12 / 9.97, 8 -> 9.49 / 22.42 / 9.88, 32 -> 9.64 / 22.71 / 10.25.
 constexpr uint32_t kParkMin    = 16;
-// default: after 3 leaf-loop rounds, once every parked leaf is tested, a wave resumes the
-// inner-node phase (lanes still at a leaf park it there) instead of following chains of
-// popped leaves with few lanes busy.  Soup / terrain: unlimited 2870 / 3048 Mrays/s, 1 round
-// 2880 / 3055, 2 rounds 2891 / 3105, 3 rounds 2904 / 3093.
+// After so many leaf-loop rounds, once every parked leaf is tested, a wave resumes the inner-node
+// phase (lanes still at a leaf park it there) instead of following chains of popped leaves with
+// few lanes busy: 1 -> 9.71 / 22.90 / 10.26, 2 -> 9.65 / 22.74 / 10.13, 4 -> 9.51 / 22.39 / 10.00,
+// unlimited 9.66 / 22.73 / 10.09.
 constexpr uint32_t kLeafRounds = 3;
 constexpr uint32_t kInstExit   = 0xFFFFFFFEu;   // stack marker: leave the current instance
 // Ize, "Robust BVH Ray Traversal" (JCGT 2013): scaling the far slab distance by
