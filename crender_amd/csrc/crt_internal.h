@@ -295,7 +295,7 @@ constexpr uint32_t kStackLds   = 16;
 // 0.60, five (as many as fit) 10.13 / 22.52 / 10.64 / 0.64: more waves share each CU's cache.
 constexpr uint32_t kTraceBlocksPerCu = 4;
 // The same where a radiance cache trains beside it: a training block (41 KB) fits in as soon as
-// one of the four ends, and a grid of three per CU took 22.0 ms for 16 passes against 21.1.
+// one of the four ends, and a grid of three per CU takes 22.6 ms for 16 passes against 21.8.
 
 // ---- allocation-free queries (noalloc.hip) ---------------------------------------------
 // Layout of the per-device scratch array (byte offsets): counters (query_cnt words), leaf-order triangle and instance indices, u and v for callers that
